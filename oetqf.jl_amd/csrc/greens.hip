@@ -263,77 +263,103 @@ k_gf_mf(DevFault f, DevHex8 h, const double *qc, const double *qw, int nq, OkCon
     for (int k = 0; k < 6; ++k) out[(k * h.ne + i) * rs + j * cs] = acc[k];
 }
 
-// K_fm = gf21 (GF.jl:206-224): thread (source cell j fastest, receiver
-// patch i); all 6 unit eigenstrains from one geometric evaluation.  Only
-// the shear traction on the fault is needed, so the image quadrature
-// accumulates its 6-term contraction (h8_image_traction) instead of the 54
-// integrals; the full-space part and the eigenstress follow as before.
-// Two wavefronts per SIMD (at most 256 registers): dip slip needs 266
-// unconstrained and spills 44 B/lane under the bound, 67 -> 56 ms at
-// 4096 x 2048 pairs.
-template <int FT>
-__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2)))
+// K_fm = gf21 (GF.jl:206-224): a group of G lanes per (source cell j,
+// receiver patch i); all 6 unit eigenstrains from one geometric evaluation.
+// Only the shear traction on the fault is needed, so the image quadrature
+// accumulates its 6-term contraction (h8_image_traction).  The group shares
+// the Gauss points; lane g takes corner g of the Eshelby sums and, after the
+// sums over the group, eigenstrain g.  Bound by FP64 arithmetic: one thread
+// per pair left close pairs (thousands of points, one after another) running
+// alone.  One thread per pair and fixed six-point rules before, now: 46 ->
+// 25.8 ms at 4096 patches x 2048 cells, 20 -> 1.4 ms at 800 x 324 refined
+// cells (dip slip), 55 -> 0.3 ms at 216 x 40 coarse cells.  Three or four
+// wavefronts per SIMD spill in the point loop (37 and 55 ms).  The pairs run
+// along the block's contiguous dimension (cells of a receiver-major operator,
+// patches of a column-major host block), so that a wavefront's stores share
+// lines.
+template <int FT, int G>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 k_gf_fm(DevHex8 h, DevFault f, double mu, double nu, double *out, int64_t rs, int64_t cs)
 {
-    const int64_t nf = f.nx * f.nxi;
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nf * h.ne) return;
-    const int64_t j = t % h.ne, i = t / h.ne;
-    const int64_t a = i % f.nx, b = i / f.nx;
-    const double x = f.x[a], y = f.y[b], z = f.z[b];
-    const double lo[3] = {h.qx[j] - h.dx[j] / 2.0, h.qy[j], h.qz[j] - h.dz[j]};
-    const double hi[3] = {h.qx[j] + h.dx[j] / 2.0, h.qy[j] + h.dy[j], h.qz[j]};
+    __shared__ double2 gl[OQ_H8_NGL];
+    h8_load_rules(gl);
+    const int64_t nf = f.nx * f.nxi, npair = nf * h.ne, step = (int64_t)gridDim.x * (256 / G);
+    const int g = threadIdx.x % G;
     const double ca = FT == 0 ? -mu * f.sd : mu * f.s2d, cb = FT == 0 ? mu * f.cd : mu * f.c2d;
-    double E[6] = {0, 0, 0, 0, 0, 0};
-    h8_image_traction<FT>(x, y, z, lo, hi, nu, ca, cb, E);
-    Hex8Kelvin K;
-    const bool inside = hex8_kelvin(x, y, z, lo, hi, K);
     const double ci = 1.0 / (16.0 * M_PI * mu * (1.0 - nu));
-    for (int p = 0; p < 6; ++p) {
-        double s[6], mv[6];
-        hex8_stress_unit_kelvin(K, inside, p, mu, nu, s);
-        hex8_moment(p, mu, nu, mv);
-        double ti = 0.0;
+    for (int64_t t = (int64_t)blockIdx.x * (256 / G) + threadIdx.x / G; t < npair; t += step) {
+        const int64_t j = cs <= rs ? t % h.ne : t / nf, i = cs <= rs ? t / h.ne : t % nf;
+        const int64_t a = i % f.nx, b = i / f.nx;
+        const double x = f.x[a], y = f.y[b], z = f.z[b];
+        const double lo[3] = {h.qx[j] - h.dx[j] / 2.0, h.qy[j], h.qz[j] - h.dz[j]};
+        const double hi[3] = {h.qx[j] + h.dx[j] / 2.0, h.qy[j] + h.dy[j], h.qz[j]};
+        double E[6] = {0, 0, 0, 0, 0, 0};
+        h8_image_traction<FT, G>(x, y, z, lo, hi, nu, ca, cb, g, gl, E);
 #pragma unroll
-        for (int q = 0; q < 6; ++q) ti += E[q] * mv[q];
-        out[i * rs + (p * h.ne + j) * cs] = traction_vol(FT, s, f) + ti * ci;
+        for (int q = 0; q < 6; ++q) E[q] = h8_group_sum<G>(E[q]);
+        Hex8Kelvin K;
+        hex8_kelvin_zero(K);
+        if (g < 8) hex8_kelvin_corner(x, y, z, lo, hi, g, 1.0, K);
+        hex8_kelvin_reduce<G>(K);
+        if (g < 6) {
+            double s[6], mv[6];
+            hex8_stress_unit<false>(K, nullptr, hex8_inside(x, y, z, lo, hi) ? 1.0 : 0.0, g, mu, nu, s);
+            hex8_moment(g, mu, nu, mv);
+            double ti = 0.0;
+#pragma unroll
+            for (int q = 0; q < 6; ++q) ti += E[q] * mv[q];
+            out[i * rs + (g * h.ne + j) * cs] = traction_vol(FT, s, f) + ti * ci;
+        }
     }
 }
 
-// K_mm = gf22 (GF.jl:262-289): thread (source cell i fastest, receiver
-// cell j); entry [(k)nrec + j, (p)nsrc + i] += w_q sigma_k.  Receivers come
-// from rm, sources from sm: the same mesh for the dense block, a set of
-// shifted receiver cells and one source column for the grid kernel table.
-__global__ void __launch_bounds__(128) k_gf_mm(DevHex8 rm, DevHex8 sm, const double *qc,
-                                               const double *qw, int nq, double mu, double nu,
-                                               double *out, int64_t rs, int64_t cs)
+// K_mm = gf22 (GF.jl:262-289): a group of G lanes per (source cell i,
+// receiver cell j); entry [(k)nrec + j, (p)nsrc + i] += w_q sigma_k.  The
+// stress is linear in the Eshelby sums and the image integrals, so the
+// receiver's quadrature adds those up (weighted) and the six eigenstrains are
+// contracted once, one per lane.  One thread per pair and fixed six-point
+// rules before, now: 22 -> 16.8 ms at 2048^2 pairs, 14.8 -> 5.4 ms at 324^2
+// refined cells with 8 receiver points, 12 -> 0.2 ms at 40^2.  The 36 sums
+// and the generated body fill the registers of one wavefront per SIMD; held
+// to two, the point loop spills (33 ms).  Receivers come from rm, sources
+// from sm: the same mesh for the dense block, a set of shifted receiver cells
+// and one source column for the grid kernel table.
+template <int G>
+__global__ void __launch_bounds__(256) k_gf_mm(DevHex8 rm, DevHex8 sm, const double *qc, const double *qw, int nq,
+                                               double mu, double nu, double *out, int64_t rs, int64_t cs)
 {
-    const int64_t nrec = rm.ne, nsrc = sm.ne;
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nrec * nsrc) return;
-    const int64_t i = t % nsrc, j = t / nsrc;
-    // The 36 sums live in LDS (a column per thread): in registers they would
-    // be live through the image quadrature and push it into scratch spills.
-    __shared__ double acc[36][128];
-    const int c = threadIdx.x;
+    __shared__ double2 gl[OQ_H8_NGL];
+    h8_load_rules(gl);
+    const int64_t nrec = rm.ne, nsrc = sm.ne, npair = nrec * nsrc, step = (int64_t)gridDim.x * (256 / G);
+    const int g = threadIdx.x % G;
+    for (int64_t t = (int64_t)blockIdx.x * (256 / G) + threadIdx.x / G; t < npair; t += step) {
+        const int64_t i = cs <= rs ? t % nsrc : t / nrec, j = cs <= rs ? t / nsrc : t % nrec;
+        const double lo[3] = {sm.qx[i] - sm.dx[i] / 2.0, sm.qy[i], sm.qz[i] - sm.dz[i]};
+        const double hi[3] = {sm.qx[i] + sm.dx[i] / 2.0, sm.qy[i] + sm.dy[i], sm.qz[i]};
+        double D[36], in = 0.0;
 #pragma unroll
-    for (int m = 0; m < 36; ++m) acc[m][c] = 0.0;
-    for (int q = 0; q < nq; ++q) {
-        const double rx = rm.cx[j] + qc[3 * q] * rm.dx[j] / 2.0;
-        const double ry = rm.cy[j] + qc[3 * q + 1] * rm.dy[j] / 2.0;
-        const double rz = rm.cz[j] + qc[3 * q + 2] * rm.dz[j] / 2.0;
-        Hex8Pair P;
-        hex8_pair(rx, ry, rz, sm.qx[i], sm.qy[i], sm.qz[i], sm.dx[i], sm.dy[i], sm.dz[i], nu, P);
-        for (int p = 0; p < 6; ++p) {
+        for (int m = 0; m < 36; ++m) D[m] = 0.0;
+        for (int q = 0; q < nq; ++q)
+            h8_image_integral<G>(rm.cx[j] + qc[3 * q] * rm.dx[j] / 2.0, rm.cy[j] + qc[3 * q + 1] * rm.dy[j] / 2.0,
+                                 rm.cz[j] + qc[3 * q + 2] * rm.dz[j] / 2.0, lo, hi, nu, qw[q], g, gl, D);
+#pragma unroll
+        for (int m = 0; m < 36; ++m) D[m] = h8_group_sum<G>(D[m]);
+        Hex8Kelvin K;
+        hex8_kelvin_zero(K);
+        for (int q = 0; q < nq; ++q) {
+            const double rx = rm.cx[j] + qc[3 * q] * rm.dx[j] / 2.0, ry = rm.cy[j] + qc[3 * q + 1] * rm.dy[j] / 2.0,
+                         rz = rm.cz[j] + qc[3 * q + 2] * rm.dz[j] / 2.0;
+            if (g < 8) hex8_kelvin_corner(rx, ry, rz, lo, hi, g, qw[q], K);
+            in += hex8_inside(rx, ry, rz, lo, hi) ? qw[q] : 0.0;
+        }
+        hex8_kelvin_reduce<G>(K);
+        if (g < 6) {
             double s[6];
-            hex8_stress_unit(P, p, mu, nu, s);
+            hex8_stress_unit<true>(K, D, in, g, mu, nu, s);
 #pragma unroll
-            for (int k = 0; k < 6; ++k) acc[p * 6 + k][c] += s[k] * qw[q];
+            for (int k = 0; k < 6; ++k) out[(k * nrec + j) * rs + (g * nsrc + i) * cs] = s[k];
         }
     }
-    for (int p = 0; p < 6; ++p)
-#pragma unroll
-        for (int k = 0; k < 6; ++k) out[(k * nrec + j) * rs + (p * nsrc + i) * cs] = acc[p * 6 + k][c];
 }
 
 // Dense fault-fault block: K[(i,j),(k,l)] = st[|i-k|, j, l] (the expansion
@@ -389,16 +415,36 @@ int launch_gf_mf(const DevFault &f, const DevHex8 &h, const double *qc, const do
     return OQ_OK;
 }
 
+// Lanes per hex8 pair: 8 fill the device once there are a few ten thousand
+// pairs and waste nothing (8 corners, 6 eigenstrains, about 130 points); with
+// fewer pairs a wavefront takes each, so that a close pair's points do not
+// run on 8 lanes while the device is idle.
+static constexpr int64_t kWavePairs = 32768;
+// blocks of 256 threads, grid-stride over the pairs
+static inline unsigned pair_blocks(int64_t n, int G)
+{
+    const int64_t b = (n * G + 255) / 256;
+    return (unsigned)(b < (1 << 22) ? b : (1 << 22));
+}
+
+template <int FT>
+static void gf_fm_ft(const DevHex8 &h, const DevFault &f, double mu, double nu, double *out, int64_t rs, int64_t cs,
+                     int64_t n, hipStream_t s)
+{
+    if (n < kWavePairs)
+        hipLaunchKernelGGL((k_gf_fm<FT, 64>), dim3(pair_blocks(n, 64)), dim3(256), 0, s, h, f, mu, nu, out, rs, cs);
+    else
+        hipLaunchKernelGGL((k_gf_fm<FT, 8>), dim3(pair_blocks(n, 8)), dim3(256), 0, s, h, f, mu, nu, out, rs, cs);
+}
+
 int launch_gf_fm(const DevHex8 &h, const DevFault &f, double lambda, double mu, int ftype,
                  double *out, int64_t rs, int64_t cs, hipStream_t s)
 {
     const double nu = lambda / 2.0 / (lambda + mu);  // GF.jl:203
     const int64_t n = f.nx * f.nxi * h.ne;
     OQ_PAIRS_FIT(n);
-    if (ftype == 0)
-        hipLaunchKernelGGL(k_gf_fm<0>, dim3(nblocks(n, 128)), dim3(128), 0, s, h, f, mu, nu, out, rs, cs);
-    else
-        hipLaunchKernelGGL(k_gf_fm<1>, dim3(nblocks(n, 128)), dim3(128), 0, s, h, f, mu, nu, out, rs, cs);
+    if (ftype == 0) gf_fm_ft<0>(h, f, mu, nu, out, rs, cs, n, s);
+    else gf_fm_ft<1>(h, f, mu, nu, out, rs, cs, n, s);
     OQ_HIP(hipGetLastError());
     return OQ_OK;
 }
@@ -416,8 +462,12 @@ int launch_gf_mm_pairs(const DevHex8 &rm, const DevHex8 &sm, const double *qc, c
     const double nu = lambda / 2.0 / (lambda + mu);  // GF.jl:259
     const int64_t n = rm.ne * sm.ne;
     OQ_PAIRS_FIT(n);
-    hipLaunchKernelGGL(k_gf_mm, dim3(nblocks(n, 128)), dim3(128), 0, s, rm, sm, qc, qw, nq, mu, nu,
-                       out, rs, cs);
+    if (n < kWavePairs)
+        hipLaunchKernelGGL(k_gf_mm<64>, dim3(pair_blocks(n, 64)), dim3(256), 0, s, rm, sm, qc, qw, nq, mu, nu, out,
+                           rs, cs);
+    else
+        hipLaunchKernelGGL(k_gf_mm<8>, dim3(pair_blocks(n, 8)), dim3(256), 0, s, rm, sm, qc, qw, nq, mu, nu, out,
+                           rs, cs);
     OQ_HIP(hipGetLastError());
     return OQ_OK;
 }

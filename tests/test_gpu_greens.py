@@ -3,6 +3,8 @@
 Reference: src/BEM/GF.jl:31-71 (K_ff), :123-174 (K_mf), :194-227 (K_fm),
 :250-296 (K_mm); the GPU path is called through the C ABI.
 """
+from types import SimpleNamespace
+
 import numpy as np
 import pytest
 
@@ -89,3 +91,35 @@ def test_gf_receivers_on_cell_faces(oq, oracle):
     r = oracle.gf_fm(ma, mf, 3e10, 3e10, nquad=6)
     assert np.all(np.isfinite(g))
     assert relerr(g, r) <= TOL
+
+
+# Lanes per hex8 pair (8, or 64 below 32768 pairs) on both sides of the line,
+# and pairs from far to nearly touching: cells under the surface, thin layers
+# and cells long against their depth take up to 12 Gauss points per axis and
+# bisection.  The oracle (whose own quadrature is good to 1e-11 in these
+# norms) evaluates a sample of the receivers.
+@pytest.mark.parametrize("nx,nxi,cells,ftype", [(64, 32, (4, 2, 2), "ss"), (63, 32, (4, 2, 2), "ds"),
+                                                (5, 3, (1, 1, 1), "ss"), (64, 33, (3, 3, 2), "ds")])
+@pytest.mark.parametrize("top,thick", [(0.0, 20e3), (-500.0, 3e3)])
+def test_hex8_pairs_any_distance_match_oracle(oq, oracle, nx, nxi, cells, ftype, top, thick):
+    mf = oq.gen_mesh("RectOkada", 40e3, 20e3, 40e3 / nx, 20e3 / nxi, 70.0)
+    ma = oq.hex8_box(-30e3, -9e3, top, 60e3, 20e3, -thick, *cells)
+    ft = oq.StrikeSlip() if ftype == "ss" else oq.DipSlip()
+    g = oq.stress_greens_function(ma, mf, 3e10, 2e10, ftype=ft)
+    I, J = np.array([0, nx - 1]), np.array([0, nxi // 2, nxi - 1])
+    sub = SimpleNamespace(x=mf.x[I], ax=mf.ax[I], y=mf.y[J], z=mf.z[J], axi=mf.axi[J], nx=len(I), nxi=len(J),
+                          dx=mf.dx, dep=mf.dep, dip=mf.dip)
+    r = oracle.gf_fm(ma, sub, 3e10, 2e10, ftype=ft.code)
+    assert relerr(g[(I[:, None] + nx * J[None, :]).ravel(order="F")], r) <= TOL
+
+
+@pytest.mark.parametrize("cells,qtype", [((13, 14, 1), "Gauss1"), ((2, 2, 3), "Gauss2"), ((1, 1, 1), "Gauss3")])
+@pytest.mark.parametrize("top,thick", [(0.0, 20e3), (-500.0, 3e3)])
+def test_hex8_cell_pairs_any_distance_match_oracle(oq, oracle, cells, qtype, top, thick):
+    ma = oq.hex8_box(-30e3, -9e3, top, 60e3, 20e3, -thick, *cells, rfx=0.4)
+    g = oq.stress_greens_function(ma, 3e10, 2e10, qtype=qtype, checkeigvals=False)
+    qc, qw = oq.get_quadrature(qtype)
+    sel = np.array([0, ma.ne - 1]) if ma.ne > 1 else np.array([0])
+    sub = SimpleNamespace(**{k: getattr(ma, k)[sel] for k in ("cx", "cy", "cz", "qx", "qy", "qz", "dx", "dy", "dz")})
+    r = oracle.gf_mm_rows(ma, sub, 3e10, 2e10, qc=qc, qw=qw)
+    assert relerr(g[(np.arange(6)[:, None] * ma.ne + sel[None, :]).ravel()], r) <= TOL
