@@ -1,5 +1,6 @@
-// greens.hip -- stress Green's-function builders on gfx950 (FP64), one
-// thread per source-receiver pair, and their C-ABI entry points.
+// greens.hip -- stress Green's-function builders on gfx950 (FP64), a thread
+// (Okada) or a group of lanes (hex8) per source-receiver pair, and their
+// C-ABI entry points.
 //
 // Reference: src/BEM/GF.jl (K_ff :31-71, K_mf :123-174, K_fm :194-227,
 // K_mm :250-296), threaded there over source columns (P1); here the whole
@@ -11,8 +12,9 @@
 #include <stdlib.h>
 #include <string.h>
 
-#include <complex>
 #include <atomic>
+#include <complex>
+#include <mutex>
 #include <vector>
 
 #include "hex8_dev.h"
@@ -70,17 +72,87 @@ double cosd(double deg)
     return cos_deg_small(360.0 - arx);
 }
 
+// Operator-sized blocks between their release and the next allocation of
+// about that size.  The driver clears freed device memory at about 36 GB/s,
+// and a program that assembles one model after another soon waits for that
+// on every allocation (57 ms for the 2.1 GB of the composite model, whose
+// assembly takes 7 ms).  At most kReuseBytes are held, the oldest go first,
+// and all of them when an allocation of the library fails.  A block enters
+// only after its device has been waited for (as hipFree does), so it can be
+// handed to any thread and stream.
+static constexpr size_t kReuseMin = (size_t)32 << 20, kReuseBytes = (size_t)4 << 30;
+struct ReuseBlock {
+    void *p;
+    size_t bytes;
+    int device;
+};
+static std::mutex g_reuse_mutex;
+static std::vector<ReuseBlock> &reuse_blocks()
+{
+    static std::vector<ReuseBlock> *v = new std::vector<ReuseBlock>();  // outlives every handle
+    return *v;
+}
+
+// Frees the oldest blocks until at most `keep` bytes are held.
+static void reuse_trim(size_t keep)
+{
+    std::lock_guard<std::mutex> lock(g_reuse_mutex);
+    auto &v = reuse_blocks();
+    size_t held = 0;
+    for (const auto &b : v) held += b.bytes;
+    while (!v.empty() && held > keep) {
+        held -= v.front().bytes;
+        if (runtime_usable()) (void)hipFree(v.front().p);
+        v.erase(v.begin());
+    }
+}
+
+static hipError_t malloc_or_trim(void **p, size_t n)
+{
+    hipError_t e = hipMalloc(p, n);
+    if (e == hipSuccess) return e;
+    (void)hipGetLastError();
+    reuse_trim(0);
+    return hipMalloc(p, n);
+}
+
 int DevBuf::alloc(size_t n)
 {
     release();
     if (n == 0) n = 8;
-    if (hipMalloc(&p, n) != hipSuccess) {
+    if (malloc_or_trim(&p, n) != hipSuccess) {
         p = nullptr;
         set_error("hipMalloc of " + std::to_string(n) + " bytes failed");
         return OQ_ERR_NOMEM;
     }
     bytes = n;
     return OQ_OK;
+}
+
+int DevBuf::alloc_reuse(size_t n)
+{
+    release();
+    int dev = -1;
+    if (n < kReuseMin || hipGetDevice(&dev) != hipSuccess) return alloc(n);
+    {
+        std::lock_guard<std::mutex> lock(g_reuse_mutex);
+        auto &v = reuse_blocks();
+        for (size_t i = 0; i < v.size(); ++i)
+            if (v[i].device == dev && v[i].bytes >= n && v[i].bytes - n <= n / 8) {
+                p = v[i].p;
+                bytes = n;
+                cap = v[i].bytes;
+                device = dev;
+                v.erase(v.begin() + (long)i);
+                return OQ_OK;
+            }
+    }
+    const int rc = alloc(n);
+    if (!rc) {
+        cap = n;
+        device = dev;
+    }
+    return rc;
 }
 
 int DevBuf::upload(const void *h, size_t n, hipStream_t s)
@@ -94,9 +166,22 @@ int DevBuf::upload(const void *h, size_t n, hipStream_t s)
 
 void DevBuf::release()
 {
-    if (p && runtime_usable()) (void)hipFree(p);
+    int dev = -1;
+    if (p && runtime_usable()) {
+        if (device >= 0 && cap <= kReuseBytes && hipGetDevice(&dev) == hipSuccess && dev == device &&
+            hipDeviceSynchronize() == hipSuccess) {
+            {
+                std::lock_guard<std::mutex> lock(g_reuse_mutex);
+                reuse_blocks().push_back({p, cap, device});
+            }
+            reuse_trim(kReuseBytes);
+        } else {
+            (void)hipFree(p);
+        }
+    }
     p = nullptr;
-    bytes = 0;
+    bytes = cap = 0;
+    device = -1;
 }
 
 int check_fault(const oq_fault_mesh *m)

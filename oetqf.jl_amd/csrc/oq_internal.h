@@ -53,15 +53,31 @@ struct DevHex8 {
     int64_t ne;
 };
 
-// RAII device buffer.
+// RAII device buffer.  alloc_reuse is for operator-sized blocks that the
+// caller writes in full: released ones stay with the library for the next
+// such allocation (see greens.hip), so their contents are arbitrary.
 struct DevBuf {
     void *p = nullptr;
     size_t bytes = 0;
+    size_t cap = 0;   // alloc_reuse: size of the block (>= bytes)
+    int device = -1;  // >= 0: from alloc_reuse on that device
     DevBuf() = default;
     DevBuf(const DevBuf &) = delete;
     DevBuf &operator=(const DevBuf &) = delete;
     ~DevBuf() { release(); }
     int alloc(size_t n);
+    int alloc_reuse(size_t n);
+    void take(DevBuf &o)  // moves o's block here
+    {
+        release();
+        p = o.p;
+        bytes = o.bytes;
+        cap = o.cap;
+        device = o.device;
+        o.p = nullptr;
+        o.bytes = o.cap = 0;
+        o.device = -1;
+    }
     int upload(const void *h, size_t n, hipStream_t s = 0);
     void release();
     template <class T> T *as() const { return static_cast<T *>(p); }

@@ -753,18 +753,24 @@ __global__ void __launch_bounds__(256) k_mm_grid_table(const double *__restrict_
     }
 }
 
-// The dense K_mm block (row pitch ld) from the tiles (operator expansion).
-__global__ void __launch_bounds__(256) k_expand_mm_grid(const double *__restrict__ T, int64_t nx,
-                                                        int64_t ny, int64_t nz, int64_t nxp,
+// The dense K_mm block (row pitch ld) from the tiles.  A block takes a row at
+// a time, so that the row's part of the indexing is done once and a column's
+// in 32 bits; bound by the writes.
+__global__ void __launch_bounds__(256) k_expand_mm_grid(const double *__restrict__ T, int nx, int ny, int nz, int nxp,
                                                         double *__restrict__ k, int64_t ld)
 {
-    const int64_t nxy = nx * ny, m6 = 6 * nz * nxy, npl = 6 * nz, Wp = 2 * nxp + 1, Wy = 2 * ny - 1;
-    const int64_t step = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < m6 * m6; t += step) {
-        const int64_t row = t / m6, col = t % m6;
-        const int64_t PO = row / nxy, o = row % nxy, PI = col / nxy, o2 = col % nxy;
-        const int64_t jy = o / nx, jx = o % nx, iy = o2 / nx, ix = o2 % nx;
-        k[row * ld + col] = T[((PO * npl + PI) * Wy + (jy - iy + ny - 1)) * Wp + (jx - ix + nxp)];
+    const unsigned nxy = (unsigned)(nx * ny), npl = (unsigned)(6 * nz), m6 = npl * nxy;
+    const int Wp = 2 * nxp + 1, Wy = 2 * ny - 1;
+    for (unsigned row = blockIdx.x; row < m6; row += gridDim.x) {
+        const unsigned PO = row / nxy, o = row - PO * nxy;
+        const int jy = (int)(o / (unsigned)nx), jx = (int)o - jy * nx;
+        const double *Tr = T + ((size_t)PO * npl * Wy + (jy + ny - 1)) * Wp + jx + nxp;
+        double *kr = k + (int64_t)row * ld;
+        for (unsigned col = threadIdx.x; col < m6; col += 256) {
+            const unsigned PI = col / nxy, o2 = col - PI * nxy;
+            const int iy = (int)(o2 / (unsigned)nx), ix = (int)o2 - iy * nx;
+            kr[col] = Tr[((int64_t)PI * Wy - iy) * Wp - ix];
+        }
     }
 }
 
@@ -1071,21 +1077,34 @@ __global__ void __launch_bounds__(256) k_grid_gtable(const double *__restrict__ 
     }
 }
 
-// Dense K_fm (fault rows, mantle columns from nf) and K_mf (mantle rows,
-// fault columns) of a receiver-major operator (pitch ld) from the tables.
-__global__ void __launch_bounds__(256) k_expand_strike(const double *__restrict__ F, const double *__restrict__ G,
-                                                       int64_t nx, int64_t nxi, int64_t nxc, int64_t Q, int64_t m,
-                                                       int64_t D, double *__restrict__ k, int64_t ld)
+// Dense K_fm (nf x 6ne, pitch ldf) and K_mf (6ne x nf, pitch ldm) from the
+// tables along strike, a row at a time as k_expand_mm_grid.
+__global__ void __launch_bounds__(256) k_expand_fm(const double *__restrict__ F, int nx, int nxi, int nxc, int Q, int m,
+                                                   int64_t D, double *__restrict__ k, int64_t ldf)
 {
-    const int64_t nf = nx * nxi, m6 = Q * nxc, step = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < 2 * nf * m6; t += step) {
-        if (t < nf * m6) {  // K_fm: row f = a + nx b, column nf + q nxc + jx
-            const int64_t f = t / m6, col = t % m6, a = f % nx, b = f / nx, q = col / nxc, jx = col % nxc;
-            k[f * ld + nf + col] = F[(b * Q + q) * D + a - m * jx + m * (nxc - 1)];
-        } else {            // K_mf: row nf + q' nxc + jx, column a + nx b
-            const int64_t u = t - nf * m6, row = u / nf, f = u % nf, a = f % nx, b = f / nx;
-            const int64_t qq = row / nxc, jx = row % nxc;
-            k[(nf + row) * ld + f] = G[(qq * nxi + b) * D + m * jx - a + nx - 1];
+    const unsigned m6 = (unsigned)(Q * nxc);
+    for (int64_t f = blockIdx.x; f < (int64_t)nx * nxi; f += gridDim.x) {
+        const int b = (int)(f / nx), a = (int)(f - (int64_t)b * nx);
+        const double *Fr = F + (size_t)b * Q * D + a + m * (nxc - 1);
+        double *kr = k + f * ldf;
+        for (unsigned col = threadIdx.x; col < m6; col += 256) {
+            const unsigned q = col / (unsigned)nxc, jx = col - q * (unsigned)nxc;
+            kr[col] = Fr[(int64_t)q * D - (int64_t)m * jx];
+        }
+    }
+}
+
+__global__ void __launch_bounds__(256) k_expand_mf(const double *__restrict__ G, int nx, int nxi, int nxc, int Q, int m,
+                                                   int64_t D, double *__restrict__ k, int64_t ldm)
+{
+    const unsigned nf = (unsigned)(nx * nxi);
+    for (int64_t row = blockIdx.x; row < (int64_t)Q * nxc; row += gridDim.x) {
+        const int64_t qq = row / nxc, jx = row - qq * nxc;
+        const double *Gr = G + (size_t)qq * nxi * D + m * jx + nx - 1;
+        double *kr = k + row * ldm;
+        for (unsigned f = threadIdx.x; f < nf; f += 256) {
+            const unsigned b = f / (unsigned)nx, a = f - b * (unsigned)nx;
+            kr[f] = Gr[(int64_t)b * D - (int64_t)a];
         }
     }
 }
@@ -1431,10 +1450,7 @@ static int fft_setup(oq_rhs *h, const double *st)
 
 static int finalize_toeplitz(oq_rhs *h, DevBuf &st)
 {
-    h->K.p = st.p;
-    h->K.bytes = st.bytes;
-    st.p = nullptr;
-    st.bytes = 0;
+    h->K.take(st);
     if (h->kdtype == OQ_K_FFT) return fft_setup(h, h->K.as<double>());
     int lc, nc, nt;
     toep_shape(h, &lc, &nc, &nt);
@@ -1445,7 +1461,8 @@ static int finalize_toeplitz(oq_rhs *h, DevBuf &st)
 // and y centres on uniform spacings hx, hy, the same extents within a layer
 // and the same reference-point offsets (to 1e-11 of the largest cell
 // extent; a generated box is exact to rounding).
-static int mm_grid_detect(const oq_hex8_mesh *m, MmGrid &g, double &hx, double &hy)
+// Returns nullptr, or why the cells are no such grid.
+static const char *mm_grid_detect(const oq_hex8_mesh *m, MmGrid &g, double &hx, double &hy)
 {
     const int64_t ne = m->ne;
     const double ext = fmax(fabs(m->dx[0]), fmax(fabs(m->dy[0]), fabs(m->dz[0])));
@@ -1455,8 +1472,8 @@ static int mm_grid_detect(const oq_hex8_mesh *m, MmGrid &g, double &hx, double &
     while (nx < ne && near(m->cy[nx], m->cy[0]) && near(m->cz[nx], m->cz[0])) ++nx;
     int64_t nxy = nx;
     while (nxy < ne && near(m->cz[nxy], m->cz[0])) ++nxy;
-    OQ_REQUIRE(nxy % nx == 0 && ne % nxy == 0,
-               "OQ_K_FFT_GRID: the mantle cells do not form a grid (x fastest, then y, then layer)");
+    if (nxy % nx != 0 || ne % nxy != 0)
+        return "OQ_K_FFT_GRID: the mantle cells do not form a grid (x fastest, then y, then layer)";
     const int64_t ny = nxy / nx, nz = ne / nxy;
     hx = nx > 1 ? (m->cx[nx - 1] - m->cx[0]) / (double)(nx - 1) : 0.0;
     hy = ny > 1 ? (m->cy[(ny - 1) * nx] - m->cy[0]) / (double)(ny - 1) : 0.0;
@@ -1467,13 +1484,14 @@ static int mm_grid_detect(const oq_hex8_mesh *m, MmGrid &g, double &hx, double &
                         near(m->dz[c], m->dz[b]) && near(m->qx[c] - m->cx[c], m->qx[0] - m->cx[0]) &&
                         near(m->qy[c] - m->cy[c], m->qy[0] - m->cy[0]) &&
                         near(m->qz[c] - m->cz[c], m->qz[b] - m->cz[b]);
-        OQ_REQUIRE(ok, "OQ_K_FFT_GRID: the mantle cells are not a uniform horizontal grid (equal spacing "
-                       "and extents along x and y, the same layers under every column)");
+        if (!ok)
+            return "OQ_K_FFT_GRID: the mantle cells are not a uniform horizontal grid (equal spacing "
+                   "and extents along x and y, the same layers under every column)";
     }
     g.nx = nx;
     g.ny = ny;
     g.nz = nz;
-    return OQ_OK;
+    return nullptr;
 }
 
 // Shape of the convolution blocks: 256 threads over (source planes x outputs
@@ -1508,7 +1526,7 @@ static bool mm_strike_detect(const oq_fault_mesh *mf, MmGrid &g, double hx)
 {
     const int64_t nx = mf->nx;
     const double dxf = nx > 1 ? (mf->x[nx - 1] - mf->x[0]) / (double)(nx - 1) : mf->dx;
-    if (!(dxf > 0.0) || g.nx > 64) return false;
+    if (!(dxf > 0.0)) return false;
     const double tol = 1e-11 * dxf;
     for (int64_t a = 0; a < nx; ++a) {
         const double sh = (double)a * dxf;
@@ -1531,6 +1549,7 @@ static bool mm_strike_detect(const oq_fault_mesh *mf, MmGrid &g, double hx)
 // blocks' LDS); false if a role does not fit (then K_fm and K_mf stay dense).
 static bool mm_strike_shape(MmGrid &g, int64_t nx, int64_t nxi)
 {
+    if (g.nx > 64) return false;
     const int64_t cap = (int64_t)(kGridOtherLds / 8), Q = 6 * g.ny * g.nz, m = g.m;
     const int64_t nr = (nx + m - 1) / m, fseg = (nr + kRW - 1) / kRW, gseg = (g.nx + kRW - 1) / kRW;
     // G's row pitches are 8 mod 32 doubles, so that the eight row slots of a
@@ -1564,10 +1583,10 @@ static bool mm_strike_shape(MmGrid &g, int64_t nx, int64_t nxi)
 // 1)) as receivers of the cells (0, jy, jz); for G, D cells per (jy, jz) at
 // X0 + dxf (e - (nx_f - 1)) as receivers of the patches (0, b), with the
 // real fault's image spacing.
-static int mm_strike_build(const oq_fault_mesh *mf, const oq_hex8_mesh *ma, double lrept, const QuadUpload &qu,
-                           double lambda, double mu, int ftype, int nrept, oq_rhs *h)
+static int mm_strike_build(const oq_fault_mesh *mf, const oq_hex8_mesh *ma, const MmGrid &g, double lrept,
+                           const QuadUpload &qu, double lambda, double mu, int ftype, int nrept, DevBuf &Ftab,
+                           DevBuf &Gtab, hipStream_t stream)
 {
-    const MmGrid &g = h->grid;
     const int64_t nx = mf->nx, nxi = mf->nxi, D = g.D, nyz = g.ny * g.nz, Q = 6 * nyz, nxy = g.nx * g.ny;
     const double dxf = nx > 1 ? (mf->x[nx - 1] - mf->x[0]) / (double)(nx - 1) : mf->dx;
     // virtual receiver patches of F
@@ -1622,18 +1641,19 @@ static int mm_strike_build(const oq_fault_mesh *mf, const oq_hex8_mesh *ma, doub
     if (!rc) rc = vu.load(&vm);
     if (rc) return rc;
     fsu.dev.lrept = lrept;
-    if ((rc = raw.alloc(nt * 8)) || (rc = h->Ftab.alloc(nt * 8)) || (rc = h->Gtab.alloc(nt * 8))) return rc;
-    if ((rc = launch_gf_fm(cu.dev, fvu.dev, lambda, mu, ftype, raw.as<double>(), Q, 1, h->stream))) return rc;
-    hipLaunchKernelGGL(k_grid_ftable, dim3(grid_capped((int64_t)nt, 256)), dim3(256), 0, h->stream,
-                       raw.as<double>(), nxi, Q, D, h->Ftab.as<double>());
+    if ((rc = raw.alloc_reuse(nt * 8)) || (rc = Ftab.alloc_reuse(nt * 8)) || (rc = Gtab.alloc_reuse(nt * 8)))
+        return rc;
+    if ((rc = launch_gf_fm(cu.dev, fvu.dev, lambda, mu, ftype, raw.as<double>(), Q, 1, stream))) return rc;
+    hipLaunchKernelGGL(k_grid_ftable, dim3(grid_capped((int64_t)nt, 256)), dim3(256), 0, stream,
+                       raw.as<double>(), nxi, Q, D, Ftab.as<double>());
     OQ_HIP(hipGetLastError());
     if ((rc = launch_gf_mf(fsu.dev, vu.dev, qu.c.as<double>(), qu.w.as<double>(), qu.nq, lambda, mu, ftype, nrept,
-                           raw.as<double>(), nxi, 1, h->stream)))
+                           raw.as<double>(), nxi, 1, stream)))
         return rc;
-    hipLaunchKernelGGL(k_grid_gtable, dim3(grid_capped((int64_t)nt, 256)), dim3(256), 0, h->stream,
-                       raw.as<double>(), nxi, g.ny, g.nz, D, h->Gtab.as<double>());
+    hipLaunchKernelGGL(k_grid_gtable, dim3(grid_capped((int64_t)nt, 256)), dim3(256), 0, stream,
+                       raw.as<double>(), nxi, g.ny, g.nz, D, Gtab.as<double>());
     OQ_HIP(hipGetLastError());
-    OQ_HIP(hipStreamSynchronize(h->stream));
+    OQ_HIP(hipStreamSynchronize(stream));
     return OQ_OK;
 }
 
@@ -1683,13 +1703,12 @@ static void mm_grid_chunks(MmGrid &g, int64_t ldm, int64_t ldf)
     g.fs = (int)((ldm + cw - 1) / cw);
 }
 
-// h->Tmm: the pair kernel (GF.jl:262-289) over receivers shifted by every
+// Tmm: the pair kernel (GF.jl:262-289) over receivers shifted by every
 // horizontal offset from the source column (cells (0, 0, iz)), rearranged
-// into the convolution tiles; h->mpart for the partial sums.
-static int mm_grid_build(oq_hex8_mesh const *m, double hx, double hy, const QuadUpload &qu, double lambda,
-                         double mu, oq_rhs *h)
+// into the convolution tiles (rows of 2 nxp + 1 entries).
+static int mm_grid_build(oq_hex8_mesh const *m, const MmGrid &g, int64_t nxp, double hx, double hy,
+                         const QuadUpload &qu, double lambda, double mu, DevBuf &Tmm, hipStream_t stream)
 {
-    const MmGrid &g = h->grid;
     const int64_t Wx = 2 * g.nx - 1, Wy = 2 * g.ny - 1, nxy = g.nx * g.ny, nrec = Wx * Wy * g.nz;
     std::vector<double> r[9];
     for (auto &v : r) v.resize((size_t)nrec);
@@ -1719,23 +1738,122 @@ static int mm_grid_build(oq_hex8_mesh const *m, double hx, double hy, const Quad
                              c[5].data(), c[6].data(), c[7].data(), c[8].data(), g.nz};
     Hex8Upload ru, su;
     DevBuf raw;
-    const int64_t npl = 6 * g.nz, nt = npl * npl * Wy * (2 * g.nxp + 1);
+    const int64_t npl = 6 * g.nz, nt = npl * npl * Wy * (2 * nxp + 1);
     int rc = ru.load(&rm);
     if (!rc) rc = su.load(&sm);
-    if (!rc) rc = raw.alloc((size_t)(6 * nrec * npl) * 8);
-    if (!rc) rc = h->Tmm.alloc((size_t)nt * 8);
-    if (!rc) rc = h->mpart.alloc((size_t)(h->grid.nchunk * 6 * h->ne) * 8);
-    const int nfp = 1 + (h->grid.strike ? h->grid.nfc : h->grid.fs), nmv = h->grid.strike ? h->grid.ngc : 1;
-    if (!rc) rc = h->fpart.alloc((size_t)(nfp * h->nf) * 8);
-    if (!rc) rc = h->mvout.alloc((size_t)(nmv * 6 * h->ne) * 8);
+    if (!rc) rc = raw.alloc_reuse((size_t)(6 * nrec * npl) * 8);
+    if (!rc) rc = Tmm.alloc_reuse((size_t)nt * 8);
     if (!rc)
         rc = launch_gf_mm_pairs(ru.dev, su.dev, qu.c.as<double>(), qu.w.as<double>(), qu.nq, lambda, mu,
-                                raw.as<double>(), npl, 1, h->stream);
+                                raw.as<double>(), npl, 1, stream);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_mm_grid_table, dim3(grid_capped(nt, 256)), dim3(256), 0, h->stream, raw.as<double>(),
-                       g.nx, g.ny, g.nz, (int64_t)g.nxp, h->Tmm.as<double>());
+    hipLaunchKernelGGL(k_mm_grid_table, dim3(grid_capped(nt, 256)), dim3(256), 0, stream, raw.as<double>(),
+                       g.nx, g.ny, g.nz, nxp, Tmm.as<double>());
     OQ_HIP(hipGetLastError());
-    OQ_HIP(hipStreamSynchronize(h->stream));
+    OQ_HIP(hipStreamSynchronize(stream));
+    return OQ_OK;
+}
+
+// Partial sums of the grid operator.
+static int mm_grid_parts(oq_rhs *h)
+{
+    const MmGrid &g = h->grid;
+    int rc = h->mpart.alloc((size_t)(g.nchunk * 6 * h->ne) * 8);
+    if (!rc) rc = h->fpart.alloc((size_t)((1 + (g.strike ? g.nfc : g.fs)) * h->nf) * 8);
+    if (!rc) rc = h->mvout.alloc((size_t)((g.strike ? g.ngc : 1) * 6 * h->ne) * 8);
+    return rc;
+}
+
+static inline unsigned row_blocks(int64_t rows) { return (unsigned)(rows < 65536 ? rows : 65536); }
+
+static void launch_expand_strike(const double *F, const double *G, int64_t nx, int64_t nxi, const MmGrid &g, double *fm,
+                                 int64_t ldf, double *mf, int64_t ldm, hipStream_t s)
+{
+    const int Q = (int)(6 * g.ny * g.nz);
+    if (fm)
+        hipLaunchKernelGGL(k_expand_fm, dim3(row_blocks(nx * nxi)), dim3(256), 0, s, F, (int)nx, (int)nxi, (int)g.nx, Q,
+                           (int)g.m, g.D, fm, ldf);
+    if (mf)
+        hipLaunchKernelGGL(k_expand_mf, dim3(row_blocks(Q * g.nx)), dim3(256), 0, s, G, (int)nx, (int)nxi, (int)g.nx,
+                           Q, (int)g.m, g.D, mf, ldm);
+}
+
+static void launch_expand_mm(const double *T, const MmGrid &g, int64_t nxp, double *k, int64_t ld, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_expand_mm_grid, dim3(row_blocks(6 * g.nx * g.ny * g.nz)), dim3(256), 0, s, T, (int)g.nx,
+                       (int)g.ny, (int)g.nz, (int)nxp, k, ld);
+}
+
+// x is not within 1e-6 of a whole number of spacings h (h = 0: of 0)
+static bool off_lattice(double x, double h, double ext)
+{
+    if (!(h > 0.0)) return fabs(x) > 1e-6 * ext;
+    const double r = x / h;
+    return fabs(r - nearbyint(r)) > 1e-6;
+}
+
+// The mantle blocks of the dense operator, K_fm (nf x 6ne, pitch ldf), K_mf
+// (6ne x nf, pitch ldm) and K_mm (6ne x 6ne, pitch ldm), from the meshes.
+// A pair's entries depend on its horizontal offset only (the free surface is
+// horizontal).  Over a mantle on a uniform horizontal grid the pairs that
+// differ are therefore few: K_mm has nz^2 (2ny - 1)(2nx - 1) of them instead
+// of ne^2, and K_fm and K_mf, where the mantle's x spacing is a whole number
+// of fault spacings, D = nx_f + m (nx - 1) offsets along strike per line
+// instead of nx_f nx.  Those are evaluated and written out to the dense rows
+// (4096 patches + 16 x 16 x 8 cells: 48 ms of pairs become 4.3 ms and 0.8 ms
+// of expansion; the entries equal those of the pair kernels over all pairs to
+// rounding, 1e-12).  Taken where it halves the pairs at least, and where no
+// receiver sits on a line or face across which the stress jumps or is
+// singular and that a shift by rounding could move it over: along x and y,
+// receivers off the cells' faces, and cells' receivers off the patches' edges
+// or off the fault plane.  Otherwise every pair is evaluated.
+static int dense_blocks(const oq_fault_mesh *mf, const oq_hex8_mesh *ma, const FaultUpload &fu, const Hex8Upload &hu,
+                        const oq_quadrature *quad, const QuadUpload &qu, double lambda, double mu, int ftype, int nrept,
+                        double *fm, int64_t ldf, double *mfp, double *mm, int64_t ldm, hipStream_t s)
+{
+    const int64_t nx = mf->nx, nxi = mf->nxi;
+    MmGrid g;
+    double hx = 0.0, hy = 0.0;
+    const bool grid = mm_grid_detect(ma, g, hx, hy) == nullptr;
+    const bool strike = grid && mm_strike_detect(mf, g, hx) && 2 * g.D <= nx * g.nx;
+    const double X = ma->cx[0], Y = ma->cy[0], T = ma->dx[0], ext = fmax(fabs(T), fabs(ma->dy[0]));
+    bool tfm = strike, tmf = strike, tmm = grid && g.nx * g.ny >= 8;
+    const double dxf = nx > 1 ? (mf->x[nx - 1] - mf->x[0]) / (double)(nx - 1) : mf->dx;
+    for (int e = -1; e <= 1; e += 2)  // patch centres and the cells' x faces
+        tfm = tfm && off_lattice(mf->x[0] - (ma->qx[0] + e * T / 2.0), dxf, ext);
+    for (int64_t q = 0; q < quad->nq && (tmf || tmm); ++q) {
+        const double rx = X + quad->coords[3 * q] * T / 2.0, ry = Y + quad->coords[3 * q + 1] * ma->dy[0] / 2.0;
+        for (int e = 0; e <= 1; ++e)
+            tmm = tmm && off_lattice(rx - (ma->qx[0] + (e - 0.5) * T), hx, ext) &&
+                  off_lattice(ry - (ma->qy[0] + e * ma->dy[0]), hy, ext);
+        bool edge = false;
+        for (int p = -nrept; p <= nrept; ++p)
+            for (int e = 0; e <= 1; ++e) edge = edge || !off_lattice(rx - mf->ax[e] - p * fu.dev.lrept, dxf, ext);
+        if (!edge) continue;
+        for (int64_t j = 0; j < g.ny * g.nz && tmf; ++j) {  // distance of the receiver lines from the fault plane
+            const int64_t jy = j % g.ny, jz = j / g.ny, c = jz * g.nx * g.ny + jy * g.nx;
+            const double y = ma->cy[c] + quad->coords[3 * q + 1] * ma->dy[c] / 2.0;
+            const double z = ma->cz[c] + quad->coords[3 * q + 2] * ma->dz[c] / 2.0;
+            const double d = fabs(y * fu.dev.sd - (z + mf->dep) * fu.dev.cd);
+            tmf = d > 1e-3 * dxf;
+        }
+    }
+    int rc = OQ_OK;
+    DevBuf F, G, Tm;
+    if (tfm || tmf) rc = mm_strike_build(mf, ma, g, fu.dev.lrept, qu, lambda, mu, ftype, nrept, F, G, s);
+    if (!rc && (tfm || tmf))
+        launch_expand_strike(F.as<double>(), G.as<double>(), nx, nxi, g, tfm ? fm : nullptr, ldf, tmf ? mfp : nullptr,
+                             ldm, s);
+    if (!rc && !tfm) rc = launch_gf_fm(hu.dev, fu.dev, lambda, mu, ftype, fm, ldf, 1, s);
+    if (!rc && !tmf)
+        rc = launch_gf_mf(fu.dev, hu.dev, qu.c.as<double>(), qu.w.as<double>(), qu.nq, lambda, mu, ftype, nrept, mfp,
+                          ldm, 1, s);
+    if (!rc && tmm) rc = mm_grid_build(ma, g, g.nx, hx, hy, qu, lambda, mu, Tm, s);
+    if (!rc && tmm) launch_expand_mm(Tm.as<double>(), g, g.nx, mm, ldm, s);
+    if (!rc && !tmm) rc = launch_gf_mm(hu.dev, qu.c.as<double>(), qu.w.as<double>(), qu.nq, lambda, mu, mm, ldm, 1, s);
+    if (rc) return rc;
+    OQ_HIP(hipGetLastError());
+    OQ_HIP(hipStreamSynchronize(s));  // the tables go out of scope
     return OQ_OK;
 }
 
@@ -1770,10 +1888,7 @@ static int mm_grid_pick(oq_rhs *h)
 // traction rates.  The blocks are filled by the caller.
 static int fft_coupled_alloc(oq_rhs *h, DevBuf &st)
 {
-    h->stk.p = st.p;
-    h->stk.bytes = st.bytes;
-    st.p = nullptr;
-    st.bytes = 0;
+    h->stk.take(st);
     int rc = fft_setup(h, h->stk.as<double>());
     const int64_t m6 = 6 * h->ne;
     h->ldm = (m6 + kPad - 1) / kPad * kPad;
@@ -1783,8 +1898,8 @@ static int fft_coupled_alloc(oq_rhs *h, DevBuf &st)
     // neither dense block exists
     const bool dense = !(h->mmgrid && h->grid.strike);
     const size_t bf = (size_t)(h->nf * h->ldm) * 8, bm = (size_t)(m6 * (h->mmgrid ? h->ldf : h->ld)) * 8;
-    if (!rc && dense) rc = h->Kf.alloc(bf);
-    if (!rc && dense) rc = h->K.alloc(bm);
+    if (!rc && dense) rc = h->Kf.alloc_reuse(bf);
+    if (!rc && dense) rc = h->K.alloc_reuse(bm);
     if (!rc) rc = h->sm.alloc((size_t)h->ldm * 8);
     if (!rc && !h->mmgrid) rc = h->tauff.alloc((size_t)h->nf * 8);  // the grid model uses fpart
     if (rc) return rc;
@@ -1794,24 +1909,29 @@ static int fft_coupled_alloc(oq_rhs *h, DevBuf &st)
     return OQ_OK;
 }
 
+// Zeroes the columns past N of the dense operator (the blocks fill the rest).
+static int clear_padding(double *k, oq_rhs *h)
+{
+    if (h->ld > h->N)
+        OQ_HIP(hipMemset2DAsync(k + h->N, (size_t)h->ld * 8, 0, (size_t)(h->ld - h->N) * 8, (size_t)h->N, h->stream));
+    return OQ_OK;
+}
+
 // Converts the FP64 operator in k64 (N x ld) to h->K in h->kdtype.
 static int finalize_k(oq_rhs *h, DevBuf &k64)
 {
     const int64_t n = h->N * h->ld;
     if (h->kdtype == OQ_K_FP64) {
-        h->K.p = k64.p;
-        h->K.bytes = k64.bytes;
-        k64.p = nullptr;
-        k64.bytes = 0;
+        h->K.take(k64);
         return OQ_OK;
     }
     int rc;
     if (h->kdtype == OQ_K_FP32) {
-        if ((rc = h->K.alloc((size_t)n * 4))) return rc;
+        if ((rc = h->K.alloc_reuse((size_t)n * 4))) return rc;
         hipLaunchKernelGGL(k_to_fp32, dim3(grid_capped(n, 256)), dim3(256), 0, h->stream, k64.as<double>(),
                            h->K.as<float>(), n);
     } else {
-        if ((rc = h->K.alloc((size_t)n * 2))) return rc;
+        if ((rc = h->K.alloc_reuse((size_t)n * 2))) return rc;
         hipLaunchKernelGGL(k_to_bf16, dim3(grid_capped(n, 256)), dim3(256), 0, h->stream, k64.as<double>(),
                            h->K.as<unsigned short>(), n);
     }
@@ -1919,11 +2039,8 @@ int oq_rhs_create(int device, int64_t nx, int64_t nxi, int64_t ne, const oq_rs_p
         *out = h;
         return OQ_OK;
     }
-    rc = k64.alloc((size_t)(h->N * ld) * 8);
-    if (!rc && hipMemsetAsync(k64.p, 0, (size_t)(h->N * ld) * 8, h->stream) != hipSuccess) {
-        set_error("hipMemsetAsync failed");
-        rc = OQ_ERR_HIP;
-    }
+    rc = k64.alloc_reuse((size_t)(h->N * ld) * 8);
+    if (!rc) rc = clear_padding(k64.as<double>(), h);
     if (!rc) {
         rc = upload_toeplitz(gf11, gf11_is_dft, nx, nxi, tmp, h->stream);
         if (!rc) rc = launch_expand_toeplitz(tmp.as<double>(), nx, nxi, k64.as<double>(), ld, h->stream);
@@ -1981,7 +2098,8 @@ int oq_rhs_create_from_mesh(int device, const oq_fault_mesh *mf, const oq_hex8_m
     double hx = 0.0, hy = 0.0;
     if (grid) {
         OQ_REQUIRE(ne > 0, "OQ_K_FFT_GRID is for the coupled model (a hex8 mantle)");
-        if ((rc = mm_grid_detect(ma, g, hx, hy))) return rc;
+        const char *why = mm_grid_detect(ma, g, hx, hy);
+        OQ_REQUIRE(why == nullptr, why);
         kdtype = OQ_K_FFT;
     }
     oq_rhs *h = new oq_rhs();
@@ -2009,19 +2127,24 @@ int oq_rhs_create_from_mesh(int device, const oq_fault_mesh *mf, const oq_hex8_m
         if (!rc && hipStreamSynchronize(h->stream) != hipSuccess) rc = OQ_ERR_HIP;
         if (!rc) rc = fft_coupled_alloc(h, st);
         if (h->mmgrid && h->grid.strike) {
-            if (!rc) rc = mm_strike_build(mf, ma, fu.dev.lrept, qu, lambda, mu, ftype, (int)nrept, h);
-        } else {
+            if (!rc)
+                rc = mm_strike_build(mf, ma, h->grid, fu.dev.lrept, qu, lambda, mu, ftype, (int)nrept, h->Ftab,
+                                          h->Gtab, h->stream);
+        } else if (h->mmgrid) {
             if (!rc) rc = launch_gf_fm(hu.dev, fu.dev, lambda, mu, ftype, h->Kf.as<double>(), h->ldm, 1, h->stream);
             if (!rc)
                 rc = launch_gf_mf(fu.dev, hu.dev, qu.c.as<double>(), qu.w.as<double>(), qu.nq, lambda, mu, ftype,
-                                  (int)nrept, h->K.as<double>(), h->mmgrid ? h->ldf : ld, 1, h->stream);
+                                  (int)nrept, h->K.as<double>(), h->ldf, 1, h->stream);
         }
-        if (!rc && h->mmgrid) rc = mm_grid_build(ma, hx, hy, qu, lambda, mu, h);
-        if (!rc && h->mmgrid) rc = mm_roles_build(h);
-        if (!rc && h->mmgrid) rc = mm_grid_pick(h);
-        else if (!rc)
-            rc = launch_gf_mm(hu.dev, qu.c.as<double>(), qu.w.as<double>(), qu.nq, lambda, mu,
-                              h->K.as<double>() + nf, ld, 1, h->stream);
+        if (!rc && h->mmgrid) {
+            rc = mm_grid_build(ma, h->grid, h->grid.nxp, hx, hy, qu, lambda, mu, h->Tmm, h->stream);
+            if (!rc) rc = mm_grid_parts(h);
+            if (!rc) rc = mm_roles_build(h);
+            if (!rc) rc = mm_grid_pick(h);
+        } else if (!rc) {
+            rc = dense_blocks(mf, ma, fu, hu, quad, qu, lambda, mu, ftype, (int)nrept, h->Kf.as<double>(), h->ldm,
+                              h->K.as<double>(), h->K.as<double>() + nf, ld, h->stream);
+        }
         if (!rc && hipStreamSynchronize(h->stream) != hipSuccess) {
             set_error("device assembly failed");
             rc = OQ_ERR_HIP;
@@ -2048,23 +2171,15 @@ int oq_rhs_create_from_mesh(int device, const oq_fault_mesh *mf, const oq_hex8_m
         *out = h;
         return OQ_OK;
     }
-    if (!rc) rc = k64.alloc((size_t)(h->N * ld) * 8);
-    if (!rc && hipMemsetAsync(k64.p, 0, (size_t)(h->N * ld) * 8, h->stream) != hipSuccess) {
-        set_error("hipMemsetAsync failed");
-        rc = OQ_ERR_HIP;
-    }
+    if (!rc) rc = k64.alloc_reuse((size_t)(h->N * ld) * 8);
+    if (!rc) rc = clear_padding(k64.as<double>(), h);
     if (!rc) rc = st.alloc((size_t)(nf * mf->nxi) * 8);
     if (!rc) rc = launch_gf_ff(fu.dev, lambda, mu, ftype, (int)nrept, st.as<double>(), h->stream);
     if (!rc) rc = launch_expand_toeplitz(st.as<double>(), mf->nx, mf->nxi, k64.as<double>(), ld, h->stream);
     if (!rc && ne > 0) {
         double *K = k64.as<double>();
-        rc = launch_gf_fm(hu.dev, fu.dev, lambda, mu, ftype, K + nf, ld, 1, h->stream);
-        if (!rc)
-            rc = launch_gf_mf(fu.dev, hu.dev, qu.c.as<double>(), qu.w.as<double>(), qu.nq, lambda,
-                              mu, ftype, (int)nrept, K + nf * ld, ld, 1, h->stream);
-        if (!rc)
-            rc = launch_gf_mm(hu.dev, qu.c.as<double>(), qu.w.as<double>(), qu.nq, lambda, mu,
-                              K + nf * ld + nf, ld, 1, h->stream);
+        rc = dense_blocks(mf, ma, fu, hu, quad, qu, lambda, mu, ftype, (int)nrept, K + nf, ld, K + nf * ld,
+                          K + nf * ld + nf, ld, h->stream);
     }
     if (!rc && hipStreamSynchronize(h->stream) != hipSuccess) {
         set_error("device assembly failed");
@@ -2204,9 +2319,8 @@ int oq_rhs_get_k(oq_rhs *h, double *k)
                                     (size_t)m6 * 8, (size_t)nf, hipMemcpyDeviceToDevice, h->stream));
         if (h->mmgrid && h->grid.strike) {
             const MmGrid &g = h->grid;
-            hipLaunchKernelGGL(k_expand_strike, dim3(grid_capped(2 * nf * m6, 256)), dim3(256), 0, h->stream,
-                               h->Ftab.as<double>(), h->Gtab.as<double>(), h->nx, h->nxi, g.nx, 6 * g.ny * g.nz, g.m,
-                               g.D, tmp.as<double>(), h->ld);
+            launch_expand_strike(h->Ftab.as<double>(), h->Gtab.as<double>(), h->nx, h->nxi, g, tmp.as<double>() + nf,
+                                 h->ld, tmp.as<double>() + nf * h->ld, h->ld, h->stream);
             OQ_HIP(hipGetLastError());
         }
         if (h->mmgrid) {
@@ -2215,9 +2329,7 @@ int oq_rhs_get_k(oq_rhs *h, double *k)
                                         (size_t)h->ldf * 8, (size_t)nf * 8, (size_t)m6, hipMemcpyDeviceToDevice,
                                         h->stream));
             const MmGrid &g = h->grid;
-            hipLaunchKernelGGL(k_expand_mm_grid, dim3(grid_capped(m6 * m6, 256)), dim3(256), 0, h->stream,
-                               h->Tmm.as<double>(), g.nx, g.ny, g.nz, (int64_t)g.nxp,
-                               tmp.as<double>() + nf * h->ld + nf, h->ld);
+            launch_expand_mm(h->Tmm.as<double>(), g, g.nxp, tmp.as<double>() + nf * h->ld + nf, h->ld, h->stream);
             OQ_HIP(hipGetLastError());
         } else {
             OQ_HIP(hipMemcpy2DAsync(tmp.as<double>() + nf * h->ld, (size_t)h->ld * 8, h->K.p, (size_t)h->ld * 8,

@@ -1,7 +1,7 @@
 // CPU emulation of the grid model's along-strike tables
 // (oetqf.jl_amd/csrc/rhs.hip: the virtual geometry of mm_strike_build, the
 // raw layouts of k_gf_fm / k_gf_mf, k_grid_ftable / k_grid_gtable), the F
-// and G block loops of k_grid_fused, k_expand_strike and the role table of
+// and G block loops of k_grid_fused, k_expand_fm, k_expand_mf and the role table of
 // mm_roles_build, their index arithmetic restated over bounds-checked
 // buffers, against dense products of synthetic translation-invariant pair
 // functions.  The shapes follow mm_strike_shape.  The restatement follows the
