@@ -1142,7 +1142,7 @@ int oq_ensemble_create(int device, const oq_fault_mesh *mf, const oq_hex8_mesh *
     oq_ensemble *e = new oq_ensemble();
     e->kdtype = kdtype;
     // the split operator is made from the FP64 assembly
-    int rc = oq_rhs_create_from_mesh(device, mf, ma, lambda, mu, ftype, nrept, buffer_ratio, quad,
+    int rc = rhs_create_for_batch(device, mf, ma, lambda, mu, ftype, nrept, buffer_ratio, quad,
                                      &members[0], visc, kdtype == OQ_K_FP16X2 ? OQ_K_FP64 : kdtype,
                                      &e->h);
     if (rc) {

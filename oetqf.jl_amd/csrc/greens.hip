@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "hex8_dev.h"
+#include "hex8_seq_dev.h"
 #include "okada_dev.h"
 #include "oq_internal.h"
 
@@ -447,6 +448,70 @@ __global__ void __launch_bounds__(256) k_gf_mm(DevHex8 rm, DevHex8 sm, const dou
     }
 }
 
+// The pair kernels of the operators of lockstep batches, a thread per pair
+// (see hex8_seq_dev.h): the six eigenstrains of K_fm from one evaluation,
+// and K_mm with its 36 sums in LDS (in registers they would be live through
+// the quadrature and spill).
+template <int FT>
+__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2)))
+k_gf_fm_seq(DevHex8 h, DevFault f, double mu, double nu, double *out, int64_t rs, int64_t cs)
+{
+    const int64_t nf = f.nx * f.nxi;
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= nf * h.ne) return;
+    const int64_t j = t % h.ne, i = t / h.ne;
+    const int64_t a = i % f.nx, b = i / f.nx;
+    const double x = f.x[a], y = f.y[b], z = f.z[b];
+    const double lo[3] = {h.qx[j] - h.dx[j] / 2.0, h.qy[j], h.qz[j] - h.dz[j]};
+    const double hi[3] = {h.qx[j] + h.dx[j] / 2.0, h.qy[j] + h.dy[j], h.qz[j]};
+    const double ca = FT == 0 ? -mu * f.sd : mu * f.s2d, cb = FT == 0 ? mu * f.cd : mu * f.c2d;
+    double E[6] = {0, 0, 0, 0, 0, 0};
+    seq::h8_image_traction<FT>(x, y, z, lo, hi, nu, ca, cb, E);
+    Hex8Kelvin K;
+    const bool inside = seq::hex8_kelvin(x, y, z, lo, hi, K);
+    const double ci = 1.0 / (16.0 * M_PI * mu * (1.0 - nu));
+    for (int p = 0; p < 6; ++p) {
+        double s[6], mv[6];
+        seq::hex8_stress_unit_kelvin(K, inside, p, mu, nu, s);
+        seq::hex8_moment(p, mu, nu, mv);
+        double ti = 0.0;
+#pragma unroll
+        for (int q = 0; q < 6; ++q) ti += E[q] * mv[q];
+        out[i * rs + (p * h.ne + j) * cs] = traction_vol(FT, s, f) + ti * ci;
+    }
+}
+
+__global__ void __launch_bounds__(128) k_gf_mm_seq(DevHex8 rm, DevHex8 sm, const double *qc, const double *qw, int nq,
+                                                   double mu, double nu, double *out, int64_t rs, int64_t cs)
+{
+    const int64_t nrec = rm.ne, nsrc = sm.ne;
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= nrec * nsrc) return;
+    const int64_t i = t % nsrc, j = t / nsrc;
+    // The 36 sums live in LDS (a column per thread): in registers they would
+    // be live through the image quadrature and push it into scratch spills.
+    __shared__ double acc[36][128];
+    const int c = threadIdx.x;
+#pragma unroll
+    for (int m = 0; m < 36; ++m) acc[m][c] = 0.0;
+    for (int q = 0; q < nq; ++q) {
+        const double rx = rm.cx[j] + qc[3 * q] * rm.dx[j] / 2.0;
+        const double ry = rm.cy[j] + qc[3 * q + 1] * rm.dy[j] / 2.0;
+        const double rz = rm.cz[j] + qc[3 * q + 2] * rm.dz[j] / 2.0;
+        seq::Hex8Pair P;
+        seq::hex8_pair(rx, ry, rz, sm.qx[i], sm.qy[i], sm.qz[i], sm.dx[i], sm.dy[i], sm.dz[i], nu, P);
+        for (int p = 0; p < 6; ++p) {
+            double s[6];
+            seq::hex8_stress_unit(P, p, mu, nu, s);
+#pragma unroll
+            for (int k = 0; k < 6; ++k) acc[p * 6 + k][c] += s[k] * qw[q];
+        }
+    }
+    for (int p = 0; p < 6; ++p)
+#pragma unroll
+        for (int k = 0; k < 6; ++k) out[(k * nrec + j) * rs + (p * nsrc + i) * cs] = acc[p * 6 + k][c];
+}
+
 // Dense fault-fault block: K[(i,j),(k,l)] = st[|i-k|, j, l] (the expansion
 // test/BEM/tests.jl:46-49 checks the FFT form against).
 __global__ void __launch_bounds__(256) k_expand_toeplitz(const double *st, int64_t nx,
@@ -553,6 +618,23 @@ int launch_gf_mm_pairs(const DevHex8 &rm, const DevHex8 &sm, const double *qc, c
     else
         hipLaunchKernelGGL(k_gf_mm<8>, dim3(pair_blocks(n, 8)), dim3(256), 0, s, rm, sm, qc, qw, nq, mu, nu, out,
                            rs, cs);
+    OQ_HIP(hipGetLastError());
+    return OQ_OK;
+}
+
+// K_fm and K_mm of a lockstep batch's operator (receiver-major).
+int launch_gf_hex8_seq(const DevHex8 &h, const DevFault &f, const double *qc, const double *qw, int nq, double lambda,
+                       double mu, int ftype, double *fm, double *mm, int64_t ld, hipStream_t s)
+{
+    const double nu = lambda / 2.0 / (lambda + mu);
+    const int64_t n = f.nx * f.nxi * h.ne, n2 = h.ne * h.ne;
+    OQ_PAIRS_FIT(n);
+    OQ_PAIRS_FIT(n2);
+    if (ftype == 0)
+        hipLaunchKernelGGL(k_gf_fm_seq<0>, dim3(nblocks(n, 128)), dim3(128), 0, s, h, f, mu, nu, fm, ld, (int64_t)1);
+    else
+        hipLaunchKernelGGL(k_gf_fm_seq<1>, dim3(nblocks(n, 128)), dim3(128), 0, s, h, f, mu, nu, fm, ld, (int64_t)1);
+    hipLaunchKernelGGL(k_gf_mm_seq, dim3(nblocks(n2, 128)), dim3(128), 0, s, h, h, qc, qw, nq, mu, nu, mm, ld, (int64_t)1);
     OQ_HIP(hipGetLastError());
     return OQ_OK;
 }

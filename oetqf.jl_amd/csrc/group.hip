@@ -1593,7 +1593,7 @@ int oq_group_create(int device, int64_t ngeo, const oq_fault_mesh *mf,
     for (int64_t g = 0; g < ngeo && !rc; ++g) {
         oq_rhs *h = nullptr;
         const oq_hex8_mesh *mg = ma ? ma[g] : nullptr;
-        rc = oq_rhs_create_from_mesh(device, &mf[g], mg, lambda, mu, ftype, nrept, buffer_ratio,
+        rc = rhs_create_for_batch(device, &mf[g], mg, lambda, mu, ftype, nrept, buffer_ratio,
                                      mg ? quad : nullptr, &members[g * nmembers],
                                      mg ? visc[g] : nullptr, OQ_K_FP32, &h);
         e->rhs.push_back(h);

@@ -103,6 +103,10 @@ int launch_gf_mm(const DevHex8 &h, const double *qc, const double *qw,
 int launch_gf_mm_pairs(const DevHex8 &rm, const DevHex8 &sm, const double *qc,
                        const double *qw, int nq, double lambda, double mu,
                        double *out, int64_t rs, int64_t cs, hipStream_t s);
+// K_fm (receiver-major, pitch ld) and K_mm for the operator of a lockstep
+// batch (one thread per pair, a fixed order of operations; hex8_seq_dev.h).
+int launch_gf_hex8_seq(const DevHex8 &h, const DevFault &f, const double *qc, const double *qw, int nq, double lambda,
+                       double mu, int ftype, double *fm, double *mm, int64_t ld, hipStream_t s);
 // Expands the Toeplitz kernel st (nx,nxi,nxi) into the fault-fault block of
 // a dense receiver-major operator (row pitch ld).
 int launch_expand_toeplitz(const double *st, int64_t nx, int64_t nxi,

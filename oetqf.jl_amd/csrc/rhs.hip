@@ -29,6 +29,7 @@
 #include <utility>
 #include <vector>
 
+#include "grid_spectral.h"
 #include "rhs_impl.h"
 
 namespace oq {
@@ -37,6 +38,26 @@ namespace oq {
 static constexpr int64_t kPad = 512;  // row pitch multiple (elements)
 
 // ---------------- prologue ----------------
+// update_strain_rate! (equation.jl:207-222) of mantle cell i: e[6] from its stress.
+__device__ __forceinline__ void strain_rate(const RhsDev &d, const double *__restrict__ sg, int64_t i, double e[6])
+{
+    const int64_t ne = d.lay.ne;
+    const double sxx0 = sg[i], sxy = sg[i + ne], sxz = sg[i + 2 * ne];
+    const double syy0 = sg[i + 3 * ne], syz = sg[i + 4 * ne], szz0 = sg[i + 5 * ne];
+    const double skk = (sxx0 + syy0 + szz0) / 3.0;
+    const double sxx = sxx0 - skk, syy = syy0 - skk, szz = szz0 - skk;
+    const double tn = sqrt(sxx * sxx + syy * syy + szz * szz +
+                           2.0 * (sxy * sxy + sxz * sxz + syz * syz));
+    double f = 0.0;
+    for (int l = 0; l < d.nlaws; ++l) f += d.gamma[l * ne + i] * pow(tn, d.nexp[l * ne + i]);
+    e[0] = f * sxx;
+    e[1] = f * sxy;
+    e[2] = f * sxz;
+    e[3] = f * syy;
+    e[4] = f * syz;
+    e[5] = f * szz;
+}
+
 __global__ void __launch_bounds__(256) k_rhs_prologue(RhsDev d, const double *__restrict__ u,
                                                       double *__restrict__ du,
                                                       double *__restrict__ s,
@@ -53,17 +74,8 @@ __global__ void __launch_bounds__(256) k_rhs_prologue(RhsDev d, const double *__
     }
     const int64_t i = t - nf;
     if (i >= ne) return;
-    // update_strain_rate! + relative_strain_rate! (equation.jl:207-230)
-    const double *sg = u + d.lay.sig;
-    const double sxx0 = sg[i], sxy = sg[i + ne], sxz = sg[i + 2 * ne];
-    const double syy0 = sg[i + 3 * ne], syz = sg[i + 4 * ne], szz0 = sg[i + 5 * ne];
-    const double skk = (sxx0 + syy0 + szz0) / 3.0;
-    const double sxx = sxx0 - skk, syy = syy0 - skk, szz = szz0 - skk;
-    const double tn = sqrt(sxx * sxx + syy * syy + szz * szz +
-                           2.0 * (sxy * sxy + sxz * sxz + syz * syz));
-    double f = 0.0;
-    for (int l = 0; l < d.nlaws; ++l) f += d.gamma[l * ne + i] * pow(tn, d.nexp[l * ne + i]);
-    const double e[6] = {f * sxx, f * sxy, f * sxz, f * syy, f * syz, f * szz};
+    double e[6];
+    strain_rate(d, u + d.lay.sig, i, e);
     double *de = du + d.lay.eps;
 #pragma unroll
     for (int k = 0; k < 6; ++k) {
@@ -406,99 +418,13 @@ __global__ void __launch_bounds__(256) k_fft_kernel(const double *__restrict__ s
     }
 }
 
-// x1 <- x0 - w x1, x0 <- x0 + w x1 on registers
-__device__ __forceinline__ void bfly(double &r0, double &i0, double &r1, double &i1, double wr, double wi)
-{
-    const double xr = r1 * wr - i1 * wi, xi = r1 * wi + i1 * wr;
-    r1 = r0 - xr;
-    i1 = i0 - xi;
-    r0 += xr;
-    i0 += xi;
-}
+__device__ __forceinline__ int64_t bitrev(int64_t x, int bits) { return gsp_bitrev((int)x, bits); }  // bits >= 1
 
-// In-place radix-2 FFT of re/im[0..L) (bit-reversed input order), sign -1
-// (forward) or +1 (inverse); the block's threads share the butterflies of
-// each stage.  Stages len, 2len and 4len run together: a thread that owns
-// the eight entries p + k len/2 (k < 8) of a 4len-block holds every pair of
-// the three stages, so three stages cost one barrier (3 for L = 512 instead
-// of 9); one or two stages left over run the same way with four or two
-// entries per thread.
-__device__ __forceinline__ void lds_fft(double *re, double *im, int64_t L, const double *cs,
-                                        const double *sn, double sign)
+// the transform of a block's one sequence of length L
+__device__ __forceinline__ void lds_fft1(double *re, double *im, int64_t L, const double *cs, const double *sn,
+                                         double sign)
 {
-    int64_t len = 2;
-    for (; 4 * len <= L; len <<= 3) {
-        const int64_t half = len >> 1, s1 = L / len, s2 = s1 >> 1, s4 = s1 >> 2;
-        for (int64_t b = threadIdx.x; b < L / 8; b += blockDim.x) {
-            const int64_t p = b & (half - 1), a0 = (b - p) * 8 + p;
-            double r[8], i[8];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                r[k] = re[a0 + k * half];
-                i[k] = im[a0 + k * half];
-            }
-            const double w1r = cs[p * s1], w1i = sign * sn[p * s1];
-#pragma unroll
-            for (int k = 0; k < 8; k += 2) bfly(r[k], i[k], r[k + 1], i[k + 1], w1r, w1i);  // stage len
-#pragma unroll
-            for (int k = 0; k < 2; ++k) {  // stage 2len: positions p, p + half
-                const int64_t x = (p + k * half) * s2;
-                bfly(r[k], i[k], r[k + 2], i[k + 2], cs[x], sign * sn[x]);
-                bfly(r[k + 4], i[k + 4], r[k + 6], i[k + 6], cs[x], sign * sn[x]);
-            }
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {  // stage 4len: positions p + k half
-                const int64_t x = (p + k * half) * s4;
-                bfly(r[k], i[k], r[k + 4], i[k + 4], cs[x], sign * sn[x]);
-            }
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                re[a0 + k * half] = r[k];
-                im[a0 + k * half] = i[k];
-            }
-        }
-        __syncthreads();
-    }
-    if (2 * len <= L) {  // two stages left: len and 2len
-        const int64_t half = len >> 1, s1 = L / len, s2 = s1 >> 1;
-        for (int64_t b = threadIdx.x; b < L / 4; b += blockDim.x) {
-            const int64_t p = b & (half - 1), a0 = (b - p) * 4 + p, a1 = a0 + half, a2 = a0 + len,
-                          a3 = a2 + half;
-            double r0 = re[a0], i0 = im[a0], r1 = re[a1], i1 = im[a1];
-            double r2 = re[a2], i2 = im[a2], r3 = re[a3], i3 = im[a3];
-            const double w1r = cs[p * s1], w1i = sign * sn[p * s1];
-            bfly(r0, i0, r1, i1, w1r, w1i);
-            bfly(r2, i2, r3, i3, w1r, w1i);
-            bfly(r0, i0, r2, i2, cs[p * s2], sign * sn[p * s2]);
-            bfly(r1, i1, r3, i3, cs[(p + half) * s2], sign * sn[(p + half) * s2]);
-            re[a0] = r0;
-            im[a0] = i0;
-            re[a1] = r1;
-            im[a1] = i1;
-            re[a2] = r2;
-            im[a2] = i2;
-            re[a3] = r3;
-            im[a3] = i3;
-        }
-        __syncthreads();
-    } else if (len <= L) {  // one stage left (len == L)
-        const int64_t half = len >> 1, step = L / len;
-        for (int64_t b = threadIdx.x; b < L / 2; b += blockDim.x) {
-            const int64_t p = b & (half - 1), a0 = (b - p) * 2 + p, a1 = a0 + half;
-            double r0 = re[a0], i0 = im[a0], r1 = re[a1], i1 = im[a1];
-            bfly(r0, i0, r1, i1, cs[p * step], sign * sn[p * step]);
-            re[a0] = r0;
-            im[a0] = i0;
-            re[a1] = r1;
-            im[a1] = i1;
-        }
-        __syncthreads();
-    }
-}
-
-__device__ __forceinline__ int64_t bitrev(int64_t x, int bits)
-{
-    return (int64_t)(__brev((unsigned)x) >> (32 - bits));  // bits >= 1 since L >= 2
+    lds_fft(re, im, (int)L, 1, (int)L, cs, sn, 1, sign, (int)threadIdx.x, (int)blockDim.x);
 }
 
 // relative_velocity! (equation.jl:35-42) and the forward FFT of the padded
@@ -520,7 +446,7 @@ __global__ void __launch_bounds__(256) k_fft_fwd(RhsDev d, const double *__restr
         im[r] = 0.0;
     }
     __syncthreads();
-    lds_fft(re, im, L, cs, sn, -1.0);
+    lds_fft1(re, im, L, cs, sn, -1.0);
     for (int64_t f = threadIdx.x; f <= h; f += blockDim.x) {
         Sh[2 * (l + nxi * f)] = re[f];
         Sh[2 * (l + nxi * f) + 1] = im[f];
@@ -582,7 +508,7 @@ __global__ void __launch_bounds__(256) k_fft_fwd_stage(RhsDev d, StageCoef sc, c
         im[r] = 0.0;
     }
     __syncthreads();
-    lds_fft(re, im, L, cs, sn, -1.0);
+    lds_fft1(re, im, L, cs, sn, -1.0);
     for (int64_t f = threadIdx.x; f <= h; f += blockDim.x) {
         Sh[2 * (l + nxi * f)] = re[f];
         Sh[2 * (l + nxi * f) + 1] = im[f];
@@ -647,7 +573,7 @@ __global__ void __launch_bounds__(256) k_fft_inv(RhsDev d, const double *__restr
         }
     }
     __syncthreads();
-    lds_fft(re, im, L, cs, sn, 1.0);
+    lds_fft1(re, im, L, cs, sn, 1.0);
     // fault only: the rate-and-state update; coupled (ne > 0): the K_ff
     // traction rates go to du = tauff for the fault rows' K_fm pass
     for (int64_t n = threadIdx.x; n < nx; n += blockDim.x) {
@@ -1109,6 +1035,140 @@ __global__ void __launch_bounds__(256) k_expand_mf(const double *__restrict__ G,
     }
 }
 
+// ---------------- grid operator in the frequency domain (grid_spectral.h) ----------------
+static constexpr int kGspT = 512;  // threads of the transform kernels
+static constexpr int kGspM = 256;  // threads of the products
+
+// Blocks [0, nxi): fault rows; then the 6 nz mantle planes (component p of
+// layer iz), each of which forms its component of the strain rates.
+__global__ void __launch_bounds__(kGspT) k_gsp_fwd(RhsDev d, GridSpec g, const double *__restrict__ u,
+                                                   double *__restrict__ du)
+{
+    extern __shared__ double gsp_sh[];
+    const int b = (int)blockIdx.x, tid = (int)threadIdx.x;
+    if (b < g.nxi) {
+        const double *v = u + d.lay.v + (int64_t)g.nx * b;
+        gsp_fwd_fault(g, b, gsp_sh, tid, kGspT, [&](int n) { return v[n] - d.vpl; });
+        return;
+    }
+    const int PI = b - g.nxi, nz = g.npl / 6, p = PI / nz, iz = PI - p * nz;
+    const int64_t c0 = (int64_t)iz * g.nxc * g.ny;
+    const double *sg = u + d.lay.sig;
+    double *de = du + d.lay.eps + p * d.lay.ne;
+    gsp_fwd_plane(g, PI, gsp_sh, tid, kGspT, [&](int c) {
+        double e[6], x = 0.0;
+        strain_rate(d, sg, c0 + c, e);
+#pragma unroll
+        for (int k = 0; k < 6; ++k)
+            if (k == p) x = e[k];
+        de[c0 + c] = x;
+        return x - d.deps0[p];
+    });
+}
+
+__global__ void __launch_bounds__(kGspM) k_gsp_mul(GridSpec g, GspBlocks nb)
+{
+    extern __shared__ __attribute__((aligned(16))) double gsp_sh[];
+    double2 *red = reinterpret_cast<double2 *>(gsp_sh);
+    int b = (int)blockIdx.x;
+    const int tid = (int)threadIdx.x;
+    if (b < nb.f) {
+        gsp_mul_f(g, b, tid, kGspM);
+        return;
+    }
+    b -= nb.f;
+    if (b < nb.g) {
+        gsp_mul_g(g, b, tid, kGspM);
+        return;
+    }
+    b -= nb.g;
+    if (b < nb.m) {
+        gsp_mul_m1(g, b, red, tid, kGspM);
+        __syncthreads();
+        gsp_mul_m2(g, b, red, tid, kGspM);
+        return;
+    }
+    b -= nb.m;
+    gsp_mul_k1(g, b, red, tid, kGspM);
+    __syncthreads();
+    gsp_mul_k2(g, b, red, tid, kGspM);
+}
+
+// Blocks [0, nxi): fault rows and their rate-and-state update; then the planes' stress rates.
+__global__ void __launch_bounds__(kGspT) k_gsp_inv(RhsDev d, GridSpec g, const double *__restrict__ u,
+                                                   double *__restrict__ du)
+{
+    extern __shared__ double gsp_sh[];
+    const int b = (int)blockIdx.x, tid = (int)threadIdx.x;
+    if (b < g.nxi) {
+        const int64_t q0 = (int64_t)g.nx * b;
+        gsp_inv_fault(g, b, gsp_sh, tid, kGspT, [&](int n, double tau) { fault_update(d, q0 + n, tau, u, du); });
+        return;
+    }
+    const int PO = b - g.nxi;
+    double *ds = du + d.lay.sig + (int64_t)PO * g.nxc * g.ny;
+    gsp_inv_plane(g, PO, gsp_sh, tid, kGspT, [&](int c, double v) { ds[c] = v; });
+}
+
+// One-time spectra of the tables.  F: block (q, b), the row's D offsets in LDS.
+__global__ void __launch_bounds__(256) k_gsp_tab_f(GridSpec g, const double *__restrict__ F, int64_t D,
+                                                   double2 *__restrict__ out)
+{
+    extern __shared__ double gsp_sh[];
+    const int64_t q = blockIdx.x % g.Q, b = blockIdx.x / g.Q;
+    for (int64_t x = threadIdx.x; x < D; x += 256) gsp_sh[x] = F[(b * g.Q + q) * D + x];
+    __syncthreads();
+    for (int x = (int)threadIdx.x; x < g.H * g.m; x += 256) {
+        const int f = x / g.m, a0 = x - f * g.m;
+        out[((int64_t)f * g.Q + q) * g.RF + b * g.m + a0] = gsp_tab_f(g, gsp_sh, D, a0, f);
+    }
+}
+
+__global__ void __launch_bounds__(256) k_gsp_tab_g(GridSpec g, const double *__restrict__ G, int64_t D,
+                                                   double2 *__restrict__ out)
+{
+    extern __shared__ double gsp_sh[];
+    const int64_t q = blockIdx.x % g.Q, b = blockIdx.x / g.Q;
+    for (int64_t x = threadIdx.x; x < D; x += 256) gsp_sh[x] = G[(q * g.nxi + b) * D + x];
+    __syncthreads();
+    for (int x = (int)threadIdx.x; x < g.H * g.m; x += 256) {
+        const int f = x / g.m, a0 = x - f * g.m;
+        out[((int64_t)f * g.RF + b * g.m + a0) * g.Q + q] = gsp_tab_g(g, gsp_sh, D, a0, f);
+    }
+}
+
+// M along x: rows (PO, PI, yy) of the tiles, then along y into [fy][f][PI][PO].
+__global__ void __launch_bounds__(256) k_gsp_tab_mx(GridSpec g, const double *__restrict__ T, int nxp,
+                                                    double2 *__restrict__ X)
+{
+    const int64_t n = (int64_t)g.npl * g.npl * (2 * g.ny - 1) * g.H, Wp = 2 * nxp + 1;
+    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < n; t += (int64_t)gridDim.x * 256) {
+        const int64_t row = t / g.H;
+        X[t] = gsp_tab_mx(g, T + row * Wp, nxp, (int)(t - row * g.H));
+    }
+}
+
+__global__ void __launch_bounds__(256) k_gsp_tab_my(GridSpec g, const double2 *__restrict__ X, double2 *__restrict__ M)
+{
+    const int64_t np2 = (int64_t)g.npl * g.npl, n = np2 * g.Py * g.H, Wy = 2 * g.ny - 1;
+    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < n; t += (int64_t)gridDim.x * 256) {
+        const int64_t PO = t % g.npl, r = t / g.npl, PI = r % g.npl, w = r / g.npl;
+        const int fy = (int)(w / g.H), f = (int)(w - (int64_t)fy * g.H);
+        M[t] = gsp_tab_my(g, X + (PO * g.npl + PI) * Wy * g.H + f, fy);
+    }
+}
+
+static void gsp_enqueue(const oq_rhs *h, const double *u, double *du)
+{
+    const GridSpec &g = h->spec;
+    const size_t lds = (size_t)gsp_lds(g) * 8;
+    const GspBlocks nb = gsp_blocks(g, kGspM);
+    hipLaunchKernelGGL(k_gsp_fwd, dim3((unsigned)(g.nxi + g.npl)), dim3(kGspT), lds, h->stream, h->dev, g, u, du);
+    hipLaunchKernelGGL(k_gsp_mul, dim3((unsigned)(nb.f + nb.g + nb.m + nb.k)), dim3(kGspM),
+                       (size_t)gsp_red(g, kGspM) * 16, h->stream, g, nb);
+    hipLaunchKernelGGL(k_gsp_inv, dim3((unsigned)(g.nxi + g.npl)), dim3(kGspT), lds, h->stream, h->dev, g, u, du);
+}
+
 static inline size_t fft_lds(int64_t nx) { return (size_t)(3 * fft_len(nx)) * 8; }
 
 // LDS bytes of a block with lchunk dip rows
@@ -1167,6 +1227,11 @@ static int grid_lds_attrs(size_t lds)
 
 int rhs_enqueue_matvec(oq_rhs *h, const double *u, double *du)
 {
+    if (h->spectral) {  // the strain rates and sources are formed there
+        gsp_enqueue(h, u, du);
+        OQ_HIP(hipGetLastError());
+        return OQ_OK;
+    }
     if (h->kdtype == OQ_K_FFT && h->ne > 0) {
         // coupled model (equation.jl:185-205 with dτ_dt! by DFT, :200): K_ff s_f
         // by the DFT convolution into tauff, then the fault rows' K_fm s_m plus
@@ -1262,7 +1327,7 @@ int rhs_enqueue_fft_stage(oq_rhs *h, const StageCoef &sc, const double *dtp, con
 
 int rhs_enqueue(oq_rhs *h, const double *u, double *du)
 {
-    if (h->kdtype == OQ_K_FFT && h->ne == 0) return rhs_enqueue_matvec(h, u, du);  // s is formed there
+    if (h->spectral || (h->kdtype == OQ_K_FFT && h->ne == 0)) return rhs_enqueue_matvec(h, u, du);  // s is formed there
     const int64_t n = h->nf + h->ne;
     hipLaunchKernelGGL(k_rhs_prologue, dim3(nblk(n, 256)), dim3(256), 0, h->stream, h->dev, u, du,
                        h->s64.as<double>(), h->kdtype == OQ_K_BF16 ? h->s32.as<float>() : nullptr,
@@ -1857,6 +1922,58 @@ static int dense_blocks(const oq_fault_mesh *mf, const oq_hex8_mesh *ma, const F
     return OQ_OK;
 }
 
+// Spectra of the tables (h->spec with its shape set; Ftab, Gtab, Tmm and the
+// DFT K_ff in place) and the work buffer of the three launches.
+static int gsp_build(oq_rhs *h)
+{
+    GridSpec &g = h->spec;
+    const int64_t D = h->grid.D, HQR = (int64_t)g.H * g.Q * g.RF, np2 = (int64_t)g.npl * g.npl, PH = (int64_t)g.Py * g.H;
+    std::vector<double> tw((size_t)g.Lt);
+    for (int64_t k = 0; k < g.Lt / 2; ++k) {
+        tw[(size_t)k] = cos(2.0 * M_PI * (double)k / (double)g.Lt);
+        tw[(size_t)(g.Lt / 2 + k)] = sin(2.0 * M_PI * (double)k / (double)g.Lt);
+    }
+    const int64_t sz[8] = {(int64_t)g.H * g.Q, (int64_t)g.H * g.RF, PH * g.npl, (int64_t)g.hb * g.nxi,
+                           (int64_t)g.nfs * g.H * g.RF, (int64_t)g.ngs * g.H * g.Q, PH * g.npl, (int64_t)g.hb * g.nxi};
+    int64_t tot = 0;
+    for (int64_t n : sz) tot += n;
+    DevBuf X;
+    int rc = h->spTw.upload(tw.data(), tw.size() * 8, h->stream);
+    if (!rc) rc = h->spF.alloc_reuse((size_t)HQR * 16);
+    if (!rc) rc = h->spG.alloc_reuse((size_t)HQR * 16);
+    if (!rc) rc = h->spM.alloc_reuse((size_t)(np2 * PH) * 16);
+    if (!rc) rc = h->spW.alloc((size_t)tot * 16);
+    if (!rc) rc = X.alloc_reuse((size_t)(np2 * (2 * g.ny - 1) * g.H) * 16);
+    if (rc) return rc;
+    double2 *w = h->spW.as<double2>();
+    double2 **dst[8] = {&g.Sm, &g.Sf, &g.S2, &g.Sk, &g.Of, &g.Og, &g.Om, &g.Ok};
+    for (int i = 0; i < 8; ++i) {
+        *dst[i] = w;
+        w += sz[i];
+    }
+    g.tw = h->spTw.as<double>();
+    g.K = h->fg.as<double>();
+    g.F = h->spF.as<double2>();
+    g.G = h->spG.as<double2>();
+    g.M = h->spM.as<double2>();
+    const unsigned rows = (unsigned)((int64_t)g.Q * g.nxi);
+    hipLaunchKernelGGL(k_gsp_tab_f, dim3(rows), dim3(256), (size_t)D * 8, h->stream, g, h->Ftab.as<double>(), D,
+                       h->spF.as<double2>());
+    hipLaunchKernelGGL(k_gsp_tab_g, dim3(rows), dim3(256), (size_t)D * 8, h->stream, g, h->Gtab.as<double>(), D,
+                       h->spG.as<double2>());
+    hipLaunchKernelGGL(k_gsp_tab_mx, dim3(grid_capped(np2 * (2 * g.ny - 1) * g.H, 256)), dim3(256), 0, h->stream, g,
+                       h->Tmm.as<double>(), h->grid.nxp, X.as<double2>());
+    hipLaunchKernelGGL(k_gsp_tab_my, dim3(grid_capped(np2 * PH, 256)), dim3(256), 0, h->stream, g, X.as<double2>(),
+                       h->spM.as<double2>());
+    OQ_HIP(hipGetLastError());
+    const int lds = (int)(gsp_lds(g) * 8);
+    OQ_HIP(hipFuncSetAttribute((const void *)k_gsp_fwd, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    OQ_HIP(hipFuncSetAttribute((const void *)k_gsp_inv, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    OQ_HIP(hipStreamSynchronize(h->stream));
+    h->spectral = true;
+    return OQ_OK;
+}
+
 // Fused or split launches for the grid model: 20 operator applications of
 // each on zeroed state after 3 of warm-up, keep the faster (ties: fused).
 static int mm_grid_pick(oq_rhs *h)
@@ -1971,6 +2088,143 @@ static void destroy(oq_rhs *h)
     delete h;
 }
 
+static int create_from_mesh(int device, const oq_fault_mesh *mf, const oq_hex8_mesh *ma, double lambda, double mu,
+                            int ftype, int64_t nrept, double buffer_ratio, const oq_quadrature *quad,
+                            const oq_rs_props *fault, const oq_visc_props *visc, int kdtype, bool batch, oq_rhs **out)
+{
+    OQ_REQUIRE(out != nullptr, "out is NULL");
+    *out = nullptr;
+    int rc;
+    if ((rc = check_fault(mf))) return rc;
+    OQ_REQUIRE(ftype == 0 || ftype == 1, "ftype must be StrikeSlip (0) or DipSlip (1)");
+    OQ_REQUIRE(buffer_ratio >= 0.0, "Argument `buffer_ratio` must be ≥ 0.");
+    OQ_REQUIRE(nrept >= 0, "nrept must be >= 0");
+    const int64_t ne = ma ? ma->ne : 0;
+    if (ma && (rc = check_hex8(ma))) return rc;
+    if (ma && (rc = check_quad(quad))) return rc;
+    // OQ_K_FFT_GRID = the coupled OQ_K_FFT model with K_mm on the mantle grid
+    const bool grid = kdtype == OQ_K_FFT_GRID;
+    MmGrid g;
+    double hx = 0.0, hy = 0.0;
+    if (grid) {
+        OQ_REQUIRE(ne > 0, "OQ_K_FFT_GRID is for the coupled model (a hex8 mantle)");
+        const char *why = mm_grid_detect(ma, g, hx, hy);
+        OQ_REQUIRE(why == nullptr, why);
+        kdtype = OQ_K_FFT;
+    }
+    oq_rhs *h = new oq_rhs();
+    rc = alloc_common(h, device, mf->nx, mf->nxi, ne, kdtype);
+    if (!rc && grid) {
+        h->mmgrid = true;
+        h->grid = g;
+        rc = mm_grid_shape(h->grid);
+        if (!rc)
+            h->grid.strike = mm_strike_detect(mf, h->grid, hx) && mm_strike_shape(h->grid, mf->nx, mf->nxi);
+    }
+    if (!rc) rc = upload_props(h, fault, visc);
+    FaultUpload fu;
+    Hex8Upload hu;
+    QuadUpload qu;
+    DevBuf k64, st;
+    if (!rc) rc = fu.load(mf);
+    if (!rc) fu.dev.lrept = (buffer_ratio + 1.0) * (mf->dx * (double)mf->nx);
+    if (!rc && ma) rc = hu.load(ma);
+    if (!rc && ma) rc = qu.load(quad);
+    const int64_t nf = h->nf, ld = h->ld;
+    if (!rc && kdtype == OQ_K_FFT && ne > 0) {
+        rc = st.alloc((size_t)(nf * mf->nxi) * 8);
+        if (!rc) rc = launch_gf_ff(fu.dev, lambda, mu, ftype, (int)nrept, st.as<double>(), h->stream);
+        if (!rc && hipStreamSynchronize(h->stream) != hipSuccess) rc = OQ_ERR_HIP;
+        if (!rc) rc = fft_coupled_alloc(h, st);
+        if (h->mmgrid && h->grid.strike) {
+            if (!rc)
+                rc = mm_strike_build(mf, ma, h->grid, fu.dev.lrept, qu, lambda, mu, ftype, (int)nrept, h->Ftab,
+                                          h->Gtab, h->stream);
+        } else if (h->mmgrid) {
+            if (!rc) rc = launch_gf_fm(hu.dev, fu.dev, lambda, mu, ftype, h->Kf.as<double>(), h->ldm, 1, h->stream);
+            if (!rc)
+                rc = launch_gf_mf(fu.dev, hu.dev, qu.c.as<double>(), qu.w.as<double>(), qu.nq, lambda, mu, ftype,
+                                  (int)nrept, h->K.as<double>(), h->ldf, 1, h->stream);
+        }
+        if (!rc && h->mmgrid) {
+            rc = mm_grid_build(ma, h->grid, h->grid.nxp, hx, hy, qu, lambda, mu, h->Tmm, h->stream);
+            const MmGrid &gg = h->grid;
+            if (!rc && gg.strike && gg.D * 8 <= 64 * 1024 &&
+                gsp_shape(h->spec, mf->nx, mf->nxi, gg.m, gg.nx, gg.ny, gg.nz, kGspM, 160 * 1024)) {
+                rc = gsp_build(h);
+            } else {
+                if (!rc) rc = mm_grid_parts(h);
+                if (!rc) rc = mm_roles_build(h);
+                if (!rc) rc = mm_grid_pick(h);
+            }
+        } else if (!rc) {
+            rc = dense_blocks(mf, ma, fu, hu, quad, qu, lambda, mu, ftype, (int)nrept, h->Kf.as<double>(), h->ldm,
+                              h->K.as<double>(), h->K.as<double>() + nf, ld, h->stream);
+        }
+        if (!rc && hipStreamSynchronize(h->stream) != hipSuccess) {
+            set_error("device assembly failed");
+            rc = OQ_ERR_HIP;
+        }
+        if (rc) {
+            destroy(h);
+            return rc;
+        }
+        *out = h;
+        return OQ_OK;
+    }
+    if (!rc && (kdtype == OQ_K_TOEPLITZ || kdtype == OQ_K_FFT)) {
+        rc = st.alloc((size_t)(nf * mf->nxi) * 8);
+        if (!rc) rc = launch_gf_ff(fu.dev, lambda, mu, ftype, (int)nrept, st.as<double>(), h->stream);
+        if (!rc && hipStreamSynchronize(h->stream) != hipSuccess) {
+            set_error("device assembly failed");
+            rc = OQ_ERR_HIP;
+        }
+        if (!rc) rc = finalize_toeplitz(h, st);
+        if (rc) {
+            destroy(h);
+            return rc;
+        }
+        *out = h;
+        return OQ_OK;
+    }
+    if (!rc) rc = k64.alloc_reuse((size_t)(h->N * ld) * 8);
+    if (!rc) rc = clear_padding(k64.as<double>(), h);
+    if (!rc) rc = st.alloc((size_t)(nf * mf->nxi) * 8);
+    if (!rc) rc = launch_gf_ff(fu.dev, lambda, mu, ftype, (int)nrept, st.as<double>(), h->stream);
+    if (!rc) rc = launch_expand_toeplitz(st.as<double>(), mf->nx, mf->nxi, k64.as<double>(), ld, h->stream);
+    if (!rc && ne > 0) {
+        double *K = k64.as<double>();
+        if (batch) {
+            rc = launch_gf_mf(fu.dev, hu.dev, qu.c.as<double>(), qu.w.as<double>(), qu.nq, lambda, mu, ftype,
+                              (int)nrept, K + nf * ld, ld, 1, h->stream);
+            if (!rc)
+                rc = launch_gf_hex8_seq(hu.dev, fu.dev, qu.c.as<double>(), qu.w.as<double>(), qu.nq, lambda, mu, ftype,
+                                        K + nf, K + nf * ld + nf, ld, h->stream);
+        } else {
+            rc = dense_blocks(mf, ma, fu, hu, quad, qu, lambda, mu, ftype, (int)nrept, K + nf, ld, K + nf * ld,
+                              K + nf * ld + nf, ld, h->stream);
+        }
+    }
+    if (!rc && hipStreamSynchronize(h->stream) != hipSuccess) {
+        set_error("device assembly failed");
+        rc = OQ_ERR_HIP;
+    }
+    if (!rc) rc = finalize_k(h, k64);
+    if (rc) {
+        destroy(h);
+        return rc;
+    }
+    *out = h;
+    return OQ_OK;
+}
+
+int rhs_create_for_batch(int device, const oq_fault_mesh *mf, const oq_hex8_mesh *ma, double lambda, double mu, int ftype,
+                         int64_t nrept, double buffer_ratio, const oq_quadrature *quad, const oq_rs_props *fault,
+                         const oq_visc_props *visc, int kdtype, oq_rhs **out)
+{
+    return create_from_mesh(device, mf, ma, lambda, mu, ftype, nrept, buffer_ratio, quad, fault, visc, kdtype, true, out);
+}
+
 }  // namespace oq
 
 using namespace oq;
@@ -2082,116 +2336,8 @@ int oq_rhs_create_from_mesh(int device, const oq_fault_mesh *mf, const oq_hex8_m
                             const oq_rs_props *fault, const oq_visc_props *visc, int kdtype,
                             oq_rhs **out)
 {
-    OQ_REQUIRE(out != nullptr, "out is NULL");
-    *out = nullptr;
-    int rc;
-    if ((rc = check_fault(mf))) return rc;
-    OQ_REQUIRE(ftype == 0 || ftype == 1, "ftype must be StrikeSlip (0) or DipSlip (1)");
-    OQ_REQUIRE(buffer_ratio >= 0.0, "Argument `buffer_ratio` must be ≥ 0.");
-    OQ_REQUIRE(nrept >= 0, "nrept must be >= 0");
-    const int64_t ne = ma ? ma->ne : 0;
-    if (ma && (rc = check_hex8(ma))) return rc;
-    if (ma && (rc = check_quad(quad))) return rc;
-    // OQ_K_FFT_GRID = the coupled OQ_K_FFT model with K_mm on the mantle grid
-    const bool grid = kdtype == OQ_K_FFT_GRID;
-    MmGrid g;
-    double hx = 0.0, hy = 0.0;
-    if (grid) {
-        OQ_REQUIRE(ne > 0, "OQ_K_FFT_GRID is for the coupled model (a hex8 mantle)");
-        const char *why = mm_grid_detect(ma, g, hx, hy);
-        OQ_REQUIRE(why == nullptr, why);
-        kdtype = OQ_K_FFT;
-    }
-    oq_rhs *h = new oq_rhs();
-    rc = alloc_common(h, device, mf->nx, mf->nxi, ne, kdtype);
-    if (!rc && grid) {
-        h->mmgrid = true;
-        h->grid = g;
-        rc = mm_grid_shape(h->grid);
-        if (!rc)
-            h->grid.strike = mm_strike_detect(mf, h->grid, hx) && mm_strike_shape(h->grid, mf->nx, mf->nxi);
-    }
-    if (!rc) rc = upload_props(h, fault, visc);
-    FaultUpload fu;
-    Hex8Upload hu;
-    QuadUpload qu;
-    DevBuf k64, st;
-    if (!rc) rc = fu.load(mf);
-    if (!rc) fu.dev.lrept = (buffer_ratio + 1.0) * (mf->dx * (double)mf->nx);
-    if (!rc && ma) rc = hu.load(ma);
-    if (!rc && ma) rc = qu.load(quad);
-    const int64_t nf = h->nf, ld = h->ld;
-    if (!rc && kdtype == OQ_K_FFT && ne > 0) {
-        rc = st.alloc((size_t)(nf * mf->nxi) * 8);
-        if (!rc) rc = launch_gf_ff(fu.dev, lambda, mu, ftype, (int)nrept, st.as<double>(), h->stream);
-        if (!rc && hipStreamSynchronize(h->stream) != hipSuccess) rc = OQ_ERR_HIP;
-        if (!rc) rc = fft_coupled_alloc(h, st);
-        if (h->mmgrid && h->grid.strike) {
-            if (!rc)
-                rc = mm_strike_build(mf, ma, h->grid, fu.dev.lrept, qu, lambda, mu, ftype, (int)nrept, h->Ftab,
-                                          h->Gtab, h->stream);
-        } else if (h->mmgrid) {
-            if (!rc) rc = launch_gf_fm(hu.dev, fu.dev, lambda, mu, ftype, h->Kf.as<double>(), h->ldm, 1, h->stream);
-            if (!rc)
-                rc = launch_gf_mf(fu.dev, hu.dev, qu.c.as<double>(), qu.w.as<double>(), qu.nq, lambda, mu, ftype,
-                                  (int)nrept, h->K.as<double>(), h->ldf, 1, h->stream);
-        }
-        if (!rc && h->mmgrid) {
-            rc = mm_grid_build(ma, h->grid, h->grid.nxp, hx, hy, qu, lambda, mu, h->Tmm, h->stream);
-            if (!rc) rc = mm_grid_parts(h);
-            if (!rc) rc = mm_roles_build(h);
-            if (!rc) rc = mm_grid_pick(h);
-        } else if (!rc) {
-            rc = dense_blocks(mf, ma, fu, hu, quad, qu, lambda, mu, ftype, (int)nrept, h->Kf.as<double>(), h->ldm,
-                              h->K.as<double>(), h->K.as<double>() + nf, ld, h->stream);
-        }
-        if (!rc && hipStreamSynchronize(h->stream) != hipSuccess) {
-            set_error("device assembly failed");
-            rc = OQ_ERR_HIP;
-        }
-        if (rc) {
-            destroy(h);
-            return rc;
-        }
-        *out = h;
-        return OQ_OK;
-    }
-    if (!rc && (kdtype == OQ_K_TOEPLITZ || kdtype == OQ_K_FFT)) {
-        rc = st.alloc((size_t)(nf * mf->nxi) * 8);
-        if (!rc) rc = launch_gf_ff(fu.dev, lambda, mu, ftype, (int)nrept, st.as<double>(), h->stream);
-        if (!rc && hipStreamSynchronize(h->stream) != hipSuccess) {
-            set_error("device assembly failed");
-            rc = OQ_ERR_HIP;
-        }
-        if (!rc) rc = finalize_toeplitz(h, st);
-        if (rc) {
-            destroy(h);
-            return rc;
-        }
-        *out = h;
-        return OQ_OK;
-    }
-    if (!rc) rc = k64.alloc_reuse((size_t)(h->N * ld) * 8);
-    if (!rc) rc = clear_padding(k64.as<double>(), h);
-    if (!rc) rc = st.alloc((size_t)(nf * mf->nxi) * 8);
-    if (!rc) rc = launch_gf_ff(fu.dev, lambda, mu, ftype, (int)nrept, st.as<double>(), h->stream);
-    if (!rc) rc = launch_expand_toeplitz(st.as<double>(), mf->nx, mf->nxi, k64.as<double>(), ld, h->stream);
-    if (!rc && ne > 0) {
-        double *K = k64.as<double>();
-        rc = dense_blocks(mf, ma, fu, hu, quad, qu, lambda, mu, ftype, (int)nrept, K + nf, ld, K + nf * ld,
-                          K + nf * ld + nf, ld, h->stream);
-    }
-    if (!rc && hipStreamSynchronize(h->stream) != hipSuccess) {
-        set_error("device assembly failed");
-        rc = OQ_ERR_HIP;
-    }
-    if (!rc) rc = finalize_k(h, k64);
-    if (rc) {
-        destroy(h);
-        return rc;
-    }
-    *out = h;
-    return OQ_OK;
+    return create_from_mesh(device, mf, ma, lambda, mu, ftype, nrept, buffer_ratio, quad, fault, visc, kdtype, false,
+                            out);
 }
 
 int oq_rhs_eval(oq_rhs *h, double t, const double *v, const double *theta, const double *eps,
@@ -2295,7 +2441,8 @@ int oq_rhs_info(oq_rhs *h, int64_t *nstate, int64_t *n, int64_t *kbytes)
     if (nstate) *nstate = h->lay.n;
     if (n) *n = h->N;
     if (kbytes)
-        *kbytes = (int64_t)(h->K.bytes + h->Kf.bytes + h->stk.bytes + h->Tmm.bytes + h->Ftab.bytes + h->Gtab.bytes);
+        *kbytes = (int64_t)(h->K.bytes + h->Kf.bytes + h->stk.bytes + h->Tmm.bytes + h->Ftab.bytes + h->Gtab.bytes +
+                             h->spF.bytes + h->spG.bytes + h->spM.bytes);
     return OQ_OK;
 }
 

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "grid_spectral.h"
 #include "oq_internal.h"
 
 namespace oq {
@@ -235,6 +236,10 @@ struct oq_rhs {
     oq::DevBuf Ftab, Gtab, roles, roles2;  // along-strike tables; block roles (fused, interleaved; split:
                                            // convolutions first)
     bool mmgrid = false;
+    // the grid operator in the frequency domain (strike grids whose transforms fit LDS)
+    bool spectral = false;
+    oq::GridSpec spec{};
+    oq::DevBuf spF, spG, spM, spTw, spW;
     int64_t ldf = 0;
     oq::MmGrid grid{};
     oq::RhsDev dev{};
@@ -242,6 +247,11 @@ struct oq_rhs {
 };
 
 namespace oq {
+// oq_rhs_create_from_mesh for the operator of a lockstep batch: every pair
+// evaluated, by the batch's own hex8 kernels.
+int rhs_create_for_batch(int device, const oq_fault_mesh *mf, const oq_hex8_mesh *ma, double lambda, double mu, int ftype,
+                         int64_t nrept, double buffer_ratio, const oq_quadrature *quad, const oq_rs_props *fault,
+                         const oq_visc_props *visc, int kdtype, oq_rhs **out);
 // Enqueues one RHS evaluation du = f(u) on h->stream (device pointers).
 int rhs_enqueue(oq_rhs *h, const double *u, double *du);
 // Enqueues only the K-streaming kernel (requires a prior prologue).

@@ -1,0 +1,40 @@
+"""The grid operator against the dense operator of the same meshes: shapes at
+the edges of its transforms (one residue, lengths that fill or just pass a
+power of two, more columns than patches, one row or layer), and a grid whose
+transforms exceed a workgroup's LDS, which keeps the convolution blocks.
+
+Both are FP64; the transforms' rounding is a few eps of the row norms, so
+every component agrees to 1e-12 in norm (the bound of the other operators)."""
+import numpy as np
+import pytest
+
+import oetqf_amd as oq
+from helpers import relerr, rs_props, visc_props
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("nx,nxi,dip,cells,rfzh", [
+    (8, 2, 90.0, (8, 3, 1), None),             # m = 1, one layer
+    (9, 3, 90.0, (3, 4, 2), [1.0, 2.0]),       # m = 3
+    (17, 2, 60.0, (17, 1, 2), None),           # one row, P = 64 for 33 offsets
+    (16, 5, 90.0, (4, 16, 1), None),           # Py = 32 filled
+    (34, 2, 90.0, (2, 17, 1), [1.0]),          # m = 17, Py = 64
+    (34, 1, 90.0, (34, 34, 1), None),          # P = Py = 128: beyond the LDS
+])
+def test_grid_operator_matches_dense(rng, nx, nxi, dip, cells, rfzh):
+    mf = oq.gen_mesh("RectOkada", 40e3, 12e3, 40e3 / nx, 12e3 / nxi, dip)
+    ma = oq.hex8_box(-20e3, -7e3, -9e3, 40e3, 13e3, -12e3, *cells, rfzh=rfzh)
+    pf, pa = rs_props(mf, rng), visc_props(ma, rng, 2.0)
+    v = pf.vpl * np.exp(rng.standard_normal(pf.a.shape))
+    u = oq.ArrayPartition(v, pf.L / v, np.zeros((ma.ne, 6)), 1e6 * rng.standard_normal((ma.ne, 6)), np.zeros(pf.a.shape))
+    du = []
+    for kd in ("fft_grid", "fp64"):
+        p = oq.assemble_from_mesh(mf, ma, 3e10, 2e10, pf, pa, u, (0.0, 1.0), ftype=oq.DipSlip(), kdtype=kd)
+        d = oq.similar(u)
+        for _ in range(2):  # the second on used work buffers
+            p.f(d, u, None, 0.0)
+        du.append(d)
+        p.f.close()
+    for k in range(5):
+        assert relerr(du[0].x[k], du[1].x[k]) <= 1e-12, k
