@@ -940,6 +940,7 @@ struct oq_ensemble {
     oq::EnsH3 h3{};
     oq::DevBuf a, b, L, sigma, eta, vpl, f0, v0, S;
     oq::DevBuf u, y, k, part;
+    oq::DevBuf xfer;  // oq_ensemble_eval: states in the host's layout
     oq::DevBuf ct, cdt, cdtcur, cqold, cna, cnr, citer, cdone, cacc, cret;
     oq::DevBuf vpart, rec_t, rec_v;  // recorder (oq_ensemble_record)
     oq::DevBuf live;                 // EnsDev::live
@@ -1236,18 +1237,17 @@ int oq_ensemble_eval(oq_ensemble *e, const double *u, double *du)
     oq_rhs *h = e->h;
     OQ_HIP(hipSetDevice(h->device));
     const int64_t nM = e->n * e->M;
-    std::vector<const double *> src(e->M);
-    for (int64_t m = 0; m < e->M; ++m) src[m] = u + m * e->n;
-    const std::vector<double> ui = interleave(src.data(), e->n, e->M);
-    OQ_HIP(hipMemcpyAsync(e->y.p, ui.data(), (size_t)nM * 8, hipMemcpyHostToDevice, h->stream));
-    int rc = set_live(e);
-    if (!rc) rc = ens_rhs(e, e->y.as<double>(), e->k.as<double>());
+    int rc = e->xfer.p ? OQ_OK : e->xfer.alloc((size_t)nM * 8);
     if (rc) return rc;
-    std::vector<double> o((size_t)nM);
-    OQ_HIP(hipMemcpyAsync(o.data(), e->k.p, (size_t)nM * 8, hipMemcpyDeviceToHost, h->stream));
+    double *x = e->xfer.as<double>(), *y = e->y.as<double>(), *k = e->k.as<double>();
+    OQ_HIP(hipMemcpyAsync(x, u, (size_t)nM * 8, hipMemcpyHostToDevice, h->stream));
+    rc = launch_transpose(x, e->M, e->n, y, h->stream);
+    if (!rc) rc = set_live(e);
+    if (!rc) rc = ens_rhs(e, y, k);
+    if (!rc) rc = launch_transpose(k, e->n, e->M, x, h->stream);
+    if (rc) return rc;
+    OQ_HIP(hipMemcpyAsync(du, x, (size_t)nM * 8, hipMemcpyDeviceToHost, h->stream));
     OQ_HIP(hipStreamSynchronize(h->stream));
-    for (int64_t m = 0; m < e->M; ++m)
-        for (int64_t i = 0; i < e->n; ++i) du[m * e->n + i] = o[(size_t)(i * e->M + m)];
     return OQ_OK;
 }
 
@@ -1285,11 +1285,11 @@ static int ens_begin(oq_ensemble *e, const double *u0, const double *tv, const d
         OQ_HIP(hipStreamSynchronize(h->stream));
     }
     e->alg = alg;
-    std::vector<const double *> src(M);
-    for (int64_t m = 0; m < M; ++m) src[m] = u0 + m * e->n;
-    const std::vector<double> ui = interleave(src.data(), e->n, M);
     const std::vector<int> zi(M, 0);
-    OQ_HIP(hipMemcpyAsync(e->u.p, ui.data(), (size_t)nM * 8, hipMemcpyHostToDevice, h->stream));
+    // through y, which every step writes before it reads it
+    OQ_HIP(hipMemcpyAsync(e->y.p, u0, (size_t)nM * 8, hipMemcpyHostToDevice, h->stream));
+    int rc = launch_transpose(e->y.as<double>(), M, e->n, e->u.as<double>(), h->stream);
+    if (rc) return rc;
     OQ_HIP(hipMemcpyAsync(e->ct.p, tv, M * 8, hipMemcpyHostToDevice, h->stream));
     OQ_HIP(hipMemcpyAsync(e->cdt.p, dtv, M * 8, hipMemcpyHostToDevice, h->stream));
     OQ_HIP(hipMemcpyAsync(e->cqold.p, qv, M * 8, hipMemcpyHostToDevice, h->stream));
@@ -1313,7 +1313,7 @@ static int ens_begin(oq_ensemble *e, const double *u0, const double *tv, const d
     e->rec_drained.assign(na, na + M);  // records from before a resume are not in the rings
     // FSAL seed: k1 = f(u) (on a resume the same bits as the k7 of the last
     // accepted step: the RHS kernels are deterministic); for VCABM5 phi_0 = f(u)
-    int rc = set_live(e);
+    rc = set_live(e);
     if (!rc) rc = ens_rhs(e, e->u.as<double>(), e->k.as<double>());
     if (rc) return rc;
     drop_graphs(e);
@@ -1502,15 +1502,12 @@ int oq_ensemble_state(oq_ensemble *e, double *t, double *u, int64_t *naccept, in
     if (naccept) OQ_HIP(hipMemcpyAsync(naccept, e->cna.p, M * 8, hipMemcpyDeviceToHost, h->stream));
     if (nreject) OQ_HIP(hipMemcpyAsync(nreject, e->cnr.p, M * 8, hipMemcpyDeviceToHost, h->stream));
     if (retcode) OQ_HIP(hipMemcpyAsync(retcode, e->cret.p, M * 4, hipMemcpyDeviceToHost, h->stream));
-    std::vector<double> o;
-    if (u) {
-        o.resize((size_t)nM);
-        OQ_HIP(hipMemcpyAsync(o.data(), e->u.p, (size_t)nM * 8, hipMemcpyDeviceToHost, h->stream));
+    if (u) {  // through y, scratch between steps
+        const int rc = launch_transpose(e->u.as<double>(), e->n, M, e->y.as<double>(), h->stream);
+        if (rc) return rc;
+        OQ_HIP(hipMemcpyAsync(u, e->y.p, (size_t)nM * 8, hipMemcpyDeviceToHost, h->stream));
     }
     OQ_HIP(hipStreamSynchronize(h->stream));
-    if (u)
-        for (int64_t m = 0; m < M; ++m)
-            for (int64_t i = 0; i < e->n; ++i) u[m * e->n + i] = o[(size_t)(i * M + m)];
     return OQ_OK;
 }
 

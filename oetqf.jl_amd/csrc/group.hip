@@ -1225,6 +1225,7 @@ struct oq_group {
     oq::DevBuf P;         // partial row sums of the units (capacity pcap doubles)
     size_t pcap = 0;
     oq::DevBuf u, y, k, part;
+    oq::DevBuf xfer;  // oq_group_eval: states in the host's layout
     oq::DevBuf ct, cdt, cdtcur, cqold, cna, cnr, citer, cdone, cacc, cret;
     oq::DevBuf live;  // GrpDev::live
     oq::GrpDev dev{};
@@ -1532,31 +1533,23 @@ static void grp_destroy(oq_group *e)
     delete e;
 }
 
-// host member-major states (geometry g: M members of n_g entries) <-> device
-// entry-major segments
-static void to_entry_major(const oq_group *e, const double *src, std::vector<double> &dst)
+// Member-major states (geometry g: M members of n_g entries, the host's
+// layout) <-> entry-major segments, both on the device.  soffs holds the
+// offsets of both: a segment has n_g M entries either way.
+static int to_entry_major(const oq_group *e, const double *src, double *dst)
 {
-    dst.resize((size_t)e->ntot);
-    const int64_t M = e->M;
-    int64_t hoff = 0;
-    for (int64_t g = 0; g < e->G; ++g) {
-        const int64_t n = e->nst[g], base = e->soffs[g];
-        for (int64_t m = 0; m < M; ++m)
-            for (int64_t i = 0; i < n; ++i) dst[(size_t)(base + i * M + m)] = src[hoff + m * n + i];
-        hoff += n * M;
-    }
+    int rc = OQ_OK;
+    for (int64_t g = 0; g < e->G && !rc; ++g)
+        rc = launch_transpose(src + e->soffs[g], e->M, e->nst[g], dst + e->soffs[g], e->stream);
+    return rc;
 }
 
-static void from_entry_major(const oq_group *e, const std::vector<double> &src, double *dst)
+static int from_entry_major(const oq_group *e, const double *src, double *dst)
 {
-    const int64_t M = e->M;
-    int64_t hoff = 0;
-    for (int64_t g = 0; g < e->G; ++g) {
-        const int64_t n = e->nst[g], base = e->soffs[g];
-        for (int64_t m = 0; m < M; ++m)
-            for (int64_t i = 0; i < n; ++i) dst[hoff + m * n + i] = src[(size_t)(base + i * M + m)];
-        hoff += n * M;
-    }
+    int rc = OQ_OK;
+    for (int64_t g = 0; g < e->G && !rc; ++g)
+        rc = launch_transpose(src + e->soffs[g], e->nst[g], e->M, dst + e->soffs[g], e->stream);
+    return rc;
 }
 
 }  // namespace oq
@@ -1875,16 +1868,18 @@ int oq_group_eval(oq_group *e, const double *u, double *du)
 {
     OQ_REQUIRE(e && u && du, "NULL argument");
     OQ_HIP(hipSetDevice(e->device));
-    std::vector<double> ui;
-    to_entry_major(e, u, ui);
-    OQ_HIP(hipMemcpyAsync(e->y.p, ui.data(), ui.size() * 8, hipMemcpyHostToDevice, e->stream));
-    int rc = set_live(e);
-    if (!rc) rc = grp_rhs(e, e->y.as<double>(), e->k.as<double>());
+    const size_t nb = (size_t)e->ntot * 8;
+    int rc = e->xfer.p ? OQ_OK : e->xfer.alloc(nb);
     if (rc) return rc;
-    std::vector<double> o((size_t)e->ntot);
-    OQ_HIP(hipMemcpyAsync(o.data(), e->k.p, o.size() * 8, hipMemcpyDeviceToHost, e->stream));
+    double *x = e->xfer.as<double>();
+    OQ_HIP(hipMemcpyAsync(x, u, nb, hipMemcpyHostToDevice, e->stream));
+    rc = to_entry_major(e, x, e->y.as<double>());
+    if (!rc) rc = set_live(e);
+    if (!rc) rc = grp_rhs(e, e->y.as<double>(), e->k.as<double>());
+    if (!rc) rc = from_entry_major(e, e->k.as<double>(), x);
+    if (rc) return rc;
+    OQ_HIP(hipMemcpyAsync(du, x, nb, hipMemcpyDeviceToHost, e->stream));
     OQ_HIP(hipStreamSynchronize(e->stream));
-    from_entry_major(e, o, du);
     return OQ_OK;
 }
 
@@ -1937,10 +1932,11 @@ static int grp_begin(oq_group *e, const double *u0, const double *tv, const doub
         OQ_HIP(hipStreamSynchronize(e->stream));  // the host vectors are read before they go
     }
     e->alg = alg;
-    std::vector<double> ui;
-    to_entry_major(e, u0, ui);
     const std::vector<int> zi(GM, 0);
-    OQ_HIP(hipMemcpyAsync(e->u.p, ui.data(), ui.size() * 8, hipMemcpyHostToDevice, e->stream));
+    // through y, which every step writes before it reads it
+    OQ_HIP(hipMemcpyAsync(e->y.p, u0, (size_t)e->ntot * 8, hipMemcpyHostToDevice, e->stream));
+    int rc = to_entry_major(e, e->y.as<double>(), e->u.as<double>());
+    if (rc) return rc;
     OQ_HIP(hipMemcpyAsync(e->ct.p, tv, GM * 8, hipMemcpyHostToDevice, e->stream));
     OQ_HIP(hipMemcpyAsync(e->cdt.p, dtv, GM * 8, hipMemcpyHostToDevice, e->stream));
     OQ_HIP(hipMemcpyAsync(e->cqold.p, qv, GM * 8, hipMemcpyHostToDevice, e->stream));
@@ -1959,7 +1955,7 @@ static int grp_begin(oq_group *e, const double *u0, const double *tv, const doub
     c.maxiters = o->maxiters > 0 ? o->maxiters : (long long)1e18;
     // FSAL seed: k1 = f(u) (on a resume with the same tile shapes, the same
     // bits as the k7 of the last accepted step)
-    int rc = set_live(e);
+    rc = set_live(e);
     if (!rc) rc = grp_rhs(e, e->u.as<double>(), e->k.as<double>());
     if (rc) return rc;
     drop_graphs(e);
@@ -2072,13 +2068,12 @@ int oq_group_state(oq_group *e, double *t, double *u, int64_t *naccept, int64_t 
     if (naccept) OQ_HIP(hipMemcpyAsync(naccept, e->cna.p, GM * 8, hipMemcpyDeviceToHost, e->stream));
     if (nreject) OQ_HIP(hipMemcpyAsync(nreject, e->cnr.p, GM * 8, hipMemcpyDeviceToHost, e->stream));
     if (retcode) OQ_HIP(hipMemcpyAsync(retcode, e->cret.p, GM * 4, hipMemcpyDeviceToHost, e->stream));
-    std::vector<double> o;
-    if (u) {
-        o.resize((size_t)e->ntot);
-        OQ_HIP(hipMemcpyAsync(o.data(), e->u.p, o.size() * 8, hipMemcpyDeviceToHost, e->stream));
+    if (u) {  // through y, scratch between steps
+        const int rc = from_entry_major(e, e->u.as<double>(), e->y.as<double>());
+        if (rc) return rc;
+        OQ_HIP(hipMemcpyAsync(u, e->y.p, (size_t)e->ntot * 8, hipMemcpyDeviceToHost, e->stream));
     }
     OQ_HIP(hipStreamSynchronize(e->stream));
-    if (u) from_entry_major(e, o, u);
     return OQ_OK;
 }
 

@@ -112,6 +112,11 @@ int launch_gf_hex8_seq(const DevHex8 &h, const DevFault &f, const double *qc, co
 int launch_expand_toeplitz(const double *st, int64_t nx, int64_t nxi,
                            double *k, int64_t ld, hipStream_t s);
 
+// dst (cols x rows) = transpose of src (rows x cols), both row-major: the
+// member-major host layout of a batch's states <-> its entry-major device
+// layout.
+int launch_transpose(const double *src, int64_t rows, int64_t cols, double *dst, hipStream_t s);
+
 // Real DFT of length 2nx-1 of the symmetric extension of every (j, l) column
 // of the Toeplitz kernel (GF.jl:60-67) and its inverse, on the device:
 // st (nx*nxi*nxi) <-> interleaved complex (2*nx*nxi*nxi).
