@@ -32,7 +32,7 @@ typedef unsigned int u4x __attribute__((ext_vector_type(4)));
 namespace oq {
 
 struct EnsDev {
-    int64_t nf, ne, N, ld, M, Mp, n;  // Mp: padded member count (multiple of 64; 256 for FP32 and split FP16)
+    int64_t nf, ne, N, ld, M, Mp, n;  // Mp: padded member count (of the GEMM's member tile)
     StateLayout lay;                   // offsets in entries (rows)
     const double *a, *b, *L, *sigma;   // nf x M
     const double *eta, *vpl, *f0, *v0; // M
@@ -486,74 +486,92 @@ __global__ void __launch_bounds__(512) k_ens_gemm_h3(EnsDev d, EnsH3 h)
     }
 }
 
-// ---------------- FP32 GEMM streaming K once (OQ_K_FP32) ----------------
-// The same block shape as k_ens_gemm_h3: a 64-row x 256-member tile per
-// workgroup of 8 wavefronts, so each row of K is read from HBM once per RHS
-// (the 128 x 64 tiles of k_ens_gemm read it once per 64 members).  Wave w
-// owns rows [32 (w % 2), +32) x members [64 (w / 2), +64): two 32 x 32 tiles
-// of v_mfma_f32_32x32x2f32.  Stages of 32 columns (K: 64 rows x 128 B, S:
-// 256 members x 128 B, member-major) go through double-buffered LDS with the
-// global loads two stages ahead in registers.  Within a stage the 16 MFMA
-// k-steps take columns 16 (lane / 32) + j, so a lane's A and B fragments
-// for all 16 steps are 64 contiguous bytes each.  The FP32 accumulators are
-// added into FP64 every 256 columns.
-static constexpr int kFBM = 64, kFBN = 256, kFKS = 32, kFRow = 144, kFChunk = 256;
-static constexpr int kFStage = (kFBM + kFBN) * kFRow;
-static constexpr size_t kFLds = 2 * (size_t)kFStage;
+// ---------------- FP32 GEMM (OQ_K_FP32) ----------------
+// A workgroup of NW wavefronts takes BM = 32 NW / WM rows x BN = 32 TB WM
+// members; wave w owns rows [32 (w % WR), +32) x members [32 TB (w / WR),
+// +32 TB): TB tiles of v_mfma_f32_32x32x2f32.  Stages of 32 columns (128 B of
+// each row of K and of each member of S, member-major) go through
+// double-buffered LDS with the global loads two stages ahead in registers.
+// Within a stage the 16 MFMA k-steps take columns 16 (lane / 32) + j, so a
+// lane's A and B fragments for all 16 steps are 64 contiguous bytes each.
+// The FP32 accumulators are folded every 256 columns (a chunk) into FP64.
+//
+// The member tile follows the ensemble (32, 64, 128 or 256 members: K is read
+// once per RHS up to 256, and no more than 31 columns of a tile are padding up
+// to 64), and where the row blocks do not fill the device the chunks are
+// shared out over gridDim.z: each block then stores its chunks' FP32 sums and
+// k_ens_finish adds them up in FP64 in the order of the undivided loop, so
+// every shape gives the same bits.  Measured at N = 2927: 24 members 208 ->
+// 15 us (46 workgroups of 256 members before, 276 of 32 now).
+static constexpr int kFKS = 32, kFRow = 144, kFChunk = 256;
+
+struct EnsF32Shape {
+    int bn = 0, bm = 0, threads = 0;  // members, rows, threads per workgroup
+    int nz = 1, cps = 0;              // workgroups along the chunks, chunks per workgroup
+    int nchunk = 0;
+    size_t lds = 0;
+};
 
 // S (entry-major [column][member], pitch Mp) -> member-major [member][column]
-// (pitch ld), 64 x 64 tiles through LDS.
+// (pitch ld), tiles of 64 columns x 32 members through LDS.
 __global__ void __launch_bounds__(256) k_ens_s_member_major(EnsDev d, const float *__restrict__ S,
                                                             float *__restrict__ Sm)
 {
     if (!*d.live) return;
-    __shared__ float tile[64][65];
-    const int64_t c0 = (int64_t)blockIdx.x * 64, m0 = (int64_t)blockIdx.y * 64;
-    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-    for (int r = ty; r < 64; r += 4) tile[r][tx] = S[(c0 + r) * d.Mp + m0 + tx];  // r: column
+    __shared__ float tile[64][33];
+    const int64_t c0 = (int64_t)blockIdx.x * 64, m0 = (int64_t)blockIdx.y * 32;
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    for (int r = ty; r < 64; r += 8) tile[r][tx] = S[(c0 + r) * d.Mp + m0 + tx];  // r: column
     __syncthreads();
-    for (int r = ty; r < 64; r += 4) Sm[(m0 + r) * d.ld + c0 + tx] = tile[tx][r];  // r: member
+    const int cx = threadIdx.x & 63, my = threadIdx.x >> 6;
+    for (int r = my; r < 32; r += 4) Sm[(m0 + r) * d.ld + c0 + cx] = tile[cx][r];  // r: member
 }
 
-__global__ void __launch_bounds__(512) k_ens_gemm_f32(EnsDev d, const float *__restrict__ K,
-                                                      const float *__restrict__ Sm,
-                                                      double *__restrict__ Y)
+template <int WM, int TB, int NW, bool SPLIT>
+__global__ void __launch_bounds__(64 * NW) k_ens_gemm_f32(EnsDev d, EnsF32Shape sh, const float *__restrict__ K,
+                                                          const float *__restrict__ Sm, double *__restrict__ Y,
+                                                          float *__restrict__ part)
 {
     if (!*d.live) return;
+    constexpr int WR = NW / WM, BM = 32 * WR, BN = 32 * TB * WM, T = 64 * NW;
+    constexpr int PK = BM * 8 / T, PS = BN * 8 / T, STAGE = (BM + BN) * kFRow;
     extern __shared__ __attribute__((aligned(16))) unsigned char flds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wr = wave & 1, wm = wave >> 1;
-    const int64_t rb = (int64_t)blockIdx.x * kFBM, m0 = (int64_t)blockIdx.y * kFBN;
+    const int wr = wave % WR, wm = wave / WR;
+    const int64_t rb = (int64_t)blockIdx.x * BM, m0 = (int64_t)blockIdx.y * BN;
     const int64_t rowb = 4 * d.ld;  // bytes per row of K and of Sm
-    const unsigned char *kg, *sg[4];
-    int kl, sl[4];
-    {
-        const int r = tid >> 3, pc = tid & 7;
+    const unsigned char *kg[PK], *sg[PS];
+    int kl[PK], sl[PS];
+#pragma unroll
+    for (int i = 0; i < PK; ++i) {
+        const int p = tid + T * i, r = p >> 3, pc = p & 7;
         const int64_t row = rb + r < d.N ? rb + r : d.N - 1;
-        kg = reinterpret_cast<const unsigned char *>(K) + row * rowb + 16 * pc;
-        kl = r * kFRow + 16 * pc;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int p = tid + 512 * i, mm = p >> 3, qc = p & 7;
-            sg[i] = reinterpret_cast<const unsigned char *>(Sm) + (m0 + mm) * rowb + 16 * qc;
-            sl[i] = (kFBM + mm) * kFRow + 16 * qc;
-        }
+        kg[i] = reinterpret_cast<const unsigned char *>(K) + row * rowb + 16 * pc;
+        kl[i] = r * kFRow + 16 * pc;
     }
-    u4x pa[5], pb[5];
-    auto gload = [&](u4x *pr, int64_t k0) {  // k0: first column of the stage
-        pr[0] = __builtin_nontemporal_load(reinterpret_cast<const u4x *>(kg + 4 * k0));
 #pragma unroll
-        for (int i = 0; i < 4; ++i) pr[1 + i] = *reinterpret_cast<const u4x *>(sg[i] + 4 * k0);
+    for (int i = 0; i < PS; ++i) {
+        const int p = tid + T * i, mm = p >> 3, qc = p & 7;
+        sg[i] = reinterpret_cast<const unsigned char *>(Sm) + (m0 + mm) * rowb + 16 * qc;
+        sl[i] = (BM + mm) * kFRow + 16 * qc;
+    }
+    u4x pa[PK + PS], pb[PK + PS];
+    auto gload = [&](u4x *pr, int64_t k0) {  // k0: first column of the stage
+#pragma unroll
+        for (int i = 0; i < PK; ++i) pr[i] = __builtin_nontemporal_load(reinterpret_cast<const u4x *>(kg[i] + 4 * k0));
+#pragma unroll
+        for (int i = 0; i < PS; ++i) pr[PK + i] = *reinterpret_cast<const u4x *>(sg[i] + 4 * k0);
     };
     auto lstore = [&](const u4x *pr, unsigned char *st) {
-        *reinterpret_cast<u4x *>(st + kl) = pr[0];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) *reinterpret_cast<u4x *>(st + sl[i]) = pr[1 + i];
+        for (int i = 0; i < PK; ++i) *reinterpret_cast<u4x *>(st + kl[i]) = pr[i];
+#pragma unroll
+        for (int i = 0; i < PS; ++i) *reinterpret_cast<u4x *>(st + sl[i]) = pr[PK + i];
     };
-    f16v acc[2];
-    double y[2][16];
+    f16v acc[TB];
+    double y[TB][16];
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
+    for (int b = 0; b < TB; ++b) {
         acc[b] = f16v{0};
 #pragma unroll
         for (int i = 0; i < 16; ++i) y[b][i] = 0.0;
@@ -561,72 +579,156 @@ __global__ void __launch_bounds__(512) k_ens_gemm_f32(EnsDev d, const float *__r
     const int lr = lane & 31, lg = lane >> 5;
     auto compute = [&](const unsigned char *cur) {
         const unsigned char *pA = cur + (wr * 32 + lr) * kFRow + 64 * lg;
-        f4x a[4], bv[2][4];
+        f4x a[4], bv[TB][4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) a[q] = *reinterpret_cast<const f4x *>(pA + 16 * q);
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            const unsigned char *pB = cur + (kFBM + wm * 64 + b * 32 + lr) * kFRow + 64 * lg;
+        for (int b = 0; b < TB; ++b) {
+            const unsigned char *pB = cur + (BM + wm * 32 * TB + b * 32 + lr) * kFRow + 64 * lg;
 #pragma unroll
             for (int q = 0; q < 4; ++q) bv[b][q] = *reinterpret_cast<const f4x *>(pB + 16 * q);
         }
 #pragma unroll
         for (int j = 0; j < 16; ++j)
 #pragma unroll
-            for (int b = 0; b < 2; ++b)
+            for (int b = 0; b < TB; ++b)
                 acc[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[j / 4][j % 4], bv[b][j / 4][j % 4], acc[b],
                                                               0, 0, 0);
     };
+    // element i of tile b: row 32 wr + (i / 4) 8 + (lane / 32) 4 + i % 4,
+    // member 32 (TB wm + b) + lane % 32
+    const int64_t row0 = rb + wr * 32 + lg * 4, mem = m0 + wm * 32 * TB + lr;
     auto fold = [&](int64_t st) {
         if (((st + 1) * kFKS) % kFChunk != 0) return;
+        const int64_t c = (st + 1) * kFKS / kFChunk - 1;
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
+        for (int b = 0; b < TB; ++b) {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) y[b][i] += (double)acc[b][i];
+            for (int i = 0; i < 16; ++i) {
+                if constexpr (SPLIT) {
+                    const int64_t row = row0 + (i / 4) * 8 + (i % 4);
+                    if (row < d.N) part[(c * d.N + row) * d.Mp + mem + b * 32] = acc[b][i];
+                } else {
+                    y[b][i] += (double)acc[b][i];
+                }
+            }
             acc[b] = f16v{0};
         }
     };
-    // pipeline as k_ens_gemm_h3 (nst even: ld is a multiple of 512)
-    const int64_t nst = d.ld / kFKS;
-    auto kof = [&](int64_t st) { return (st < nst ? st : nst - 1) * kFKS; };
-    gload(pa, 0);
-    gload(pb, kof(1));
+    // Pipeline: at the top of stage st, registers hold stage st + 1 and stage
+    // st + 2 is issued into the other set; stage st + 1 goes to LDS after
+    // stage st's MFMAs.  A chunk is 8 stages, so the loop runs in pairs with
+    // static register sets; past the end the last stage is loaded again and
+    // stored into the buffer nobody reads.
+    constexpr int64_t SPC = kFChunk / kFKS;
+    const int64_t c0 = (int64_t)blockIdx.z * sh.cps, c1 = c0 + sh.cps < sh.nchunk ? c0 + sh.cps : sh.nchunk;
+    const int64_t s0 = SPLIT ? c0 * SPC : 0, s1 = SPLIT ? c1 * SPC : sh.nchunk * SPC;
+    auto kof = [&](int64_t st) { return (st < s1 ? st : s1 - 1) * kFKS; };
+    gload(pa, kof(s0));
+    gload(pb, kof(s0 + 1));
     lstore(pa, flds);
     __syncthreads();
-    for (int64_t st = 0; st < nst; st += 2) {
+    for (int64_t st = s0; st < s1; st += 2) {
         gload(pa, kof(st + 2));
         compute(flds);
-        lstore(pb, flds + kFStage);
+        lstore(pb, flds + STAGE);
         fold(st);
         __syncthreads();
         gload(pb, kof(st + 3));
-        compute(flds + kFStage);
+        compute(flds + STAGE);
         lstore(pa, flds);
         fold(st + 1);
         __syncthreads();
     }
+    if constexpr (!SPLIT) {
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
+        for (int i = 0; i < 16; ++i) {
+            const int64_t row = row0 + (i / 4) * 8 + (i % 4);
+            if (row >= d.N) continue;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) y[b][i] += (double)acc[b][i];  // the last partial chunk
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const int64_t row = rb + wr * 32 + (i / 4) * 8 + lg * 4 + (i % 4);
-        if (row >= d.N) continue;
-#pragma unroll
-        for (int b = 0; b < 2; ++b) Y[row * d.Mp + m0 + wm * 64 + b * 32 + lr] = y[b][i];
+            for (int b = 0; b < TB; ++b) Y[row * d.Mp + mem + b * 32] = y[b][i];
+        }
     }
 }
 
-// epilogue of the split-FP16 GEMM: one thread per (row, member)
+template <int WM, int TB, int NW>
+static void ens_f32_shape(EnsF32Shape &s)
+{
+    s.bn = 32 * TB * WM;
+    s.bm = 32 * (NW / WM);
+    s.threads = 64 * NW;
+    s.lds = 2 * (size_t)((s.bm + s.bn) * kFRow);
+}
+
+// Member tile: the smallest of 32, 64, 128 and 256 that holds M (256 beyond).
+// Chunks are shared out until there are two workgroups per CU (one of the
+// wide ones).
+static EnsF32Shape ens_f32_pick(int64_t M)
+{
+    EnsF32Shape s;
+    if (M <= 32) ens_f32_shape<1, 1, 4>(s);
+    else if (M <= 64) ens_f32_shape<1, 2, 4>(s);
+    else if (M <= 128) ens_f32_shape<2, 2, 8>(s);
+    else ens_f32_shape<4, 2, 8>(s);
+    return s;
+}
+
+static void ens_f32_split(EnsF32Shape &s, int64_t N, int64_t ld, int64_t Mp)
+{
+    s.nchunk = (int)(ld / kFChunk);
+    const int64_t base = (N + s.bm - 1) / s.bm * (Mp / s.bn), want = s.threads == 256 ? 512 : 256;
+    int64_t nz = want / base;
+    if (nz > s.nchunk) nz = s.nchunk;
+    if (nz < 1) nz = 1;
+    s.cps = (int)((s.nchunk + nz - 1) / nz);
+    s.nz = (s.nchunk + s.cps - 1) / s.cps;
+}
+
+template <int WM, int TB, int NW>
+static int ens_f32_attr(const EnsF32Shape &s)
+{
+    OQ_HIP(hipFuncSetAttribute((const void *)k_ens_gemm_f32<WM, TB, NW, false>,
+                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)s.lds));
+    OQ_HIP(hipFuncSetAttribute((const void *)k_ens_gemm_f32<WM, TB, NW, true>,
+                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)s.lds));
+    return OQ_OK;
+}
+
+template <int WM, int TB, int NW>
+static void ens_f32_launch(const EnsDev &d, const EnsF32Shape &s, const float *K, const float *Sm, double *Y, float *part,
+                           hipStream_t st)
+{
+    const dim3 grid((unsigned)((d.N + s.bm - 1) / s.bm), (unsigned)(d.Mp / s.bn), (unsigned)s.nz);
+    if (s.nz > 1)
+        hipLaunchKernelGGL((k_ens_gemm_f32<WM, TB, NW, true>), grid, dim3(64 * NW), s.lds, st, d, s, K, Sm, Y, part);
+    else
+        hipLaunchKernelGGL((k_ens_gemm_f32<WM, TB, NW, false>), grid, dim3(64 * NW), s.lds, st, d, s, K, Sm, Y, part);
+}
+
+#define OQ_ENS_F32(s, f, ...)                              \
+    ((s).bn == 32 ? f<1, 1, 4>(__VA_ARGS__) : (s).bn == 64 ? f<1, 2, 4>(__VA_ARGS__) \
+     : (s).bn == 128 ? f<2, 2, 8>(__VA_ARGS__) : f<4, 2, 8>(__VA_ARGS__))
+
+// epilogue of the GEMMs: one thread per (row, member); nchunk > 0: the row
+// sum is added up here from the chunks' FP32 sums, in order
 __global__ void __launch_bounds__(256) k_ens_finish(EnsDev d, const double *__restrict__ Y,
+                                                    const float *__restrict__ part, int nchunk,
                                                     const double *__restrict__ u, double *__restrict__ du)
 {
     if (!*d.live) return;
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= d.N * d.M) return;
     const int64_t row = t / d.M, m = t % d.M;
-    ens_epilogue(d, row, m, Y[row * d.Mp + m], u, du);
+    double y = 0.0;
+    if (nchunk > 0) {
+        const float *p = part + row * d.Mp + m;
+        const int64_t cs = d.N * d.Mp;
+#pragma unroll 8
+        for (int c = 0; c < nchunk; ++c) y += (double)p[c * cs];
+    } else {
+        y = Y[row * d.Mp + m];
+    }
+    ens_epilogue(d, row, m, y, u, du);
 }
 
 // ---------------- batched Tsit5 ----------------
@@ -936,7 +1038,8 @@ struct oq_ensemble {
     int kdtype = OQ_K_FP32;
     int64_t M = 0, Mp = 0, n = 0;
     oq::DevBuf hK, hrsc, hS, hssc, hY;  // OQ_K_FP16X2: split operator, split S, scales, Y
-    oq::DevBuf Sm, fY;                  // OQ_K_FP32: member-major S, Y
+    oq::DevBuf Sm, fY, fpart;           // OQ_K_FP32: member-major S, Y or the chunks' sums
+    oq::EnsF32Shape f32{};
     oq::EnsH3 h3{};
     oq::DevBuf a, b, L, sigma, eta, vpl, f0, v0, S;
     oq::DevBuf u, y, k, part;
@@ -985,17 +1088,18 @@ static int ens_rhs(oq_ensemble *e, const double *u, double *du)
         hipLaunchKernelGGL(k_ens_gemm_h3, dim3(nbk(h->N, kHBM), (unsigned)(e->Mp / kHBN)), dim3(512), kHLds,
                            h->stream, e->dev, e->h3);
         hipLaunchKernelGGL(k_ens_finish, dim3(nbk(h->N * e->M, 256)), dim3(256), 0, h->stream, e->dev,
-                           e->h3.Y, u, du);
+                           e->h3.Y, nullptr, 0, u, du);
         OQ_HIP(hipGetLastError());
         return OQ_OK;
     }
     if (h->kdtype == OQ_K_FP32) {
-        hipLaunchKernelGGL(k_ens_s_member_major, dim3((unsigned)(h->ld / 64), (unsigned)(e->Mp / 64)),
+        const EnsF32Shape &f = e->f32;
+        hipLaunchKernelGGL(k_ens_s_member_major, dim3((unsigned)(h->ld / 64), (unsigned)(e->Mp / 32)),
                            dim3(256), 0, h->stream, e->dev, e->S.as<float>(), e->Sm.as<float>());
-        hipLaunchKernelGGL(k_ens_gemm_f32, dim3(nbk(h->N, kFBM), (unsigned)(e->Mp / kFBN)), dim3(512), kFLds,
-                           h->stream, e->dev, h->K.as<float>(), e->Sm.as<float>(), e->fY.as<double>());
+        OQ_ENS_F32(f, ens_f32_launch, e->dev, f, h->K.as<float>(), e->Sm.as<float>(), e->fY.as<double>(),
+                   e->fpart.as<float>(), h->stream);
         hipLaunchKernelGGL(k_ens_finish, dim3(nbk(h->N * e->M, 256)), dim3(256), 0, h->stream, e->dev,
-                           e->fY.as<double>(), u, du);
+                           e->fY.as<double>(), e->fpart.as<float>(), f.nz > 1 ? f.nchunk : 0, u, du);
         OQ_HIP(hipGetLastError());
         return OQ_OK;
     }
@@ -1153,7 +1257,8 @@ int oq_ensemble_create(int device, const oq_fault_mesh *mf, const oq_hex8_mesh *
     oq_rhs *h = e->h;
     const int64_t M = nmembers, nf = h->nf;
     e->M = M;
-    const int64_t mb = kdtype == OQ_K_FP16X2 ? kHBN : (kdtype == OQ_K_FP32 ? kFBN : EBN);
+    e->f32 = ens_f32_pick(M);
+    const int64_t mb = kdtype == OQ_K_FP16X2 ? kHBN : (kdtype == OQ_K_FP32 ? e->f32.bn : EBN);
     e->Mp = (M + mb - 1) / mb * mb;
     e->n = h->lay.n;
     std::vector<const double *> pa(M), pb(M), pL(M), ps(M);
@@ -1216,10 +1321,10 @@ int oq_ensemble_create(int device, const oq_fault_mesh *mf, const oq_hex8_mesh *
         const size_t sb = (size_t)(e->Mp * h->ld) * 4;
         rc = e->Sm.alloc(sb);
         if (!rc && hipMemsetAsync(e->Sm.p, 0, sb, h->stream) != hipSuccess) rc = OQ_ERR_HIP;
-        if (!rc) rc = e->fY.alloc((size_t)(h->N * e->Mp) * 8);
-        if (!rc && hipFuncSetAttribute((const void *)k_ens_gemm_f32,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)kFLds) != hipSuccess)
-            rc = OQ_ERR_HIP;
+        ens_f32_split(e->f32, h->N, h->ld, e->Mp);
+        if (!rc && e->f32.nz > 1) rc = e->fpart.alloc((size_t)(e->f32.nchunk * h->N * e->Mp) * 4);
+        if (!rc && e->f32.nz == 1) rc = e->fY.alloc((size_t)(h->N * e->Mp) * 8);
+        if (!rc) rc = OQ_ENS_F32(e->f32, ens_f32_attr, e->f32);
         if (!rc && hipStreamSynchronize(h->stream) != hipSuccess) rc = OQ_ERR_HIP;
         if (rc) {
             set_error("FP32 ensemble buffers: allocation or kernel set-up failed");
