@@ -20,6 +20,7 @@
 #include <math.h>
 #include <string.h>
 
+#include <type_traits>
 #include <vector>
 
 #include "adams.h"
@@ -757,42 +758,56 @@ struct EnsCtrl {  // arrays of M
     // and per-member rings rec_t/rec_v [M x rec_cap], slot (naccept-1) % cap
     long long nf, rec_cap;
     double *vpart, *rec_t, *rec_v;
-    int *live;  // the flag EnsDev::live reads (see k_ens_live)
+    int *live;  // the flag EnsDev::live reads (set by ens_begin_all)
 };
 
-// After k_ens_begin: live = 1 while any member is still running.  One block.
-__global__ void __launch_bounds__(1024) k_ens_live(EnsCtrl c)
+// Start of a step for member m: termination checks, dt clamp to dtmax and t1.
+// Returns whether it is still running.
+__device__ __forceinline__ bool ens_begin_member(const EnsCtrl &c, int m)
 {
-    __shared__ int any;
-    if (threadIdx.x == 0) any = 0;
-    __syncthreads();
-    int mine = 0;
-    for (int m = threadIdx.x; m < c.M; m += blockDim.x) mine |= !c.done[m];
-    if (mine) any = 1;  // benign race: every writer writes 1
-    __syncthreads();
-    if (threadIdx.x == 0) *c.live = any;
-}
-
-__global__ void k_ens_begin(EnsCtrl c)
-{
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= c.M) return;
     c.accept[m] = 0;
     c.dtcur[m] = 0.0;
-    if (c.done[m]) return;
-    if (!(c.t[m] < c.t1)) { c.done[m] = 1; c.retcode[m] = OQ_RET_SUCCESS; return; }
-    if (c.iter[m] >= c.maxiters) { c.done[m] = 1; c.retcode[m] = OQ_RET_MAXITERS; return; }
+    if (c.done[m]) return false;
+    if (!(c.t[m] < c.t1)) { c.done[m] = 1; c.retcode[m] = OQ_RET_SUCCESS; return false; }
+    if (c.iter[m] >= c.maxiters) { c.done[m] = 1; c.retcode[m] = OQ_RET_MAXITERS; return false; }
     double dt = c.dt[m];
     if (dt > c.dtmax) dt = c.dtmax;
     if (c.t[m] + dt > c.t1) dt = c.t1 - c.t[m];
     if (!(dt >= c.dtmin) || !isfinite(dt)) {
         c.done[m] = 1;
         c.retcode[m] = isfinite(dt) ? OQ_RET_DTMIN : OQ_RET_NONFINITE;
-        return;
+        return false;
     }
     c.dtcur[m] = dt;
     c.iter[m] += 1;
+    return true;
 }
+
+struct EnsNoCoeffs {
+    __device__ void operator()(int, double) const {}
+};
+
+// One block begins every member's step, sets the live flag (1 while any
+// member is running) and, for VCABM5, forms the members' coefficients: one
+// launch where three took 4.5 us each.
+template <class Coeffs>
+__device__ __forceinline__ void ens_begin_all(const EnsCtrl &c, Coeffs coeffs)
+{
+    __shared__ int any;
+    if (threadIdx.x == 0) any = 0;
+    __syncthreads();
+    int mine = 0;
+    for (int m = threadIdx.x; m < c.M; m += blockDim.x)
+        if (ens_begin_member(c, m)) {
+            mine = 1;
+            if (c.dtcur[m] > 0.0) coeffs(m, c.dtcur[m]);
+        }
+    if (mine) any = 1;  // benign race: every writer writes 1
+    __syncthreads();
+    if (threadIdx.x == 0) *c.live = any;
+}
+
+__global__ void __launch_bounds__(1024) k_ens_begin(EnsCtrl c) { ens_begin_all(c, EnsNoCoeffs()); }
 
 __global__ void __launch_bounds__(256) k_ens_stage(EnsCtrl c, int s, int64_t nM, int64_t M,
                                                    const double *__restrict__ u,
@@ -808,42 +823,122 @@ __global__ void __launch_bounds__(256) k_ens_stage(EnsCtrl c, int s, int64_t nM,
     y[i] = u[i] + dt * acc;
 }
 
-// per-(row chunk, member) partial sums of the squared scaled error
+// Per-(row chunk, member) partial sums of the squared scaled error.  A block
+// takes chunk blockIdx.y and TM members: 256 / TM rows of the chunk side by
+// side, U of them per thread with their loads in flight together, and the
+// squares added up in row order by the first TM threads (through LDS when
+// rows run side by side), so the sums do not depend on TM.  With one row at a
+// time 24 members of an N = 2927 model waited 28 us per step on memory
+// latency.  row(r, w, v): the scaled error of row r and its |v| (0 off the
+// fault).
 static constexpr int kEnsChunks = 512;
-__global__ void __launch_bounds__(256) k_ens_err(EnsCtrl c, int64_t n, int64_t M,
-                                                 const double *__restrict__ u,
-                                                 const double *__restrict__ y,
-                                                 const double *__restrict__ k,
+
+template <int TM, class Row>
+__device__ __forceinline__ void ens_chunk_norm(const EnsCtrl &c, int64_t n, int64_t M, double *__restrict__ part, Row row)
+{
+    constexpr int RP = 256 / TM, U = 4;
+    __shared__ double ws[RP > 1 ? U * 256 : 1], vs[RP > 1 ? 256 : 1];
+    const int mi = threadIdx.x % TM, rp = threadIdx.x / TM;
+    const int64_t m = (int64_t)blockIdx.x * TM + mi;
+    const int chunk = blockIdx.y;
+    const bool on = m < M;
+    const int64_t r0 = n * chunk / kEnsChunks, r1 = n * (chunk + 1) / kEnsChunks;
+    double acc = 0.0, vm = 0.0;
+    for (int64_t rb = r0; rb < r1; rb += RP * U) {
+        double w[U];
+#pragma unroll
+        for (int k = 0; k < U; ++k) {
+            const int64_t r = rb + k * RP + rp;
+            w[k] = 0.0;
+            if (on && r < r1) {
+                double v;
+                row(r, m, w[k], v);
+                vm = fmax(vm, v);
+            }
+        }
+        if constexpr (RP == 1) {
+#pragma unroll
+            for (int k = 0; k < U; ++k) acc += w[k] * w[k];
+        } else {
+#pragma unroll
+            for (int k = 0; k < U; ++k) ws[(k * RP + rp) * TM + mi] = w[k];
+            __syncthreads();
+            if (rp == 0)
+#pragma unroll 8
+                for (int q = 0; q < RP * U; ++q) {
+                    const double x = ws[q * TM + mi];
+                    acc += x * x;
+                }
+            __syncthreads();
+        }
+    }
+    if constexpr (RP > 1) {
+        vs[threadIdx.x] = vm;
+        __syncthreads();
+        if (rp == 0)
+            for (int q = 1; q < RP; ++q) vm = fmax(vm, vs[q * TM + mi]);
+    }
+    if (on && rp == 0) {
+        part[chunk * M + m] = acc;
+        if (c.rec_cap > 0) c.vpart[chunk * M + m] = vm;
+    }
+}
+
+template <int TM>
+__global__ void __launch_bounds__(256) k_ens_err(EnsCtrl c, int64_t n, int64_t M, const double *__restrict__ u,
+                                                 const double *__restrict__ y, const double *__restrict__ k,
                                                  double *__restrict__ part)
 {
     if (!*c.live) return;
-    const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int chunk = blockIdx.y;
-    if (m >= M) return;
     const int64_t nM = n * M;
-    const int64_t r0 = n * chunk / kEnsChunks, r1 = n * (chunk + 1) / kEnsChunks;
-    const double dt = c.dtcur[m];
-    double acc = 0.0, vm = 0.0;
-    for (int64_t r = r0; r < r1; ++r) {
+    ens_chunk_norm<TM>(c, n, M, part, [&](int64_t r, int64_t m, double &w, double &v) {
         const int64_t i = r * M + m;
+        const double dt = c.dtcur[m];
         double e = 0.0;
 #pragma unroll
         for (int j = 0; j < 7; ++j) e += kEBt[j] * k[j * nM + i];
         const double ay = fabs(y[i]);
-        const double w = dt * e / (c.abstol + fmax(fabs(u[i]), ay) * c.reltol);
-        acc += w * w;
-        if (r < c.nf) vm = fmax(vm, ay);  // rows [0, nf) of the state are v
-    }
-    part[chunk * M + m] = acc;
-    if (c.rec_cap > 0) c.vpart[chunk * M + m] = vm;
+        w = dt * e / (c.abstol + fmax(fabs(u[i]), ay) * c.reltol);
+        v = r < c.nf ? ay : 0.0;  // rows [0, nf) of the state are v
+    });
 }
 
-__global__ void k_ens_controller(EnsCtrl c, int64_t n, const double *__restrict__ part)
+// A member's sum of its 512 partial sums (in order) and, with the recorder
+// on, the largest of its |v| partials: a block takes 8 members, all threads
+// load, thread m < 8 adds from LDS.  (One thread per member waited 17 us on
+// its own loads.)
+static constexpr int kEnsCm = 8;
+__device__ __forceinline__ bool ens_sum_parts(const EnsCtrl &c, const double *__restrict__ part, double &acc, double &vm)
 {
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= c.M || c.done[m]) return;
-    double acc = 0.0;
-    for (int ch = 0; ch < kEnsChunks; ++ch) acc += part[ch * c.M + m];
+    __shared__ double ps[kEnsChunks * kEnsCm], vx[256];
+    const int mi = threadIdx.x % kEnsCm, q0 = threadIdx.x / kEnsCm, m = blockIdx.x * kEnsCm + mi;
+    constexpr int NQ = 256 / kEnsCm;
+    double v = 0.0;
+    if (m < c.M) {
+#pragma unroll
+        for (int q = 0; q < kEnsChunks / NQ; ++q)
+            ps[(q * NQ + q0) * kEnsCm + mi] = part[(int64_t)(q * NQ + q0) * c.M + m];
+        if (c.rec_cap > 0)
+            for (int ch = q0; ch < kEnsChunks; ch += NQ) v = fmax(v, c.vpart[(int64_t)ch * c.M + m]);
+    }
+    vx[threadIdx.x] = v;
+    __syncthreads();
+    if (q0 != 0 || m >= c.M) return false;
+    acc = 0.0;
+#pragma unroll 16
+    for (int ch = 0; ch < kEnsChunks; ++ch) acc += ps[ch * kEnsCm + mi];
+    vm = 0.0;
+    for (int q = 0; q < NQ; ++q) vm = fmax(vm, vx[q * kEnsCm + mi]);
+    return true;
+}
+
+__global__ void __launch_bounds__(256) k_ens_controller(EnsCtrl c, int64_t n, const double *__restrict__ part)
+{
+    if (!*c.live) return;
+    double acc, vm;
+    if (!ens_sum_parts(c, part, acc, vm)) return;
+    const int m = blockIdx.x * kEnsCm + threadIdx.x;
+    if (c.done[m]) return;
     const double beta1 = 7.0 / 50.0, beta2 = 2.0 / 25.0, qmin = 0.2, qmax = 10.0, gamma = 0.9,
                  qoldinit = 1e-4;
     const double eest = sqrt(acc / (double)n);
@@ -864,8 +959,6 @@ __global__ void k_ens_controller(EnsCtrl c, int64_t n, const double *__restrict_
         c.naccept[m] += 1;
         c.accept[m] = 1;
         if (c.rec_cap > 0) {
-            double vm = 0.0;
-            for (int ch = 0; ch < kEnsChunks; ++ch) vm = fmax(vm, c.vpart[ch * c.M + m]);
             const long long slot = (long long)m * c.rec_cap + (c.naccept[m] - 1) % c.rec_cap;
             c.rec_t[slot] = c.t[m];
             c.rec_v[slot] = vm;
@@ -905,13 +998,13 @@ struct EnsAb {
     double *yn, *fn;           // nM each
 };
 
-__global__ void k_eab_coeffs(EnsCtrl c, EnsAb a)
+__global__ void __launch_bounds__(1024) k_eab_begin(EnsCtrl c, EnsAb a)
 {
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= c.M || c.done[m] || !(c.dtcur[m] > 0.0)) return;
-    const int k = a.k[m];
-    a.kcur[m] = k;
-    ab_coeffs(k, c.dtcur[m], a.hist + m * (kAbK + 1), a.g + m * (kAbK + 1), a.beta + m * (kAbK + 1));
+    ens_begin_all(c, [&](int m, double h) {
+        const int k = a.k[m];
+        a.kcur[m] = k;
+        ab_coeffs(k, h, a.hist + m * (kAbK + 1), a.g + m * (kAbK + 1), a.beta + m * (kAbK + 1));
+    });
 }
 
 // p = u + h sum_{j<k} g_j beta_j Phi_j (members not stepping: p = u)
@@ -938,6 +1031,7 @@ __global__ void __launch_bounds__(256) k_eab_predict(EnsCtrl c, EnsAb a, int64_t
 // corrector y_{n+1} = p + h g_k Phi^p_k, Phi^p_k = f(p) - sum_{j<k} beta_j
 // Phi_j, and per-(row chunk, member) sums of the squared scaled error
 // h (g_k - g_{k-1}) Phi^p_k (and the max |v| of y_{n+1} for the recorder)
+template <int TM>
 __global__ void __launch_bounds__(256) k_eab_correct(EnsCtrl c, EnsAb a, int64_t n, int64_t M,
                                                      const double *__restrict__ u,
                                                      const double *__restrict__ p,
@@ -946,39 +1040,39 @@ __global__ void __launch_bounds__(256) k_eab_correct(EnsCtrl c, EnsAb a, int64_t
                                                      double *__restrict__ part)
 {
     if (!*c.live) return;
-    const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int chunk = blockIdx.y;
-    if (m >= M) return;
     const int64_t nM = n * M;
-    const int64_t r0 = n * chunk / kEnsChunks, r1 = n * (chunk + 1) / kEnsChunks;
-    const double h = c.dtcur[m];
-    const int k = a.kcur[m];
-    const double *g = a.g + m * (kAbK + 1), *be = a.beta + m * (kAbK + 1);
+    const int64_t mm = (int64_t)blockIdx.x * TM + threadIdx.x % TM, ms = mm < M ? mm : M - 1;
+    const double h = c.dtcur[ms];
+    const int k = a.kcur[ms];
+    const double *g = a.g + ms * (kAbK + 1), *be = a.beta + ms * (kAbK + 1);
     const double gk = h > 0.0 ? g[k] : 0.0, dg = h > 0.0 ? g[k] - g[k - 1] : 0.0;
-    double acc = 0.0, vm = 0.0;
-    for (int64_t r = r0; r < r1; ++r) {
+    double bj[kAbK];
+#pragma unroll
+    for (int j = 0; j < kAbK; ++j) bj[j] = be[j];
+    ens_chunk_norm<TM>(c, n, M, part, [&](int64_t r, int64_t m, double &w, double &v) {
         const int64_t i = r * M + m;
         double ph = fp[i];
-        if (h > 0.0)
-            for (int j = 0; j < k; ++j) ph -= be[j] * phi[j * nM + i];
+        if (h > 0.0) {
+#pragma unroll
+            for (int j = 0; j < kAbK; ++j)
+                if (j < k) ph -= bj[j] * phi[j * nM + i];
+        }
         const double yn = p[i] + h * gk * ph;
         a.yn[i] = yn;
-        const double w = h * dg * ph / (c.abstol + fmax(fabs(u[i]), fabs(yn)) * c.reltol);
-        acc += w * w;
-        if (r < c.nf) vm = fmax(vm, fabs(yn));  // rows [0, nf) of the state are v
-    }
-    part[chunk * M + m] = acc;
-    if (c.rec_cap > 0) c.vpart[chunk * M + m] = vm;
+        w = h * dg * ph / (c.abstol + fmax(fabs(u[i]), fabs(yn)) * c.reltol);
+        v = r < c.nf ? fabs(yn) : 0.0;  // rows [0, nf) of the state are v
+    });
 }
 
 // per member: step factor 1/clamp(err^(1/(k+1))/0.9, 1/2, 5), acceptance,
 // step history and order
-__global__ void k_eab_controller(EnsCtrl c, EnsAb a, int64_t n, const double *__restrict__ part)
+__global__ void __launch_bounds__(256) k_eab_controller(EnsCtrl c, EnsAb a, int64_t n, const double *__restrict__ part)
 {
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= c.M || c.done[m] || !(c.dtcur[m] > 0.0)) return;
-    double acc = 0.0;
-    for (int ch = 0; ch < kEnsChunks; ++ch) acc += part[ch * c.M + m];
+    if (!*c.live) return;
+    double acc, vm;
+    if (!ens_sum_parts(c, part, acc, vm)) return;
+    const int m = blockIdx.x * kEnsCm + threadIdx.x;
+    if (c.done[m] || !(c.dtcur[m] > 0.0)) return;
     const double eest = sqrt(acc / (double)n);
     const int k = a.kcur[m];
     const double q = (eest == 0.0) ? 0.5 : fmax(0.5, fmin(5.0, pow(eest, 1.0 / (k + 1)) / 0.9));
@@ -993,8 +1087,6 @@ __global__ void k_eab_controller(EnsCtrl c, EnsAb a, int64_t n, const double *__
         c.naccept[m] += 1;
         c.accept[m] = 1;
         if (c.rec_cap > 0) {
-            double vm = 0.0;
-            for (int ch = 0; ch < kEnsChunks; ++ch) vm = fmax(vm, c.vpart[ch * c.M + m]);
             const long long slot = (long long)m * c.rec_cap + (c.naccept[m] - 1) % c.rec_cap;
             c.rec_t[slot] = c.t[m];
             c.rec_v[slot] = vm;
@@ -1110,6 +1202,17 @@ static int ens_rhs(oq_ensemble *e, const double *u, double *du)
     return OQ_OK;
 }
 
+// members side by side in the error kernels: as many as there are, up to 256
+template <class F>
+static void ens_tiled(int64_t M, F f)
+{
+    if (M <= 16) f(std::integral_constant<int, 16>());
+    else if (M <= 32) f(std::integral_constant<int, 32>());
+    else if (M <= 64) f(std::integral_constant<int, 64>());
+    else if (M <= 128) f(std::integral_constant<int, 128>());
+    else f(std::integral_constant<int, 256>());
+}
+
 static int ens_step_ab(oq_ensemble *e);
 
 static int ens_step(oq_ensemble *e)
@@ -1119,16 +1222,18 @@ static int ens_step(oq_ensemble *e)
     const int64_t nM = e->n * e->M;
     double *u = e->u.as<double>(), *y = e->y.as<double>(), *k = e->k.as<double>();
     int rc;
-    hipLaunchKernelGGL(k_ens_begin, dim3(nbk(e->M, 256)), dim3(256), 0, h->stream, e->ctrl);
-    hipLaunchKernelGGL(k_ens_live, dim3(1), dim3(1024), 0, h->stream, e->ctrl);
+    hipLaunchKernelGGL(k_ens_begin, dim3(1), dim3(1024), 0, h->stream, e->ctrl);
     for (int s = 1; s < 7; ++s) {
         hipLaunchKernelGGL(k_ens_stage, dim3(nbk(nM, 256)), dim3(256), 0, h->stream, e->ctrl, s, nM,
                            e->M, u, k, y);
         if ((rc = ens_rhs(e, y, k + s * nM))) return rc;
     }
-    hipLaunchKernelGGL(k_ens_err, dim3(nbk(e->M, 256), kEnsChunks), dim3(256), 0, h->stream, e->ctrl,
-                       e->n, e->M, u, y, k, e->part.as<double>());
-    hipLaunchKernelGGL(k_ens_controller, dim3(nbk(e->M, 256)), dim3(256), 0, h->stream, e->ctrl, e->n,
+    ens_tiled(e->M, [&](auto tm) {
+        constexpr int TM = decltype(tm)::value;
+        hipLaunchKernelGGL(k_ens_err<TM>, dim3(nbk(e->M, TM), kEnsChunks), dim3(256), 0, h->stream, e->ctrl, e->n, e->M,
+                           u, y, k, e->part.as<double>());
+    });
+    hipLaunchKernelGGL(k_ens_controller, dim3(nbk(e->M, kEnsCm)), dim3(256), 0, h->stream, e->ctrl, e->n,
                        e->part.as<double>());
     hipLaunchKernelGGL(k_ens_commit, dim3(nbk(nM, 256)), dim3(256), 0, h->stream, e->ctrl, nM, e->M,
                        u, y, k);
@@ -1143,16 +1248,18 @@ static int ens_step_ab(oq_ensemble *e)
     oq_rhs *h = e->h;
     const int64_t nM = e->n * e->M;
     double *u = e->u.as<double>(), *p = e->y.as<double>(), *phi = e->k.as<double>(), *fp = phi + 6 * nM;
-    const dim3 gm(nbk(e->M, 256)), gn(nbk(nM, 256)), blk(256);
+    const dim3 gn(nbk(nM, 256)), blk(256);
     int rc;
-    hipLaunchKernelGGL(k_ens_begin, gm, blk, 0, h->stream, e->ctrl);
-    hipLaunchKernelGGL(k_eab_coeffs, gm, blk, 0, h->stream, e->ctrl, e->eab);
-    hipLaunchKernelGGL(k_ens_live, dim3(1), dim3(1024), 0, h->stream, e->ctrl);
+    hipLaunchKernelGGL(k_eab_begin, dim3(1), dim3(1024), 0, h->stream, e->ctrl, e->eab);
     hipLaunchKernelGGL(k_eab_predict, gn, blk, 0, h->stream, e->ctrl, e->eab, nM, e->M, u, phi, p);
     if ((rc = ens_rhs(e, p, fp))) return rc;
-    hipLaunchKernelGGL(k_eab_correct, dim3(nbk(e->M, 256), kEnsChunks), blk, 0, h->stream, e->ctrl, e->eab,
-                       e->n, e->M, u, p, fp, phi, e->part.as<double>());
-    hipLaunchKernelGGL(k_eab_controller, gm, blk, 0, h->stream, e->ctrl, e->eab, e->n, e->part.as<double>());
+    ens_tiled(e->M, [&](auto tm) {
+        constexpr int TM = decltype(tm)::value;
+        hipLaunchKernelGGL(k_eab_correct<TM>, dim3(nbk(e->M, TM), kEnsChunks), blk, 0, h->stream, e->ctrl, e->eab, e->n,
+                           e->M, u, p, fp, phi, e->part.as<double>());
+    });
+    hipLaunchKernelGGL(k_eab_controller, dim3(nbk(e->M, kEnsCm)), blk, 0, h->stream, e->ctrl, e->eab, e->n,
+                       e->part.as<double>());
     if ((rc = ens_rhs(e, e->eab.yn, e->eab.fn))) return rc;
     hipLaunchKernelGGL(k_eab_commit, gn, blk, 0, h->stream, e->ctrl, e->eab, nM, e->M, u, phi);
     OQ_HIP(hipGetLastError());
