@@ -195,6 +195,14 @@ __global__ void __launch_bounds__(256) k_ens_gemm(EnsDev d, const void *__restri
     }
 }
 
+// Workgroup tile and chunk sharing of the two member-tiled GEMMs.
+struct EnsShape {
+    int bn = 0, bm = 0, threads = 0;  // members, rows, threads per workgroup
+    int nz = 1, cps = 0;              // workgroups along the chunks, chunks per workgroup
+    int nchunk = 0;
+    size_t lds = 0;
+};
+
 // ---------------- split-FP16 GEMM (OQ_K_FP16X2) ----------------
 // FP32-class products on the FP16 matrix cores.  Each row r of K is kept as
 // K[r, j] = (Kh + 2^-11 Kl) * rsc[r] with Kh = fp16(x), Kl = fp16(2^11 (x -
@@ -219,11 +227,8 @@ __global__ void __launch_bounds__(256) k_ens_gemm(EnsDev d, const void *__restri
 typedef _Float16 h8x __attribute__((ext_vector_type(8)));
 
 static constexpr int kHCh = 512;               // columns per chunk
-static constexpr int kHBM = 64, kHBN = 256;    // block tile: rows x members
 static constexpr int kHKS = 32;                // columns per LDS stage
 static constexpr int kHRow = 144;              // LDS bytes per row/member (128 + 16 pad)
-static constexpr int kHStage = (kHBM + kHBN) * kHRow;
-static constexpr size_t kHLds = 2 * (size_t)kHStage;  // double-buffered
 
 struct EnsH3 {
     int64_t nfp, ldc, nchunk;  // padded fault columns, columns, chunks
@@ -345,145 +350,180 @@ __global__ void __launch_bounds__(256) k_h3_prep_s(EnsDev d, EnsH3 h, const floa
     }
 }
 
-// Y = K S for a 64-row x 256-member block tile, 8 wavefronts.  Wave w owns
-// rows [32 (w % 2), +32) x members [64 (w / 2), +64): two 32 x 32 MFMA
-// tiles.  Stages of 32 columns of K (64 rows) and S (256 members) go through
-// double-buffered LDS; global loads run two stages ahead in registers.
-// (Measured alternatives: 4 waves with 2 x 2 tiles spilled into AGPR
-// copies; 128-member blocks two per CU streamed K twice and ran 20 %
+// Y = K S on a tile of BM = 32 NW / WM rows x BN = 32 TB WM members, NW
+// wavefronts.  Wave w owns rows [32 (w % WR), +32) x members [32 TB (w / WR),
+// +32 TB): TB 32 x 32 MFMA tiles.  Stages of 32 columns of K and S go through
+// three LDS buffers, with the global loads four stages ahead in registers.
+// While a wave runs the MFMAs of one half of a stage (16 columns), its reads
+// of the other half's, and then of the next stage's, fragments are in flight;
+// with both halves read before the first MFMA (two buffers) LDS and matrix
+// cores took turns: 425-470 us at N = 16384, 256 members, against 450-480.
+// (Measured alternatives before that: 4 waves with 2 x 2 tiles spilled into
+// AGPR copies; 128-member blocks two per CU streamed K twice and ran 20 %
 // slower; three stages loaded straight into LDS with global_load_lds and
 // XOR-swizzled rows ran 12 % slower.)
-__global__ void __launch_bounds__(512) k_ens_gemm_h3(EnsDev d, EnsH3 h)
+//
+// The member tile and the sharing of the chunks follow the FP32 GEMM's: a
+// block with its own chunks stores each chunk's FP64 sum acc + 2^-11 acx and
+// k_ens_finish scales and adds them in order, so every shape gives the same
+// bits.
+template <int WM, int TB, int NW, bool SPLIT>
+__global__ void __launch_bounds__(64 * NW) k_ens_gemm_h3(EnsDev d, EnsH3 h, EnsShape sh, double *__restrict__ part)
 {
     if (!*d.live) return;
+    constexpr int WR = NW / WM, BM = 32 * WR, BN = 32 * TB * WM, T = 64 * NW;
+    constexpr int PK = BM * 8 / T, PS = BN * 8 / T, STAGE = (BM + BN) * kHRow;
     extern __shared__ __attribute__((aligned(16))) unsigned char hlds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wr = wave & 1, wm = wave >> 1;
-    const int64_t rb = (int64_t)blockIdx.x * kHBM, m0 = (int64_t)blockIdx.y * kHBN;
+    const int wr = wave % WR, wm = wave / WR;
+    const int64_t rb = (int64_t)blockIdx.x * BM, m0 = (int64_t)blockIdx.y * BN;
     const int64_t rowb = 4 * h.ldc;  // bytes per split row
-    // global -> LDS pieces of 16 B: K 64 rows x 8 (one per thread), S 256
-    // members x 8 (four per thread)
-    const unsigned char *kg, *sg[4];
-    int kl, sl[4];
-    {
-        const int r = tid >> 3, pc = tid & 7;
+    const unsigned char *kg[PK], *sg[PS];
+    int kl[PK], sl[PS];
+#pragma unroll
+    for (int i = 0; i < PK; ++i) {
+        const int p = tid + T * i, r = p >> 3, pc = p & 7;
         const int64_t row = rb + r < d.N ? rb + r : d.N - 1;
-        kg = reinterpret_cast<const unsigned char *>(h.K) + row * rowb + 16 * pc;
-        kl = r * kHRow + 16 * pc;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int p = tid + 512 * i, mm = p >> 3, qc = p & 7;
-            sg[i] = reinterpret_cast<const unsigned char *>(h.S) + (m0 + mm) * rowb + 16 * qc;
-            sl[i] = (kHBM + mm) * kHRow + 16 * qc;
-        }
+        kg[i] = reinterpret_cast<const unsigned char *>(h.K) + row * rowb + 16 * pc;
+        kl[i] = r * kHRow + 16 * pc;
     }
-    u4x pa[5], pb[5];
-    auto gload = [&](u4x *pr, int64_t k0) {
-        pr[0] = __builtin_nontemporal_load(reinterpret_cast<const u4x *>(kg + 4 * k0));
 #pragma unroll
-        for (int i = 0; i < 4; ++i) pr[1 + i] = *reinterpret_cast<const u4x *>(sg[i] + 4 * k0);
+    for (int i = 0; i < PS; ++i) {
+        const int p = tid + T * i, mm = p >> 3, qc = p & 7;
+        sg[i] = reinterpret_cast<const unsigned char *>(h.S) + (m0 + mm) * rowb + 16 * qc;
+        sl[i] = (BM + mm) * kHRow + 16 * qc;
+    }
+    u4x pa[PK + PS], pb[PK + PS];
+    auto gload = [&](u4x *pr, int64_t k0) {
+#pragma unroll
+        for (int i = 0; i < PK; ++i) pr[i] = __builtin_nontemporal_load(reinterpret_cast<const u4x *>(kg[i] + 4 * k0));
+#pragma unroll
+        for (int i = 0; i < PS; ++i) pr[PK + i] = *reinterpret_cast<const u4x *>(sg[i] + 4 * k0);
     };
     auto lstore = [&](const u4x *pr, unsigned char *st) {
-        *reinterpret_cast<u4x *>(st + kl) = pr[0];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) *reinterpret_cast<u4x *>(st + sl[i]) = pr[1 + i];
+        for (int i = 0; i < PK; ++i) *reinterpret_cast<u4x *>(st + kl[i]) = pr[i];
+#pragma unroll
+        for (int i = 0; i < PS; ++i) *reinterpret_cast<u4x *>(st + sl[i]) = pr[PK + i];
     };
-    f16v acc[2], acx[2];
-    double y[2][16];
+    f16v acc[TB], acx[TB];
+    double y[TB][16];
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
+    for (int b = 0; b < TB; ++b) {
         acc[b] = f16v{0};
         acx[b] = f16v{0};
 #pragma unroll
         for (int i = 0; i < 16; ++i) y[b][i] = 0.0;
     }
     const int lr = lane & 31, lg = lane >> 5;
-    auto compute = [&](const unsigned char *cur) {
-        // both k-steps' fragments first: the second step's LDS latency hides
-        // behind the first step's MFMAs
-        h8x ah[2], al[2], bh[2][2], bl[2][2];
+    struct Frag {
+        h8x ah, al, bh[TB], bl[TB];
+    };
+    auto fread = [&](Frag &f, const unsigned char *cur, int ks) {
+        const int go = (2 * ks + lg) * 32;
+        const unsigned char *pA = cur + (wr * 32 + lr) * kHRow + go;
+        f.ah = *reinterpret_cast<const h8x *>(pA);
+        f.al = *reinterpret_cast<const h8x *>(pA + 16);
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            const int go = (2 * ks + lg) * 32;
-            const unsigned char *pA = cur + (wr * 32 + lr) * kHRow + go;
-            ah[ks] = *reinterpret_cast<const h8x *>(pA);
-            al[ks] = *reinterpret_cast<const h8x *>(pA + 16);
-#pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                const unsigned char *pB = cur + (kHBM + wm * 64 + b * 32 + lr) * kHRow + go;
-                bh[ks][b] = *reinterpret_cast<const h8x *>(pB);
-                bl[ks][b] = *reinterpret_cast<const h8x *>(pB + 16);
-            }
-        }
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-#pragma unroll
-            for (int b = 0; b < 2; ++b)
-                acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[ks], bh[ks][b], acc[b], 0, 0, 0);
-#pragma unroll
-            for (int b = 0; b < 2; ++b)
-                acx[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[ks], bl[ks][b], acx[b], 0, 0, 0);
-#pragma unroll
-            for (int b = 0; b < 2; ++b)
-                acx[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[ks], bh[ks][b], acx[b], 0, 0, 0);
+        for (int b = 0; b < TB; ++b) {
+            const unsigned char *pB = cur + (BM + wm * 32 * TB + b * 32 + lr) * kHRow + go;
+            f.bh[b] = *reinterpret_cast<const h8x *>(pB);
+            f.bl[b] = *reinterpret_cast<const h8x *>(pB + 16);
         }
     };
-    // chunk scales of this lane's two members, loaded one chunk ahead so the
-    // fold does not wait on the stage prefetches
-    const double *scp = h.ssc + m0 + wm * 64 + lr;
-    double inv[2] = {scp[0], scp[32]};
+    auto mma = [&](const Frag &f) {
+#pragma unroll
+        for (int b = 0; b < TB; ++b) acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.ah, f.bh[b], acc[b], 0, 0, 0);
+#pragma unroll
+        for (int b = 0; b < TB; ++b) acx[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.ah, f.bl[b], acx[b], 0, 0, 0);
+#pragma unroll
+        for (int b = 0; b < TB; ++b) acx[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.al, f.bh[b], acx[b], 0, 0, 0);
+    };
+    // element i of tile b: row 32 wr + (i / 4) 8 + (lane / 32) 4 + i % 4,
+    // member 32 (TB wm + b) + lane % 32
+    const int64_t row0 = rb + wr * 32 + lg * 4, mem = m0 + wm * 32 * TB + lr;
+    constexpr int64_t SPC = kHCh / kHKS;
+    const int64_t c0 = SPLIT ? (int64_t)blockIdx.z * sh.cps : 0,
+                  c1 = SPLIT && c0 + sh.cps < h.nchunk ? c0 + sh.cps : h.nchunk;
+    const int64_t s0 = c0 * SPC, s1 = c1 * SPC;
+    // chunk scales of this lane's members, loaded one chunk ahead so the fold
+    // does not wait on the stage prefetches
+    const double *scp = h.ssc + mem;
+    double inv[TB];
+#pragma unroll
+    for (int b = 0; b < TB; ++b) inv[b] = SPLIT ? 0.0 : scp[b * 32];
     auto fold = [&](int64_t st) {  // chunk end: scale by the member's chunk scale, add into FP64
-        if (((st + 1) * kHKS) % kHCh != 0) return;
-        const int64_t cn = (st + 1) * kHKS / kHCh;  // next chunk
-        const int64_t cl = cn < h.nchunk ? cn : h.nchunk - 1;
-        const double nx0 = scp[cl * d.Mp], nx1 = scp[cl * d.Mp + 32];
+        if ((st + 1) % SPC != 0) return;
+        const int64_t c = (st + 1) / SPC - 1;
+        double nx[TB];
+        if constexpr (!SPLIT) {
+            const int64_t cl = c + 1 < h.nchunk ? c + 1 : h.nchunk - 1;
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
+            for (int b = 0; b < TB; ++b) nx[b] = scp[cl * d.Mp + b * 32];
+        }
 #pragma unroll
-            for (int i = 0; i < 16; ++i)
-                y[b][i] += ((double)acc[b][i] + (double)acx[b][i] * (1.0 / 2048.0)) * inv[b];
+        for (int b = 0; b < TB; ++b) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                if constexpr (SPLIT) {
+                    const int64_t row = row0 + (i / 4) * 8 + (i % 4);
+                    if (row < d.N)
+                        part[(c * d.N + row) * d.Mp + mem + b * 32] =
+                            (double)acc[b][i] + (double)acx[b][i] * (1.0 / 2048.0);
+                } else {
+                    y[b][i] += ((double)acc[b][i] + (double)acx[b][i] * (1.0 / 2048.0)) * inv[b];
+                }
+            }
             acc[b] = f16v{0};
             acx[b] = f16v{0};
+            if constexpr (!SPLIT) inv[b] = nx[b];
         }
-        inv[0] = nx0;
-        inv[1] = nx1;
     };
-    // Pipeline: at the top of stage st, registers hold stage st + 1 (set
-    // (st + 1) % 2) and stage st + 2 is issued into the other set; stage
-    // st + 1 goes to LDS after stage st's MFMAs.  nst is even (ldc is a
-    // multiple of kHCh), so the loop runs in pairs with static register sets.
-    // The body has no data-dependent branches (past the end, the last stage
-    // is loaded again and stored into the buffer nobody reads), so the
-    // compiler's wait counts keep both prefetched stages in flight.
-    const int64_t nst = h.ldc / kHKS;
-    auto kof = [&](int64_t st) { return (st < nst ? st : nst - 1) * kHKS; };
-    gload(pa, 0);
-    gload(pb, kof(1));
-    lstore(pa, hlds);
+    // At the top of stage st: its data in buffer b0, stage st + 1's in b1,
+    // both visible; f0 holds the fragments of its first half; one register
+    // set holds stage st + 2, the other st + 3.  Past the end the last stage
+    // is loaded again and its fragments are not used.
+    auto kof = [&](int64_t st) { return (st < s1 ? st : s1 - 1) * kHKS; };
+    unsigned char *b0 = hlds, *b1 = hlds + STAGE, *b2 = hlds + 2 * STAGE;
+    Frag f0, f1;
+    gload(pa, kof(s0));
+    gload(pb, kof(s0 + 1));
+    lstore(pa, b0);
+    gload(pa, kof(s0 + 2));
+    lstore(pb, b1);
+    gload(pb, kof(s0 + 3));
     __syncthreads();
-    for (int64_t st = 0; st < nst; st += 2) {
-        // even stage st: pb holds st + 1, pa is free
-        gload(pa, kof(st + 2));
-        compute(hlds);
-        lstore(pb, hlds + kHStage);
+    fread(f0, b0, 0);
+    auto stage = [&](int64_t st, u4x *pr) {
+        fread(f1, b0, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        mma(f0);
+        __builtin_amdgcn_sched_barrier(0);
+        lstore(pr, b2);
+        gload(pr, kof(st + 4));
+        fread(f0, b1, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        mma(f1);
         fold(st);
         __syncthreads();
-        // odd stage st + 1: pa holds st + 2, pb is free
-        gload(pb, kof(st + 3));
-        compute(hlds + kHStage);
-        lstore(pa, hlds);
-        fold(st + 1);
-        __syncthreads();
+        unsigned char *t = b0;
+        b0 = b1;
+        b1 = b2;
+        b2 = t;
+    };
+    for (int64_t st = s0; st < s1; st += 2) {  // a chunk is 16 stages
+        stage(st, pa);
+        stage(st + 1, pb);
     }
-    // element i of tile b: row 32 wr + (i / 4) 8 + (lane / 32) 4 + i % 4,
-    // member 64 wm + 32 b + lane % 32
+    if constexpr (!SPLIT) {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const int64_t row = rb + wr * 32 + (i / 4) * 8 + lg * 4 + (i % 4);
-        if (row >= d.N) continue;
-        const double rs = h.rsc[row];
+        for (int i = 0; i < 16; ++i) {
+            const int64_t row = row0 + (i / 4) * 8 + (i % 4);
+            if (row >= d.N) continue;
+            const double rs = h.rsc[row];
 #pragma unroll
-        for (int b = 0; b < 2; ++b) h.Y[row * d.Mp + m0 + wm * 64 + b * 32 + lr] = y[b][i] * rs;
+            for (int b = 0; b < TB; ++b) h.Y[row * d.Mp + mem + b * 32] = y[b][i] * rs;
+        }
     }
 }
 
@@ -506,13 +546,6 @@ __global__ void __launch_bounds__(512) k_ens_gemm_h3(EnsDev d, EnsH3 h)
 // 15 us (46 workgroups of 256 members before, 276 of 32 now).
 static constexpr int kFKS = 32, kFRow = 144, kFChunk = 256;
 
-struct EnsF32Shape {
-    int bn = 0, bm = 0, threads = 0;  // members, rows, threads per workgroup
-    int nz = 1, cps = 0;              // workgroups along the chunks, chunks per workgroup
-    int nchunk = 0;
-    size_t lds = 0;
-};
-
 // S (entry-major [column][member], pitch Mp) -> member-major [member][column]
 // (pitch ld), tiles of 64 columns x 32 members through LDS.
 __global__ void __launch_bounds__(256) k_ens_s_member_major(EnsDev d, const float *__restrict__ S,
@@ -529,7 +562,7 @@ __global__ void __launch_bounds__(256) k_ens_s_member_major(EnsDev d, const floa
 }
 
 template <int WM, int TB, int NW, bool SPLIT>
-__global__ void __launch_bounds__(64 * NW) k_ens_gemm_f32(EnsDev d, EnsF32Shape sh, const float *__restrict__ K,
+__global__ void __launch_bounds__(64 * NW) k_ens_gemm_f32(EnsDev d, EnsShape sh, const float *__restrict__ K,
                                                           const float *__restrict__ Sm, double *__restrict__ Y,
                                                           float *__restrict__ part)
 {
@@ -653,30 +686,32 @@ __global__ void __launch_bounds__(64 * NW) k_ens_gemm_f32(EnsDev d, EnsF32Shape 
 }
 
 template <int WM, int TB, int NW>
-static void ens_f32_shape(EnsF32Shape &s)
+static void ens_tile(EnsShape &s, int nbuf)
 {
+    static_assert(kHRow == kFRow, "one LDS row pitch");
     s.bn = 32 * TB * WM;
     s.bm = 32 * (NW / WM);
     s.threads = 64 * NW;
-    s.lds = 2 * (size_t)((s.bm + s.bn) * kFRow);
+    s.lds = (size_t)(nbuf * (s.bm + s.bn) * kFRow);
 }
 
 // Member tile: the smallest of 32, 64, 128 and 256 that holds M (256 beyond).
-// Chunks are shared out until there are two workgroups per CU (one of the
-// wide ones).
-static EnsF32Shape ens_f32_pick(int64_t M)
+// nbuf: LDS buffers of a stage.
+static EnsShape ens_pick(int64_t M, int nbuf)
 {
-    EnsF32Shape s;
-    if (M <= 32) ens_f32_shape<1, 1, 4>(s);
-    else if (M <= 64) ens_f32_shape<1, 2, 4>(s);
-    else if (M <= 128) ens_f32_shape<2, 2, 8>(s);
-    else ens_f32_shape<4, 2, 8>(s);
+    EnsShape s;
+    if (M <= 32) ens_tile<1, 1, 4>(s, nbuf);
+    else if (M <= 64) ens_tile<1, 2, 4>(s, nbuf);
+    else if (M <= 128) ens_tile<2, 2, 8>(s, nbuf);
+    else ens_tile<4, 2, 8>(s, nbuf);
     return s;
 }
 
-static void ens_f32_split(EnsF32Shape &s, int64_t N, int64_t ld, int64_t Mp)
+// Chunks are shared out until there are two workgroups per CU (one of the
+// wide ones).
+static void ens_split(EnsShape &s, int64_t N, int64_t nchunk, int64_t Mp)
 {
-    s.nchunk = (int)(ld / kFChunk);
+    s.nchunk = (int)nchunk;
     const int64_t base = (N + s.bm - 1) / s.bm * (Mp / s.bn), want = s.threads == 256 ? 512 : 256;
     int64_t nz = want / base;
     if (nz > s.nchunk) nz = s.nchunk;
@@ -686,7 +721,7 @@ static void ens_f32_split(EnsF32Shape &s, int64_t N, int64_t ld, int64_t Mp)
 }
 
 template <int WM, int TB, int NW>
-static int ens_f32_attr(const EnsF32Shape &s)
+static int ens_f32_attr(const EnsShape &s)
 {
     OQ_HIP(hipFuncSetAttribute((const void *)k_ens_gemm_f32<WM, TB, NW, false>,
                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)s.lds));
@@ -696,7 +731,7 @@ static int ens_f32_attr(const EnsF32Shape &s)
 }
 
 template <int WM, int TB, int NW>
-static void ens_f32_launch(const EnsDev &d, const EnsF32Shape &s, const float *K, const float *Sm, double *Y, float *part,
+static void ens_f32_launch(const EnsDev &d, const EnsShape &s, const float *K, const float *Sm, double *Y, float *part,
                            hipStream_t st)
 {
     const dim3 grid((unsigned)((d.N + s.bm - 1) / s.bm), (unsigned)(d.Mp / s.bn), (unsigned)s.nz);
@@ -706,14 +741,36 @@ static void ens_f32_launch(const EnsDev &d, const EnsF32Shape &s, const float *K
         hipLaunchKernelGGL((k_ens_gemm_f32<WM, TB, NW, false>), grid, dim3(64 * NW), s.lds, st, d, s, K, Sm, Y, part);
 }
 
-#define OQ_ENS_F32(s, f, ...)                              \
+template <int WM, int TB, int NW>
+static int ens_h3_attr(const EnsShape &s)
+{
+    OQ_HIP(hipFuncSetAttribute((const void *)k_ens_gemm_h3<WM, TB, NW, false>,
+                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)s.lds));
+    OQ_HIP(hipFuncSetAttribute((const void *)k_ens_gemm_h3<WM, TB, NW, true>,
+                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)s.lds));
+    return OQ_OK;
+}
+
+template <int WM, int TB, int NW>
+static void ens_h3_launch(const EnsDev &d, const EnsH3 &h, const EnsShape &s, double *part, hipStream_t st)
+{
+    const dim3 grid((unsigned)((d.N + s.bm - 1) / s.bm), (unsigned)(d.Mp / s.bn), (unsigned)s.nz);
+    if (s.nz > 1) hipLaunchKernelGGL((k_ens_gemm_h3<WM, TB, NW, true>), grid, dim3(64 * NW), s.lds, st, d, h, s, part);
+    else hipLaunchKernelGGL((k_ens_gemm_h3<WM, TB, NW, false>), grid, dim3(64 * NW), s.lds, st, d, h, s, part);
+}
+
+#define OQ_ENS_TILED(s, f, ...)                             \
     ((s).bn == 32 ? f<1, 1, 4>(__VA_ARGS__) : (s).bn == 64 ? f<1, 2, 4>(__VA_ARGS__) \
      : (s).bn == 128 ? f<2, 2, 8>(__VA_ARGS__) : f<4, 2, 8>(__VA_ARGS__))
 
-// epilogue of the GEMMs: one thread per (row, member); nchunk > 0: the row
-// sum is added up here from the chunks' FP32 sums, in order
+// Epilogue of the GEMMs: one thread per (row, member).  nchunk > 0: the row
+// sum is added up here from the chunks' sums, in order: the FP32 GEMM's FP32
+// sums, or (ssc set) the split-FP16 GEMM's FP64 ones with the member's chunk
+// scales and the row's scale rsc.
+template <class P>
 __global__ void __launch_bounds__(256) k_ens_finish(EnsDev d, const double *__restrict__ Y,
-                                                    const float *__restrict__ part, int nchunk,
+                                                    const P *__restrict__ part, int nchunk,
+                                                    const double *__restrict__ ssc, const double *__restrict__ rsc,
                                                     const double *__restrict__ u, double *__restrict__ du)
 {
     if (!*d.live) return;
@@ -722,10 +779,17 @@ __global__ void __launch_bounds__(256) k_ens_finish(EnsDev d, const double *__re
     const int64_t row = t / d.M, m = t % d.M;
     double y = 0.0;
     if (nchunk > 0) {
-        const float *p = part + row * d.Mp + m;
+        const P *p = part + row * d.Mp + m;
         const int64_t cs = d.N * d.Mp;
+        if constexpr (sizeof(P) == 8) {
 #pragma unroll 8
-        for (int c = 0; c < nchunk; ++c) y += (double)p[c * cs];
+            for (int c = 0; c < nchunk; ++c) y += p[c * cs] * ssc[c * d.Mp + m];
+            y *= rsc[row];
+            asm("" : "+v"(y));  // rounded here, as where it is stored: no fma with what follows
+        } else {
+#pragma unroll 8
+            for (int c = 0; c < nchunk; ++c) y += (double)p[c * cs];
+        }
     } else {
         y = Y[row * d.Mp + m];
     }
@@ -1129,9 +1193,9 @@ struct oq_ensemble {
     oq_rhs *h = nullptr;  // owns K (FP32/BF16), stream, sizes, shared viscosity
     int kdtype = OQ_K_FP32;
     int64_t M = 0, Mp = 0, n = 0;
-    oq::DevBuf hK, hrsc, hS, hssc, hY;  // OQ_K_FP16X2: split operator, split S, scales, Y
+    oq::DevBuf hK, hrsc, hS, hssc, hY, hpart;  // OQ_K_FP16X2: split operator, split S, scales, Y or chunk sums
     oq::DevBuf Sm, fY, fpart;           // OQ_K_FP32: member-major S, Y or the chunks' sums
-    oq::EnsF32Shape f32{};
+    oq::EnsShape shape{};               // member tile of either GEMM
     oq::EnsH3 h3{};
     oq::DevBuf a, b, L, sigma, eta, vpl, f0, v0, S;
     oq::DevBuf u, y, k, part;
@@ -1177,21 +1241,21 @@ static int ens_rhs(oq_ensemble *e, const double *u, double *du)
     if (e->kdtype == OQ_K_FP16X2) {
         hipLaunchKernelGGL(k_h3_prep_s, dim3((unsigned)e->h3.nchunk, (unsigned)(e->Mp / 16)), dim3(256), 0,
                            h->stream, e->dev, e->h3, e->S.as<float>());
-        hipLaunchKernelGGL(k_ens_gemm_h3, dim3(nbk(h->N, kHBM), (unsigned)(e->Mp / kHBN)), dim3(512), kHLds,
-                           h->stream, e->dev, e->h3);
-        hipLaunchKernelGGL(k_ens_finish, dim3(nbk(h->N * e->M, 256)), dim3(256), 0, h->stream, e->dev,
-                           e->h3.Y, nullptr, 0, u, du);
+        const EnsShape &f = e->shape;
+        OQ_ENS_TILED(f, ens_h3_launch, e->dev, e->h3, f, e->hpart.as<double>(), h->stream);
+        hipLaunchKernelGGL(k_ens_finish<double>, dim3(nbk(h->N * e->M, 256)), dim3(256), 0, h->stream, e->dev, e->h3.Y,
+                           e->hpart.as<double>(), f.nz > 1 ? f.nchunk : 0, e->h3.ssc, e->h3.rsc, u, du);
         OQ_HIP(hipGetLastError());
         return OQ_OK;
     }
     if (h->kdtype == OQ_K_FP32) {
-        const EnsF32Shape &f = e->f32;
+        const EnsShape &f = e->shape;
         hipLaunchKernelGGL(k_ens_s_member_major, dim3((unsigned)(h->ld / 64), (unsigned)(e->Mp / 32)),
                            dim3(256), 0, h->stream, e->dev, e->S.as<float>(), e->Sm.as<float>());
-        OQ_ENS_F32(f, ens_f32_launch, e->dev, f, h->K.as<float>(), e->Sm.as<float>(), e->fY.as<double>(),
+        OQ_ENS_TILED(f, ens_f32_launch, e->dev, f, h->K.as<float>(), e->Sm.as<float>(), e->fY.as<double>(),
                    e->fpart.as<float>(), h->stream);
-        hipLaunchKernelGGL(k_ens_finish, dim3(nbk(h->N * e->M, 256)), dim3(256), 0, h->stream, e->dev,
-                           e->fY.as<double>(), e->fpart.as<float>(), f.nz > 1 ? f.nchunk : 0, u, du);
+        hipLaunchKernelGGL(k_ens_finish<float>, dim3(nbk(h->N * e->M, 256)), dim3(256), 0, h->stream, e->dev,
+                           e->fY.as<double>(), e->fpart.as<float>(), f.nz > 1 ? f.nchunk : 0, nullptr, nullptr, u, du);
         OQ_HIP(hipGetLastError());
         return OQ_OK;
     }
@@ -1302,7 +1366,9 @@ static int build_h3(oq_ensemble *e)
     if (!rc) rc = e->hrsc.alloc((size_t)h->N * 8);
     if (!rc) rc = e->hS.alloc((size_t)(e->Mp * s.ldc) * 4);
     if (!rc) rc = e->hssc.alloc((size_t)(s.nchunk * e->Mp) * 8);
-    if (!rc) rc = e->hY.alloc((size_t)(h->N * e->Mp) * 8);
+    ens_split(e->shape, h->N, s.nchunk, e->Mp);
+    if (!rc && e->shape.nz > 1) rc = e->hpart.alloc((size_t)(s.nchunk * h->N * e->Mp) * 8);
+    if (!rc && e->shape.nz == 1) rc = e->hY.alloc((size_t)(h->N * e->Mp) * 8);
     if (rc) return rc;
     s.K = e->hK.as<_Float16>();
     s.rsc = e->hrsc.as<double>();
@@ -1315,8 +1381,7 @@ static int build_h3(oq_ensemble *e)
     OQ_HIP(hipGetLastError());
     OQ_HIP(hipStreamSynchronize(h->stream));
     h->K.release();
-    OQ_HIP(hipFuncSetAttribute((const void *)k_ens_gemm_h3, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)kHLds));
+    if ((rc = OQ_ENS_TILED(e->shape, ens_h3_attr, e->shape))) return rc;
     return OQ_OK;
 }
 
@@ -1364,8 +1429,8 @@ int oq_ensemble_create(int device, const oq_fault_mesh *mf, const oq_hex8_mesh *
     oq_rhs *h = e->h;
     const int64_t M = nmembers, nf = h->nf;
     e->M = M;
-    e->f32 = ens_f32_pick(M);
-    const int64_t mb = kdtype == OQ_K_FP16X2 ? kHBN : (kdtype == OQ_K_FP32 ? e->f32.bn : EBN);
+    e->shape = ens_pick(M, kdtype == OQ_K_FP16X2 ? 3 : 2);
+    const int64_t mb = kdtype == OQ_K_BF16 ? EBN : e->shape.bn;
     e->Mp = (M + mb - 1) / mb * mb;
     e->n = h->lay.n;
     std::vector<const double *> pa(M), pb(M), pL(M), ps(M);
@@ -1428,10 +1493,10 @@ int oq_ensemble_create(int device, const oq_fault_mesh *mf, const oq_hex8_mesh *
         const size_t sb = (size_t)(e->Mp * h->ld) * 4;
         rc = e->Sm.alloc(sb);
         if (!rc && hipMemsetAsync(e->Sm.p, 0, sb, h->stream) != hipSuccess) rc = OQ_ERR_HIP;
-        ens_f32_split(e->f32, h->N, h->ld, e->Mp);
-        if (!rc && e->f32.nz > 1) rc = e->fpart.alloc((size_t)(e->f32.nchunk * h->N * e->Mp) * 4);
-        if (!rc && e->f32.nz == 1) rc = e->fY.alloc((size_t)(h->N * e->Mp) * 8);
-        if (!rc) rc = OQ_ENS_F32(e->f32, ens_f32_attr, e->f32);
+        ens_split(e->shape, h->N, h->ld / kFChunk, e->Mp);
+        if (!rc && e->shape.nz > 1) rc = e->fpart.alloc((size_t)(e->shape.nchunk * h->N * e->Mp) * 4);
+        if (!rc && e->shape.nz == 1) rc = e->fY.alloc((size_t)(h->N * e->Mp) * 8);
+        if (!rc) rc = OQ_ENS_TILED(e->shape, ens_f32_attr, e->shape);
         if (!rc && hipStreamSynchronize(h->stream) != hipSuccess) rc = OQ_ERR_HIP;
         if (rc) {
             set_error("FP32 ensemble buffers: allocation or kernel set-up failed");
