@@ -8,7 +8,7 @@
 //   - every RHS is ONE GEMM  Y = K S  (N x N by N x M), K streamed once in
 //     FP32 (or BF16) through v_mfma_f32_32x32x2f32 tiles, FP32 products
 //     accumulated in the MFMA registers for 256-column chunks and folded into
-//     an FP32 (hi, lo) two-sum pair between chunks, then the fused epilogue
+//     FP64 (BF16: an FP32 two-sum pair) between chunks, then the epilogue
 //     (rate-and-state update / viscous stress rate) per (row, member);
 //   - a lockstep Tsit5: all members evaluate stage s together, each with its
 //     own dt, error norm, PI controller state and accept/reject decision.
@@ -111,91 +111,7 @@ __device__ __forceinline__ void ens_epilogue(const EnsDev &d, int64_t row, int64
     }
 }
 
-// ---------------- GEMM + fused epilogue ----------------
-// Block: 256 threads = 4 wavefronts; tile 128 rows x 64 members; each
-// wavefront owns 32 rows x 64 members = two 32x32 MFMA tiles.  K-slices of
-// BK = 16 columns are staged through LDS.
-static constexpr int EBM = 128, EBN = 64, EBK = 16, ECHUNK = 256;
-
-template <int KT>
-__global__ void __launch_bounds__(256) k_ens_gemm(EnsDev d, const void *__restrict__ Kp,
-                                                  const float *__restrict__ S,
-                                                  const double *__restrict__ u,
-                                                  double *__restrict__ du)
-{
-    if (!*d.live) return;
-    __shared__ float As[EBM][EBK + 1];
-    __shared__ float Bs[EBK][EBN + 4];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int64_t rb = (int64_t)blockIdx.x * EBM, cb = (int64_t)blockIdx.y * EBN;
-    // global -> LDS assignments
-    const int ar = tid >> 1, ak = (tid & 1) * 8;      // A: row ar, 8 columns from ak
-    const int bk = tid >> 4, bc = (tid & 15) * 4;     // B: k row bk, 4 members from bc
-    const int64_t arow = rb + ar < d.N ? rb + ar : d.N - 1;
-    f16v acc0 = {0}, acc1 = {0};
-    float hi0[16], lo0[16], hi1[16], lo1[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) hi0[i] = lo0[i] = hi1[i] = lo1[i] = 0.f;
-    const int64_t nk = d.ld;  // zero-padded columns
-    for (int64_t k0 = 0; k0 < nk; k0 += EBK) {
-        // stage A (K rows) and B (S slice)
-        if (KT == OQ_K_FP32) {
-            const float *Krow = static_cast<const float *>(Kp) + arow * d.ld + k0 + ak;
-            const f4x x0 = __builtin_nontemporal_load(reinterpret_cast<const f4x *>(Krow));
-            const f4x x1 = __builtin_nontemporal_load(reinterpret_cast<const f4x *>(Krow) + 1);
-            As[ar][ak + 0] = x0.x; As[ar][ak + 1] = x0.y; As[ar][ak + 2] = x0.z; As[ar][ak + 3] = x0.w;
-            As[ar][ak + 4] = x1.x; As[ar][ak + 5] = x1.y; As[ar][ak + 6] = x1.z; As[ar][ak + 7] = x1.w;
-        } else {
-            const unsigned short *Krow = static_cast<const unsigned short *>(Kp) + arow * d.ld + k0 + ak;
-            const u4x w = __builtin_nontemporal_load(reinterpret_cast<const u4x *>(Krow));
-            As[ar][ak + 0] = __uint_as_float(w.x << 16); As[ar][ak + 1] = __uint_as_float(w.x & 0xffff0000u);
-            As[ar][ak + 2] = __uint_as_float(w.y << 16); As[ar][ak + 3] = __uint_as_float(w.y & 0xffff0000u);
-            As[ar][ak + 4] = __uint_as_float(w.z << 16); As[ar][ak + 5] = __uint_as_float(w.z & 0xffff0000u);
-            As[ar][ak + 6] = __uint_as_float(w.w << 16); As[ar][ak + 7] = __uint_as_float(w.w & 0xffff0000u);
-        }
-        {
-            const float4 s4 = *reinterpret_cast<const float4 *>(S + (k0 + bk) * d.Mp + cb + bc);
-            Bs[bk][bc + 0] = s4.x; Bs[bk][bc + 1] = s4.y; Bs[bk][bc + 2] = s4.z; Bs[bk][bc + 3] = s4.w;
-        }
-        __syncthreads();
-        const int r = wave * 32 + (lane & 31), kk = lane >> 5;
-#pragma unroll
-        for (int k = 0; k < EBK; k += 2) {
-            const float a = As[r][k + kk];
-            const float b0 = Bs[k + kk][lane & 31];
-            const float b1 = Bs[k + kk][32 + (lane & 31)];
-            acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b0, acc0, 0, 0, 0);
-            acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b1, acc1, 0, 0, 0);
-        }
-        __syncthreads();
-        if (((k0 + EBK) % ECHUNK) == 0 || k0 + EBK >= nk) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                two_sum(hi0[i], lo0[i], acc0[i]);
-                two_sum(hi1[i], lo1[i], acc1[i]);
-                acc0[i] = 0.f;
-                acc1[i] = 0.f;
-            }
-        }
-    }
-    // fused epilogue: element i of tile t sits at row (i/4)*8 + (lane/32)*4 + i%4
-    // and member 32 t + lane%32 of this wavefront's 32 x 64 block
-    const int64_t M = d.M;
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        const int64_t m = cb + 32 * t + (lane & 31);
-        if (m >= M) continue;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int64_t row = rb + wave * 32 + (i / 4) * 8 + (lane >> 5) * 4 + (i % 4);
-            if (row >= d.N) continue;
-            const double y = t == 0 ? (double)hi0[i] + (double)lo0[i] : (double)hi1[i] + (double)lo1[i];
-            ens_epilogue(d, row, m, y, u, du);
-        }
-    }
-}
-
-// Workgroup tile and chunk sharing of the two member-tiled GEMMs.
+// Workgroup tile and chunk sharing of the member-tiled GEMMs.
 struct EnsShape {
     int bn = 0, bm = 0, threads = 0;  // members, rows, threads per workgroup
     int nz = 1, cps = 0;              // workgroups along the chunks, chunks per workgroup
@@ -527,7 +443,7 @@ __global__ void __launch_bounds__(64 * NW) k_ens_gemm_h3(EnsDev d, EnsH3 h, EnsS
     }
 }
 
-// ---------------- FP32 GEMM (OQ_K_FP32) ----------------
+// ---------------- FP32 and BF16 GEMM (OQ_K_FP32, OQ_K_BF16) ----------------
 // A workgroup of NW wavefronts takes BM = 32 NW / WM rows x BN = 32 TB WM
 // members; wave w owns rows [32 (w % WR), +32) x members [32 TB (w / WR),
 // +32 TB): TB tiles of v_mfma_f32_32x32x2f32.  Stages of 32 columns (128 B of
@@ -544,10 +460,19 @@ __global__ void __launch_bounds__(64 * NW) k_ens_gemm_h3(EnsDev d, EnsH3 h, EnsS
 // k_ens_finish adds them up in FP64 in the order of the undivided loop, so
 // every shape gives the same bits.  Measured at N = 2927: 24 members 208 ->
 // 15 us (46 workgroups of 256 members before, 276 of 32 now).
+//
+// BF: K is BF16, widened to FP32 as a stage goes to LDS; its even columns go
+// to the lower lanes' half of a row and its odd ones to the upper's (Sm comes
+// in that order), so an MFMA step adds two neighbouring columns, and the
+// chunks are folded into an FP32 two-sum pair.  42 VCABM5 steps of 8 members
+// over 6711 rows took 51.5 ms with 128 x 64 tiles, each with all the columns
+// in 16-column stages, and take 7.9 ms.
 static constexpr int kFKS = 32, kFRow = 144, kFChunk = 256;
 
 // S (entry-major [column][member], pitch Mp) -> member-major [member][column]
-// (pitch ld), tiles of 64 columns x 32 members through LDS.
+// (pitch ld), tiles of 64 columns x 32 members through LDS.  BF: of every 32
+// columns the even ones come first.
+template <bool BF>
 __global__ void __launch_bounds__(256) k_ens_s_member_major(EnsDev d, const float *__restrict__ S,
                                                             float *__restrict__ Sm)
 {
@@ -558,29 +483,31 @@ __global__ void __launch_bounds__(256) k_ens_s_member_major(EnsDev d, const floa
     for (int r = ty; r < 64; r += 8) tile[r][tx] = S[(c0 + r) * d.Mp + m0 + tx];  // r: column
     __syncthreads();
     const int cx = threadIdx.x & 63, my = threadIdx.x >> 6;
-    for (int r = my; r < 32; r += 4) Sm[(m0 + r) * d.ld + c0 + cx] = tile[cx][r];  // r: member
+    const int sx = BF ? (cx & 32) | (cx & 15) << 1 | (cx >> 4 & 1) : cx;
+    for (int r = my; r < 32; r += 4) Sm[(m0 + r) * d.ld + c0 + cx] = tile[sx][r];  // r: member
 }
 
-template <int WM, int TB, int NW, bool SPLIT>
-__global__ void __launch_bounds__(64 * NW) k_ens_gemm_f32(EnsDev d, EnsShape sh, const float *__restrict__ K,
+template <int WM, int TB, int NW, bool SPLIT, bool BF>
+__global__ void __launch_bounds__(64 * NW) k_ens_gemm_f32(EnsDev d, EnsShape sh, const void *__restrict__ K,
                                                           const float *__restrict__ Sm, double *__restrict__ Y,
                                                           float *__restrict__ part)
 {
     if (!*d.live) return;
     constexpr int WR = NW / WM, BM = 32 * WR, BN = 32 * TB * WM, T = 64 * NW;
-    constexpr int PK = BM * 8 / T, PS = BN * 8 / T, STAGE = (BM + BN) * kFRow;
+    constexpr int NK = BM * (BF ? 4 : 8);  // 16-byte pieces of K per stage
+    constexpr int PK = (NK + T - 1) / T, PS = BN * 8 / T, STAGE = (BM + BN) * kFRow;
     extern __shared__ __attribute__((aligned(16))) unsigned char flds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wr = wave % WR, wm = wave / WR;
     const int64_t rb = (int64_t)blockIdx.x * BM, m0 = (int64_t)blockIdx.y * BN;
-    const int64_t rowb = 4 * d.ld;  // bytes per row of K and of Sm
+    const int64_t rowb = 4 * d.ld, krowb = (BF ? 2 : 4) * d.ld;  // bytes per row of Sm and of K
     const unsigned char *kg[PK], *sg[PS];
     int kl[PK], sl[PS];
 #pragma unroll
     for (int i = 0; i < PK; ++i) {
-        const int p = tid + T * i, r = p >> 3, pc = p & 7;
+        const int p = (tid + T * i) % NK, r = BF ? p >> 2 : p >> 3, pc = BF ? p & 3 : p & 7;
         const int64_t row = rb + r < d.N ? rb + r : d.N - 1;
-        kg[i] = reinterpret_cast<const unsigned char *>(K) + row * rowb + 16 * pc;
+        kg[i] = static_cast<const unsigned char *>(K) + row * krowb + 16 * pc;
         kl[i] = r * kFRow + 16 * pc;
     }
 #pragma unroll
@@ -592,23 +519,35 @@ __global__ void __launch_bounds__(64 * NW) k_ens_gemm_f32(EnsDev d, EnsShape sh,
     u4x pa[PK + PS], pb[PK + PS];
     auto gload = [&](u4x *pr, int64_t k0) {  // k0: first column of the stage
 #pragma unroll
-        for (int i = 0; i < PK; ++i) pr[i] = __builtin_nontemporal_load(reinterpret_cast<const u4x *>(kg[i] + 4 * k0));
+        for (int i = 0; i < PK; ++i) pr[i] = __builtin_nontemporal_load(reinterpret_cast<const u4x *>(kg[i] + (BF ? 2 : 4) * k0));
 #pragma unroll
         for (int i = 0; i < PS; ++i) pr[PK + i] = *reinterpret_cast<const u4x *>(sg[i] + 4 * k0);
     };
     auto lstore = [&](const u4x *pr, unsigned char *st) {
 #pragma unroll
-        for (int i = 0; i < PK; ++i) *reinterpret_cast<u4x *>(st + kl[i]) = pr[i];
+        for (int i = 0; i < PK; ++i) {
+            if constexpr (BF) {
+                if (NK % T && tid + T * i >= NK) continue;
+                *reinterpret_cast<u4x *>(st + kl[i]) = pr[i] << 16;
+                *reinterpret_cast<u4x *>(st + kl[i] + 64) = pr[i] & 0xffff0000u;
+            } else {
+                *reinterpret_cast<u4x *>(st + kl[i]) = pr[i];
+            }
+        }
 #pragma unroll
         for (int i = 0; i < PS; ++i) *reinterpret_cast<u4x *>(st + sl[i]) = pr[PK + i];
     };
     f16v acc[TB];
-    double y[TB][16];
+    double y[TB][16];              // !BF
+    float hi[TB][16], lo[TB][16];  // BF
 #pragma unroll
     for (int b = 0; b < TB; ++b) {
         acc[b] = f16v{0};
 #pragma unroll
-        for (int i = 0; i < 16; ++i) y[b][i] = 0.0;
+        for (int i = 0; i < 16; ++i) {
+            y[b][i] = 0.0;
+            hi[b][i] = lo[b][i] = 0.f;
+        }
     }
     const int lr = lane & 31, lg = lane >> 5;
     auto compute = [&](const unsigned char *cur) {
@@ -642,6 +581,8 @@ __global__ void __launch_bounds__(64 * NW) k_ens_gemm_f32(EnsDev d, EnsShape sh,
                 if constexpr (SPLIT) {
                     const int64_t row = row0 + (i / 4) * 8 + (i % 4);
                     if (row < d.N) part[(c * d.N + row) * d.Mp + mem + b * 32] = acc[b][i];
+                } else if constexpr (BF) {
+                    two_sum(hi[b][i], lo[b][i], acc[b][i]);
                 } else {
                     y[b][i] += (double)acc[b][i];
                 }
@@ -680,7 +621,8 @@ __global__ void __launch_bounds__(64 * NW) k_ens_gemm_f32(EnsDev d, EnsShape sh,
             const int64_t row = row0 + (i / 4) * 8 + (i % 4);
             if (row >= d.N) continue;
 #pragma unroll
-            for (int b = 0; b < TB; ++b) Y[row * d.Mp + mem + b * 32] = y[b][i];
+            for (int b = 0; b < TB; ++b)
+                Y[row * d.Mp + mem + b * 32] = BF ? (double)hi[b][i] + (double)lo[b][i] : y[b][i];
         }
     }
 }
@@ -720,25 +662,26 @@ static void ens_split(EnsShape &s, int64_t N, int64_t nchunk, int64_t Mp)
     s.nz = (s.nchunk + s.cps - 1) / s.cps;
 }
 
-template <int WM, int TB, int NW>
+template <int WM, int TB, int NW, bool BF>
 static int ens_f32_attr(const EnsShape &s)
 {
-    OQ_HIP(hipFuncSetAttribute((const void *)k_ens_gemm_f32<WM, TB, NW, false>,
+    OQ_HIP(hipFuncSetAttribute((const void *)k_ens_gemm_f32<WM, TB, NW, false, BF>,
                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)s.lds));
-    OQ_HIP(hipFuncSetAttribute((const void *)k_ens_gemm_f32<WM, TB, NW, true>,
+    OQ_HIP(hipFuncSetAttribute((const void *)k_ens_gemm_f32<WM, TB, NW, true, BF>,
                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)s.lds));
     return OQ_OK;
 }
 
-template <int WM, int TB, int NW>
-static void ens_f32_launch(const EnsDev &d, const EnsShape &s, const float *K, const float *Sm, double *Y, float *part,
+template <int WM, int TB, int NW, bool BF>
+static void ens_f32_launch(const EnsDev &d, const EnsShape &s, const void *K, const float *Sm, double *Y, float *part,
                            hipStream_t st)
 {
     const dim3 grid((unsigned)((d.N + s.bm - 1) / s.bm), (unsigned)(d.Mp / s.bn), (unsigned)s.nz);
     if (s.nz > 1)
-        hipLaunchKernelGGL((k_ens_gemm_f32<WM, TB, NW, true>), grid, dim3(64 * NW), s.lds, st, d, s, K, Sm, Y, part);
+        hipLaunchKernelGGL((k_ens_gemm_f32<WM, TB, NW, true, BF>), grid, dim3(64 * NW), s.lds, st, d, s, K, Sm, Y, part);
     else
-        hipLaunchKernelGGL((k_ens_gemm_f32<WM, TB, NW, false>), grid, dim3(64 * NW), s.lds, st, d, s, K, Sm, Y, part);
+        hipLaunchKernelGGL((k_ens_gemm_f32<WM, TB, NW, false, BF>), grid, dim3(64 * NW), s.lds, st, d, s, K, Sm, Y,
+                           part);
 }
 
 template <int WM, int TB, int NW>
@@ -759,17 +702,21 @@ static void ens_h3_launch(const EnsDev &d, const EnsH3 &h, const EnsShape &s, do
     else hipLaunchKernelGGL((k_ens_gemm_h3<WM, TB, NW, false>), grid, dim3(64 * NW), s.lds, st, d, h, s, part);
 }
 
-#define OQ_ENS_TILED(s, f, ...)                             \
-    ((s).bn == 32 ? f<1, 1, 4>(__VA_ARGS__) : (s).bn == 64 ? f<1, 2, 4>(__VA_ARGS__) \
-     : (s).bn == 128 ? f<2, 2, 8>(__VA_ARGS__) : f<4, 2, 8>(__VA_ARGS__))
+// f<the tile of s, t>(...)
+#define OQ_ENS_TILED(s, f, t, ...)                                                          \
+    ((s).bn == 32 ? f<1, 1, 4 t>(__VA_ARGS__) : (s).bn == 64 ? f<1, 2, 4 t>(__VA_ARGS__)    \
+     : (s).bn == 128 ? f<2, 2, 8 t>(__VA_ARGS__) : f<4, 2, 8 t>(__VA_ARGS__))
+#define OQ_ENS_F32 , false
+#define OQ_ENS_BF16 , true
 
 // Epilogue of the GEMMs: one thread per (row, member).  nchunk > 0: the row
-// sum is added up here from the chunks' sums, in order: the FP32 GEMM's FP32
-// sums, or (ssc set) the split-FP16 GEMM's FP64 ones with the member's chunk
-// scales and the row's scale rsc.
-template <class P>
+// sum is added up here from the chunks' sums, in order and as the undivided
+// loop adds them: FP32 ones into FP64, BF16's into a two-sum pair, the
+// split-FP16 GEMM's FP64 ones with the member's chunk scales ssc and the
+// row's scale rsc.
+template <int KT>
 __global__ void __launch_bounds__(256) k_ens_finish(EnsDev d, const double *__restrict__ Y,
-                                                    const P *__restrict__ part, int nchunk,
+                                                    const void *__restrict__ part, int nchunk,
                                                     const double *__restrict__ ssc, const double *__restrict__ rsc,
                                                     const double *__restrict__ u, double *__restrict__ du)
 {
@@ -779,14 +726,21 @@ __global__ void __launch_bounds__(256) k_ens_finish(EnsDev d, const double *__re
     const int64_t row = t / d.M, m = t % d.M;
     double y = 0.0;
     if (nchunk > 0) {
-        const P *p = part + row * d.Mp + m;
-        const int64_t cs = d.N * d.Mp;
-        if constexpr (sizeof(P) == 8) {
+        const int64_t o = row * d.Mp + m, cs = d.N * d.Mp;
+        if constexpr (KT == OQ_K_FP16X2) {
+            const double *p = static_cast<const double *>(part) + o;
 #pragma unroll 8
             for (int c = 0; c < nchunk; ++c) y += p[c * cs] * ssc[c * d.Mp + m];
             y *= rsc[row];
             asm("" : "+v"(y));  // rounded here, as where it is stored: no fma with what follows
+        } else if constexpr (KT == OQ_K_BF16) {
+            const float *p = static_cast<const float *>(part) + o;
+            float hi = 0.f, lo = 0.f;
+#pragma unroll 8
+            for (int c = 0; c < nchunk; ++c) two_sum(hi, lo, p[c * cs]);
+            y = (double)hi + (double)lo;
         } else {
+            const float *p = static_cast<const float *>(part) + o;
 #pragma unroll 8
             for (int c = 0; c < nchunk; ++c) y += (double)p[c * cs];
         }
@@ -1194,7 +1148,7 @@ struct oq_ensemble {
     int kdtype = OQ_K_FP32;
     int64_t M = 0, Mp = 0, n = 0;
     oq::DevBuf hK, hrsc, hS, hssc, hY, hpart;  // OQ_K_FP16X2: split operator, split S, scales, Y or chunk sums
-    oq::DevBuf Sm, fY, fpart;           // OQ_K_FP32: member-major S, Y or the chunks' sums
+    oq::DevBuf Sm, fY, fpart;           // OQ_K_FP32, OQ_K_BF16: member-major S, Y or the chunks' sums
     oq::EnsShape shape{};               // member tile of either GEMM
     oq::EnsH3 h3{};
     oq::DevBuf a, b, L, sigma, eta, vpl, f0, v0, S;
@@ -1242,26 +1196,26 @@ static int ens_rhs(oq_ensemble *e, const double *u, double *du)
         hipLaunchKernelGGL(k_h3_prep_s, dim3((unsigned)e->h3.nchunk, (unsigned)(e->Mp / 16)), dim3(256), 0,
                            h->stream, e->dev, e->h3, e->S.as<float>());
         const EnsShape &f = e->shape;
-        OQ_ENS_TILED(f, ens_h3_launch, e->dev, e->h3, f, e->hpart.as<double>(), h->stream);
-        hipLaunchKernelGGL(k_ens_finish<double>, dim3(nbk(h->N * e->M, 256)), dim3(256), 0, h->stream, e->dev, e->h3.Y,
+        OQ_ENS_TILED(f, ens_h3_launch, , e->dev, e->h3, f, e->hpart.as<double>(), h->stream);
+        hipLaunchKernelGGL(k_ens_finish<OQ_K_FP16X2>, dim3(nbk(h->N * e->M, 256)), dim3(256), 0, h->stream, e->dev, e->h3.Y,
                            e->hpart.as<double>(), f.nz > 1 ? f.nchunk : 0, e->h3.ssc, e->h3.rsc, u, du);
         OQ_HIP(hipGetLastError());
         return OQ_OK;
     }
-    if (h->kdtype == OQ_K_FP32) {
-        const EnsShape &f = e->shape;
-        hipLaunchKernelGGL(k_ens_s_member_major, dim3((unsigned)(h->ld / 64), (unsigned)(e->Mp / 32)),
-                           dim3(256), 0, h->stream, e->dev, e->S.as<float>(), e->Sm.as<float>());
-        OQ_ENS_TILED(f, ens_f32_launch, e->dev, f, h->K.as<float>(), e->Sm.as<float>(), e->fY.as<double>(),
-                   e->fpart.as<float>(), h->stream);
-        hipLaunchKernelGGL(k_ens_finish<float>, dim3(nbk(h->N * e->M, 256)), dim3(256), 0, h->stream, e->dev,
-                           e->fY.as<double>(), e->fpart.as<float>(), f.nz > 1 ? f.nchunk : 0, nullptr, nullptr, u, du);
-        OQ_HIP(hipGetLastError());
-        return OQ_OK;
-    }
-    const dim3 grid(nbk(h->N, EBM), (unsigned)(e->Mp / EBN));
-        hipLaunchKernelGGL(k_ens_gemm<OQ_K_BF16>, grid, dim3(256), 0, h->stream, e->dev, h->K.p,
-                           e->S.as<float>(), u, du);
+    const EnsShape &f = e->shape;
+    const bool bf = h->kdtype == OQ_K_BF16;
+    hipLaunchKernelGGL(bf ? k_ens_s_member_major<true> : k_ens_s_member_major<false>,
+                       dim3((unsigned)(h->ld / 64), (unsigned)(e->Mp / 32)), dim3(256), 0, h->stream, e->dev,
+                       e->S.as<float>(), e->Sm.as<float>());
+    if (bf)
+        OQ_ENS_TILED(f, ens_f32_launch, OQ_ENS_BF16, e->dev, f, h->K.p, e->Sm.as<float>(), e->fY.as<double>(),
+                     e->fpart.as<float>(), h->stream);
+    else
+        OQ_ENS_TILED(f, ens_f32_launch, OQ_ENS_F32, e->dev, f, h->K.p, e->Sm.as<float>(), e->fY.as<double>(),
+                     e->fpart.as<float>(), h->stream);
+    hipLaunchKernelGGL(bf ? k_ens_finish<OQ_K_BF16> : k_ens_finish<OQ_K_FP32>, dim3(nbk(h->N * e->M, 256)), dim3(256), 0,
+                       h->stream, e->dev, e->fY.as<double>(), e->fpart.p, f.nz > 1 ? f.nchunk : 0, nullptr, nullptr, u,
+                       du);
     OQ_HIP(hipGetLastError());
     return OQ_OK;
 }
@@ -1381,7 +1335,7 @@ static int build_h3(oq_ensemble *e)
     OQ_HIP(hipGetLastError());
     OQ_HIP(hipStreamSynchronize(h->stream));
     h->K.release();
-    if ((rc = OQ_ENS_TILED(e->shape, ens_h3_attr, e->shape))) return rc;
+    if ((rc = OQ_ENS_TILED(e->shape, ens_h3_attr, , e->shape))) return rc;
     return OQ_OK;
 }
 
@@ -1430,7 +1384,7 @@ int oq_ensemble_create(int device, const oq_fault_mesh *mf, const oq_hex8_mesh *
     const int64_t M = nmembers, nf = h->nf;
     e->M = M;
     e->shape = ens_pick(M, kdtype == OQ_K_FP16X2 ? 3 : 2);
-    const int64_t mb = kdtype == OQ_K_BF16 ? EBN : e->shape.bn;
+    const int64_t mb = e->shape.bn;
     e->Mp = (M + mb - 1) / mb * mb;
     e->n = h->lay.n;
     std::vector<const double *> pa(M), pb(M), pL(M), ps(M);
@@ -1489,17 +1443,19 @@ int oq_ensemble_create(int device, const oq_fault_mesh *mf, const oq_hex8_mesh *
         ens_destroy(e);
         return rc;
     }
-    if (kdtype == OQ_K_FP32) {
+    if (kdtype != OQ_K_FP16X2) {
         const size_t sb = (size_t)(e->Mp * h->ld) * 4;
         rc = e->Sm.alloc(sb);
         if (!rc && hipMemsetAsync(e->Sm.p, 0, sb, h->stream) != hipSuccess) rc = OQ_ERR_HIP;
         ens_split(e->shape, h->N, h->ld / kFChunk, e->Mp);
         if (!rc && e->shape.nz > 1) rc = e->fpart.alloc((size_t)(e->shape.nchunk * h->N * e->Mp) * 4);
         if (!rc && e->shape.nz == 1) rc = e->fY.alloc((size_t)(h->N * e->Mp) * 8);
-        if (!rc) rc = OQ_ENS_TILED(e->shape, ens_f32_attr, e->shape);
+        if (!rc)
+            rc = kdtype == OQ_K_BF16 ? OQ_ENS_TILED(e->shape, ens_f32_attr, OQ_ENS_BF16, e->shape)
+                                     : OQ_ENS_TILED(e->shape, ens_f32_attr, OQ_ENS_F32, e->shape);
         if (!rc && hipStreamSynchronize(h->stream) != hipSuccess) rc = OQ_ERR_HIP;
         if (rc) {
-            set_error("FP32 ensemble buffers: allocation or kernel set-up failed");
+            set_error("ensemble buffers: allocation or kernel set-up failed");
             ens_destroy(e);
             return rc;
         }

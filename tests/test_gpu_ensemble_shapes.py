@@ -1,9 +1,9 @@
-"""The FP32 ensemble GEMM's shapes: member tiles of 32, 64, 128 and 256, with
+"""The ensemble GEMMs' shapes: member tiles of 32, 64, 128 and 256, with
 the chunks of a row sum shared out over workgroups (small models) and not
 (one row block per CU or more).  Every shape adds the same products in the
 same order, so a member's derivative has the same bits whatever the ensemble
 around it; and it equals the member's own FP64 right-hand side to the FP32
-operator's 2e-6."""
+operator's 2e-6 (2e-2 with the BF16 operator)."""
 import numpy as np
 import pytest
 
@@ -25,7 +25,7 @@ def _members(mf, ma, M, rng):
     return members, U
 
 
-@pytest.mark.parametrize("kdtype", ["fp32", "fp16x2"])
+@pytest.mark.parametrize("kdtype", ["fp32", "fp16x2", "bf16"])
 @pytest.mark.parametrize("coupled", [True, False])
 def test_every_member_tile_gives_the_same_bits(rng, kdtype, coupled):
     mf, ma = small_fault(90.0, x=40e3, xi=15e3, d=1.25e3), small_mantle() if coupled else None
@@ -46,4 +46,4 @@ def test_every_member_tile_gives_the_same_bits(rng, kdtype, coupled):
         um, dm = oq.similar(u).unpack(U[m]), oq.similar(u)
         p.f(dm, um, None, 0.0)
         p.f.close()
-        assert relerr(ref[m], dm.pack()) <= 2e-6, m
+        assert relerr(ref[m], dm.pack()) <= (2e-2 if kdtype == "bf16" else 2e-6), m
