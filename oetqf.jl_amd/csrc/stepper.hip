@@ -401,115 +401,136 @@ __global__ void __launch_bounds__(256) k_ab_commit(const AbCtrl *__restrict__ a,
 // For a few hundred to a few thousand patches the graph above is bound by
 // its ~23 kernel launches per step, not by arithmetic.  Here one cooperative
 // launch runs up to max_steps attempted steps: workgroup w owns patches
-// [w R, w R + R) -- their rows of K live in its LDS, and so do their entries
-// of u, the stage state and the seven stages.  Each RHS needs the whole
-// source vector s = v - vpl, published through device memory and one grid
-// barrier (two buffers by stage parity, so a workgroup that is ahead never
-// overwrites a vector another is still reading); the error norm and max|v|
-// partials need one more.  The next step's first stage rides on that last
-// barrier (both candidates for its source vector are published with the
-// partials), so a step after the first of a launch costs six barriers.
+// [w R, w R + R) -- their rows of K live in its registers, and their entries
+// of u, the stage state and the seven stages in its LDS.  Each RHS needs the
+// whole source vector s = v - vpl: one exchange between the workgroups; the
+// error norm and max|v| partials need one more.  The next step's first stage
+// rides on that one (both candidates for its source vector are published with
+// the partials), so a step after the first of a launch costs six exchanges.
 // Every workgroup then runs the same controller on the same sums in the same
 // order, so all copies of t, dt and the step counters stay identical without
-// further communication.  Barrier waits
-// are bounded by a wall-clock limit: a workgroup that times out raises the
-// abort flag and every workgroup leaves at its next barrier.
+// further communication.
+//
+// What bounds a step is the latency of the exchange.  Every value travels
+// with its exchange's number: a double is two 64-bit words, number | half,
+// stored and loaded as relaxed agent-scope atomics, so a reader polls the
+// values themselves and one store and one load cross the chip.  (A counter
+// that the workgroups add to cost a release, an add, a poll, an acquire and
+// then the loads.)  Consecutive exchanges use different words, and a workgroup
+// publishes exchange e only after it has read all of e - 1, which every other
+// one published after it had read all of e - 2: no word is overwritten before
+// it has been read by all.  Waits are bounded by a wall-clock limit: a
+// workgroup that times out raises the abort flag and every workgroup leaves at
+// its next exchange.
+//
+// With N = 512 a Tsit5 step takes 16.4 us; 24.1 with counter barriers and K in
+// LDS.
 struct PersistArgs {
     RhsDev d;
     const double *K;   // FP64 operator, N x ld
     Ctrl *ctrl;
     double *u, *k1;    // packed state and the FSAL stage
-    double *s2;        // 2 x N source vectors, then (Tsit5) 4 x N stage-1 candidates
-    double *part;      // 2 x nwg: squared-error sums, max |v|
-    unsigned *bar;     // barrier arrivals (zero at launch)
+    // two source vectors, (Tsit5) four stage-1 candidate vectors, then per
+    // workgroup its squared-error sum and max |v|: two words each, zero at launch
+    unsigned long long *x;
     int *abort;
     Recorder rec;
     int recording, R, nwg;
     long long max_steps, wait_ticks;
 };
 
-// tau[r] = K row r . s for the owned rows, K rows in LDS at a pitch of
-// ldp = ld + 2 doubles, s in LDS.  Sixteen lanes share two rows (r and
-// r + 16 of a 32-row block): lane q sums the column pairs 32k + 2q,
-// 32k + 2q + 1 of both rows with one 16-byte LDS read of s and one of each
-// row per pair (the sixteen lanes of a row read 256 contiguous bytes), two
-// accumulators per row, and four DPP steps sum the sixteen lanes.  Rows
-// past Rv repeat row Rv - 1 and are not stored.
-__device__ __forceinline__ void lds_rows(const double *Ks, const double *sv, int64_t ld, int64_t ldp, int Rv,
-                                         int tid, double *tau)
+__device__ __forceinline__ void x_put(unsigned long long *x, int64_t i, unsigned ep, double v)
 {
-    const int q = tid & 15, rp = tid >> 4;
-    for (int r0 = 0; r0 < Rv; r0 += 32) {
-        const int ra = r0 + rp, rb = ra + 16;
-        const double *ka = Ks + (size_t)(ra < Rv ? ra : Rv - 1) * ldp + 2 * q;
-        const double *kb = Ks + (size_t)(rb < Rv ? rb : Rv - 1) * ldp + 2 * q;
-        const double *sp = sv + 2 * q;
-        double a0 = 0.0, a1 = 0.0, b0 = 0.0, b1 = 0.0;
-        for (int64_t c = 0; c < ld; c += 128) {  // ld is a multiple of 512: four pairs per pass, loads first
-            double2 s2[4], x2[4], y2[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                s2[u] = *reinterpret_cast<const double2 *>(sp + c + 32 * u);
-                x2[u] = *reinterpret_cast<const double2 *>(ka + c + 32 * u);
-                y2[u] = *reinterpret_cast<const double2 *>(kb + c + 32 * u);
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                a0 += x2[u].x * s2[u].x;
-                a1 += x2[u].y * s2[u].y;
-                b0 += y2[u].x * s2[u].x;
-                b1 += y2[u].y * s2[u].y;
-            }
-        }
-        double xa = a0 + a1, xb = b0 + b1;
-        xa += dpp_f64<0xB1>(xa);   // quad_perm [1,0,3,2]
-        xb += dpp_f64<0xB1>(xb);
-        xa += dpp_f64<0x4E>(xa);   // quad_perm [2,3,0,1]
-        xb += dpp_f64<0x4E>(xb);
-        xa += dpp_f64<0x141>(xa);  // row_half_mirror: the two quads of each 8 lanes
-        xb += dpp_f64<0x141>(xb);
-        xa += dpp_f64<0x140>(xa);  // row_mirror: the two 8-lane halves of the 16
-        xb += dpp_f64<0x140>(xb);
-        if (q == 0 && ra < Rv) tau[ra] = xa;
-        if (q == 0 && rb < Rv) tau[rb] = xb;
-    }
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v), t = (unsigned long long)ep << 32;
+    __hip_atomic_store(x + 2 * i, t | (b & 0xffffffffull), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(x + 2 * i + 1, t | b >> 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <class F>
-__device__ __forceinline__ bool grid_barrier(const PersistArgs &a, unsigned &epoch, int *sh_bad, F side)
+// put(j, value j) for j = j0, j0 + 192, ... < n (at most U of them): waits for
+// each value's words to carry ep.
+template <int U, class F>
+__device__ __forceinline__ void x_get(const PersistArgs &a, const unsigned long long *x, int j0, int n, unsigned ep,
+                                      int *sh_bad, F put)
 {
-    __syncthreads();
-    ++epoch;
-    if (threadIdx.x == 0) {
-        const unsigned target = epoch * (unsigned)a.nwg;
-        __hip_atomic_fetch_add(a.bar, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-        const long long t0 = (long long)wall_clock64();
-        int bad = 0;
-        while (__hip_atomic_load(a.bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
-            if (__hip_atomic_load(a.abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-                bad = 1;
-                break;
+    unsigned long long w[U][2];
+    long long t0 = 0;
+    for (unsigned spin = 0;; ++spin) {
+        bool ok = true;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int j = j0 + 192 * u;
+            if (j < n) {
+                w[u][0] = __hip_atomic_load(x + 2 * j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                w[u][1] = __hip_atomic_load(x + 2 * j + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
-            if ((long long)wall_clock64() - t0 > a.wait_ticks) {
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (j0 + 192 * u < n) ok = ok && (unsigned)(w[u][0] >> 32) == ep && (unsigned)(w[u][1] >> 32) == ep;
+        if (ok) break;
+        if (spin % 64 == 63) {
+            const long long now = (long long)wall_clock64();
+            if (spin == 63) t0 = now;
+            if (__hip_atomic_load(a.abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) || now - t0 > a.wait_ticks) {
                 __hip_atomic_store(a.abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                bad = 1;
-                break;
+                *sh_bad = 1;
+                return;
             }
-            __builtin_amdgcn_s_sleep(1);
         }
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-        *sh_bad = bad;
-    } else if (threadIdx.x >= 64) {
-        side();  // wavefronts 1..3, while thread 0 waits
     }
-    __syncthreads();
-    return *sh_bad == 0;
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        if (j0 + 192 * u < n)
+            put(j0 + 192 * u, __longlong_as_double((long long)(w[u][1] << 32 | (w[u][0] & 0xffffffffull))));
 }
 
-__device__ __forceinline__ bool grid_barrier(const PersistArgs &a, unsigned &epoch, int *sh_bad)
-{
-    return grid_barrier(a, epoch, sh_bad, [] {});
-}
+// The owned rows of K, in registers: sixteen lanes share the rows r = tid / 16
+// and (LD = 512, R = 32) r + 16; lane q of them holds the column pairs
+// 32k + 2q, 32k + 2q + 1.  A sweep reads s from LDS (16 bytes per pair, the
+// sixteen lanes 256 contiguous bytes), keeps two accumulators per row and sums
+// the sixteen lanes in four DPP steps.  Rows past Rv repeat row Rv - 1 and are
+// not stored.
+template <int LD>
+struct OwnRows {
+    static constexpr int NR = LD == 512 ? 2 : 1, NP = LD / 32;
+    static constexpr int U = LD == 512 ? 3 : LD == 1024 ? 6 : 7;  // values per polling thread: N <= 512, 1024, 1280
+    double2 k[NR][NP];
+    __device__ __forceinline__ void load(const double *K, int64_t p0, int Rv, int tid)
+    {
+        const int q = tid & 15, rp = tid >> 4;
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+            const int row = rp + 16 * r < Rv ? rp + 16 * r : Rv - 1;
+            const double *kr = K + (p0 + row) * LD + 2 * q;
+#pragma unroll
+            for (int c = 0; c < NP; ++c) k[r][c] = *reinterpret_cast<const double2 *>(kr + 32 * c);
+        }
+    }
+    __device__ __forceinline__ void sweep(const double *sv, int Rv, int tid, double *tau) const
+    {
+        const int q = tid & 15, rp = tid >> 4;
+        const double *sp = sv + 2 * q;
+        double a0[NR] = {}, a1[NR] = {};
+#pragma unroll
+        for (int c = 0; c < NP; ++c) {
+            const double2 s2 = *reinterpret_cast<const double2 *>(sp + 32 * c);
+#pragma unroll
+            for (int r = 0; r < NR; ++r) {
+                a0[r] += k[r][c].x * s2.x;
+                a1[r] += k[r][c].y * s2.y;
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+            double x = a0[r] + a1[r];
+            x += dpp_f64<0xB1>(x);   // quad_perm [1,0,3,2]
+            x += dpp_f64<0x4E>(x);   // quad_perm [2,3,0,1]
+            x += dpp_f64<0x141>(x);  // row_half_mirror: the two quads of each 8 lanes
+            x += dpp_f64<0x140>(x);  // row_mirror: the two 8-lane halves of the 16
+            if (q == 0 && rp + 16 * r < Rv) tau[rp + 16 * r] = x;
+        }
+    }
+};
 
 // Maximum over the 64 lanes of a wavefront (the steps of wave_sum with fmax).
 __device__ __forceinline__ double wave_max(double x)
@@ -522,39 +543,42 @@ __device__ __forceinline__ double wave_max(double x)
     return fmax(readlane_f64(x, 0), readlane_f64(x, 32));
 }
 
+template <int LD>
 __global__ void __launch_bounds__(256) k_persist(PersistArgs a)
 {
-    extern __shared__ __attribute__((aligned(16))) double lds[];  // 16-byte LDS reads of K and s
+    extern __shared__ __attribute__((aligned(16))) double lds[];  // 16-byte LDS reads of s
     __shared__ Ctrl c;
     __shared__ double red[256], red2[256], tau[64], pdv[64], pdt[64], pth[64];
     __shared__ int bad, take;
     __shared__ long long nstep, nsnap;
     const int R = a.R, tid = threadIdx.x;
-    const int64_t N = a.d.N, ld = a.d.ld, n = a.d.lay.n;
+    const int64_t n = a.d.lay.n;
+    const int N = (int)a.d.N;
     const int64_t p0 = (int64_t)blockIdx.x * R;
     const int Rv = (int)((N - p0) < R ? (N - p0) : R);  // owned patches (>= 1)
     const int E = 3 * R;                                 // owned entries: [v | th | del]
-    const int64_t ldp = ld + 2;                          // K row pitch in LDS
-    double *Ks = lds;                                    // R x ldp
-    double *sv = Ks + (size_t)R * ldp;                   // ld
-    double *uo = sv + ld, *yo = uo + E, *ko = yo + E;    // E, E, 7 x E
+    double *sv = lds, *cu = sv + LD, *cb = cu + LD;      // s; the accepted step's stage-1 candidates
+    double *uo = cb + LD, *yo = uo + E, *ko = yo + E;    // E, E, 7 x E
     const int64_t comp_off[3] = {a.d.lay.v, a.d.lay.th, a.d.lay.del};
+    unsigned long long *xc = a.x + 4 * (int64_t)N, *xp = xc + 8 * (int64_t)N;  // candidates, partials
 
-    for (int64_t x = tid; x < (int64_t)Rv * ld; x += 256) Ks[(x / ld) * ldp + x % ld] = a.K[p0 * ld + x];
-    for (int64_t j = tid; j < ld; j += 256) sv[j] = 0.0;
+    OwnRows<LD> K;
+    K.load(a.K, p0, Rv, tid);
+    for (int j = tid; j < LD; j += 256) sv[j] = 0.0;
     for (int e = tid; e < E; e += 256) {
         const int cpt = e / R, i = e % R;
         uo[e] = i < Rv ? a.u[comp_off[cpt] + p0 + i] : 0.0;
         ko[e] = i < Rv ? a.k1[comp_off[cpt] + p0 + i] : 0.0;
     }
     if (tid == 0) {
+        bad = 0;
         c = *a.ctrl;
         nstep = a.recording ? *a.rec.nstep : 0;
         nsnap = a.recording ? *a.rec.nsnap : 0;
     }
     // thread 64 + r (r < Rv <= 64) keeps patch p0 + r's friction parameters
     // in registers and evaluates its dtau-free friction terms (fault_pre)
-    // while thread 0 waits at the grid barrier; after the LDS sweep only
+    // while wavefronts 0, 2 and 3 poll the exchange; after the sweep only
     // fault_dv remains
     double fa = 1.0, fb = 0.0, fL = 1.0, fs = 0.0;
     const int pr = tid - 64;
@@ -567,9 +591,10 @@ __global__ void __launch_bounds__(256) k_persist(PersistArgs a)
     auto pre = [&]() {
         if (pr >= 0 && pr < Rv) fault_pre(a.d, fa, fb, fL, fs, yo[pr], yo[R + pr], pdv[pr], pdt[pr], pth[pr]);
     };
+    const int pj = tid < 64 ? tid : tid - 64;  // polling threads' index (not wavefront 1's)
     __syncthreads();
     unsigned epoch = 0;
-    bool s1ready = false;  // stage 1's source vector crossed the last barrier
+    bool s1ready = false;  // stage 1's source vector came with the last exchange
     int s1acc = 0;
     for (long long it = 0; it < a.max_steps; ++it) {
         if (tid == 0) {  // k_step_begin
@@ -598,28 +623,39 @@ __global__ void __launch_bounds__(256) k_persist(PersistArgs a)
         __syncthreads();
         if (c.done) break;
         const double dt = c.dtcur;
+#pragma unroll
         for (int st = 1; st < 7; ++st) {
+            const bool ready = st == 1 && s1ready;
+            unsigned long long *xs = a.x + 2 * (int64_t)(st & 1) * N;
+            if (!ready) ++epoch;
             for (int e = tid; e < E; e += 256) {
                 double acc = 0.0;
                 for (int j = 0; j < st; ++j) acc += kTsA[st][j] * ko[j * E + e];
-                yo[e] = uo[e] + dt * acc;
+                const double y = uo[e] + dt * acc;
+                yo[e] = y;
+                if (!ready && e < Rv) x_put(xs, p0 + e, epoch, y - a.d.vpl);
             }
             __syncthreads();
-            if (st == 1 && s1ready) {
+            if ((tid >> 6) == 1) {
+                pre();
+            } else if (ready) {
                 // the previous step published both candidates for this stage's
                 // source vector with its error partials: s = (U + dt B) - vpl
                 // with the same operations as yo above
-                const double *U = a.s2 + (s1acc ? 2 : 4) * N, *B = U + N;
-                for (int64_t j = tid; j < N; j += 256) sv[j] = (U[j] + dt * B[j]) - a.d.vpl;
-                pre();
+                if (s1acc) {
+                    for (int j = pj; j < N; j += 192) sv[j] = (cu[j] + dt * cb[j]) - a.d.vpl;
+                } else {
+                    x_get<OwnRows<LD>::U>(a, xc + 4 * (int64_t)N, pj, N, epoch, &bad, [&](int j, double v) { cu[j] = v; });
+                    x_get<OwnRows<LD>::U>(a, xc + 6 * (int64_t)N, pj, N, epoch, &bad, [&](int j, double v) {
+                        sv[j] = (cu[j] + dt * v) - a.d.vpl;
+                    });
+                }
             } else {
-                double *sg = a.s2 + (st & 1) * N;
-                for (int i = tid; i < Rv; i += 256) sg[p0 + i] = yo[i] - a.d.vpl;
-                if (!grid_barrier(a, epoch, &bad, pre)) return;
-                for (int64_t j = tid; j < N; j += 256) sv[j] = sg[j];
+                x_get<OwnRows<LD>::U>(a, xs, pj, N, epoch, &bad, [&](int j, double v) { sv[j] = v; });
             }
             __syncthreads();
-            lds_rows(Ks, sv, ld, ldp, Rv, tid, tau);
+            if (bad) return;
+            K.sweep(sv, Rv, tid, tau);
             __syncthreads();
             if (tid < Rv) {  // one patch per thread
                 const int r = tid;
@@ -648,31 +684,36 @@ __global__ void __launch_bounds__(256) k_persist(PersistArgs a)
             red2[tid >> 6] = vm;
         }
         __syncthreads();
-        if (tid == 0) {
-            a.part[2 * blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
-            a.part[2 * blockIdx.x + 1] = fmax(fmax(red2[0], red2[1]), fmax(red2[2], red2[3]));
-        }
+        ++epoch;
+        if (tid < 2)
+            x_put(xp, 2 * blockIdx.x + tid, epoch,
+                  tid == 0 ? (red[0] + red[1]) + (red[2] + red[3])
+                           : fmax(fmax(red2[0], red2[1]), fmax(red2[2], red2[3])));
         // Stage 1 of the next attempt needs y = u + dt a21 k1 with (u, k1) =
         // (y_{n+1}, k7) after an acceptance or (u_n, k1) after a rejection,
         // and dt from the controller.  Both (u, a21 k1) candidates of the
-        // owned v entries cross this barrier with the partials, so the next
-        // step's first stage needs no barrier of its own.
-        {
-            double *C = a.s2 + 2 * N;  // [U_acc | B_acc | U_rej | B_rej]
-            for (int i = tid; i < Rv; i += 256) {
-                double b6 = 0.0, b1 = 0.0;
-                b6 += kTsA[1][0] * ko[6 * E + i];
-                b1 += kTsA[1][0] * ko[i];
-                C[p0 + i] = yo[i];
-                C[N + p0 + i] = b6;
-                C[2 * N + p0 + i] = uo[i];
-                C[3 * N + p0 + i] = b1;
-            }
+        // owned v entries, [U_acc | B_acc | U_rej | B_rej], go out with the
+        // partials, so the next step's first stage needs no exchange of its own.
+        for (int i = tid - 64; i >= 0 && i < Rv; i += 256) {
+            double b6 = 0.0, b1 = 0.0;
+            b6 += kTsA[1][0] * ko[6 * E + i];
+            b1 += kTsA[1][0] * ko[i];
+            x_put(xc, p0 + i, epoch, yo[i]);
+            x_put(xc, N + p0 + i, epoch, b6);
+            x_put(xc, 2 * (int64_t)N + p0 + i, epoch, uo[i]);
+            x_put(xc, 3 * (int64_t)N + p0 + i, epoch, b1);
         }
-        if (!grid_barrier(a, epoch, &bad)) return;
-        for (int w = tid; w < 2 * a.nwg; w += 256) red[w] = a.part[w];  // all loads in flight at once
-        __syncthreads();
+        __syncthreads();  // red is written again below
+        if (tid < 64) {
+            for (int w = tid; w < 2 * a.nwg; w += 64)
+                x_get<1>(a, xp, w, w + 1, epoch, &bad, [&](int j, double v) { red[j] = v; });
+        } else {  // wavefronts 1..3 fetch the likely candidates meanwhile
+            x_get<OwnRows<LD>::U>(a, xc, tid - 64, N, epoch, &bad, [&](int j, double v) { cu[j] = v; });
+            x_get<OwnRows<LD>::U>(a, xc + 2 * (int64_t)N, tid - 64, N, epoch, &bad, [&](int j, double v) { cb[j] = v; });
+        }
+        // wavefront 0 alone reads its own red: no barrier before the controller
         if (tid < 64) {  // k_controller, on the same sums in every workgroup
+            __builtin_amdgcn_wave_barrier();
             double sum = 0.0, vmax = 0.0;
             for (int w = 0; w < a.nwg; ++w) {
                 sum += red[2 * w];
@@ -722,6 +763,7 @@ __global__ void __launch_bounds__(256) k_persist(PersistArgs a)
             }
         }
         __syncthreads();
+        if (bad) return;
         s1acc = c.accept;  // which candidate the next stage 1 takes
         s1ready = true;
         if (c.accept) {  // k_commit (FSAL: k1 <- k7)
@@ -762,32 +804,33 @@ __global__ void __launch_bounds__(256) k_persist(PersistArgs a)
 }
 
 // Persistent VCABM5: as k_persist, with the method of enqueue_step_ab.  A
-// step needs the predicted source vector (one barrier), then the error
-// partials and the corrected source vector, published together before one
-// more barrier (the corrected vector is used only when the step is
-// accepted): two grid barriers instead of Tsit5's seven.  Buffer 0 (predicted
-// s), buffer 1 (corrected s) and the partials are each rewritten only after
-// a barrier that every workgroup crosses once it has read them.
+// step needs the predicted source vector (one exchange), then the error
+// partials and the corrected source vector, published together in one more
+// (the corrected vector is used only when the step is accepted): two
+// exchanges instead of Tsit5's six.
 // Phi_0..Phi_5 of the owned entries stay in LDS across the steps of a launch.
+template <int LD>
 __global__ void __launch_bounds__(256) k_persist_ab(PersistArgs a, AbCtrl *actrl, double *phig)
 {
-    extern __shared__ __attribute__((aligned(16))) double lds[];  // 16-byte LDS reads of K and s
+    extern __shared__ __attribute__((aligned(16))) double lds[];  // 16-byte LDS reads of s
     __shared__ AbCtrl ac;
     __shared__ double red[256], red2[256], tau[64], pdv[64], pdt[64], pth[64];
     __shared__ int bad, take;
     __shared__ long long nstep, nsnap;
     const int R = a.R, tid = threadIdx.x;
-    const int64_t N = a.d.N, ld = a.d.ld, n = a.d.lay.n;
+    const int64_t n = a.d.lay.n;
+    const int N = (int)a.d.N;
     const int64_t p0 = (int64_t)blockIdx.x * R;
     const int Rv = (int)((N - p0) < R ? (N - p0) : R);
     const int E = 3 * R;
-    const int64_t ldp = ld + 2;  // K row pitch in LDS
-    double *Ks = lds, *sv = Ks + (size_t)R * ldp;
-    double *uo = sv + ld, *po = uo + E, *fpo = po + E, *yo = fpo + E, *fo = yo + E, *ph = fo + E;  // ph: 6E
+    double *sv = lds;
+    double *uo = sv + LD, *po = uo + E, *fpo = po + E, *yo = fpo + E, *fo = yo + E, *ph = fo + E;  // ph: 6E
     const int64_t comp_off[3] = {a.d.lay.v, a.d.lay.th, a.d.lay.del};
+    unsigned long long *xp = a.x + 4 * (int64_t)N;  // partials
 
-    for (int64_t x = tid; x < (int64_t)Rv * ld; x += 256) Ks[(x / ld) * ldp + x % ld] = a.K[p0 * ld + x];
-    for (int64_t j = tid; j < ld; j += 256) sv[j] = 0.0;
+    OwnRows<LD> K;
+    K.load(a.K, p0, Rv, tid);
+    for (int j = tid; j < LD; j += 256) sv[j] = 0.0;
     for (int e = tid; e < E; e += 256) {
         const int cpt = e / R, i = e % R;
         const int64_t gi = comp_off[cpt] + p0 + i;
@@ -796,6 +839,7 @@ __global__ void __launch_bounds__(256) k_persist_ab(PersistArgs a, AbCtrl *actrl
         for (int j = 0; j <= kAbK; ++j) ph[j * E + e] = i < Rv ? phig[j * n + gi] : 0.0;
     }
     if (tid == 0) {
+        bad = 0;
         ac = *actrl;
         nstep = a.recording ? *a.rec.nstep : 0;
         nsnap = a.recording ? *a.rec.nsnap : 0;
@@ -810,27 +854,22 @@ __global__ void __launch_bounds__(256) k_persist_ab(PersistArgs a, AbCtrl *actrl
     }
     __syncthreads();
     unsigned epoch = 0;
-    // s <- x[v] - vpl (owned), barrier, s -> LDS, owned rows of K s, rates -> out
-    // dtau-free friction terms of state x, on wavefronts 1..3 during a barrier
-    auto pre_of = [&](const double *x) {
-        return [=]() {
-            if (pr >= 0 && pr < Rv) fault_pre(a.d, fa, fb, fL, fs, x[pr], x[R + pr], pdv[pr], pdt[pr], pth[pr]);
-        };
+    // dtau-free friction terms of state x, on wavefront 1 during an exchange
+    auto pre = [&](const double *x) {
+        if (pr >= 0 && pr < Rv) fault_pre(a.d, fa, fb, fL, fs, x[pr], x[R + pr], pdv[pr], pdt[pr], pth[pr]);
     };
-    // s <- x[v] - vpl for the owned patches, into source buffer buf
+    // s = x[v] - vpl of the owned patches, into source vector buf
     auto publish = [&](const double *x, int buf) {
-        double *sg = a.s2 + buf * N;
-        for (int i = tid; i < Rv; i += 256) sg[p0 + i] = x[i] - a.d.vpl;
+        for (int i = tid; i < Rv; i += 256) x_put(a.x + 2 * (int64_t)buf * N, p0 + i, epoch, x[i] - a.d.vpl);
     };
-    // after a barrier that follows every workgroup's publish: s -> LDS, the
-    // owned rows of K s, rates -> out
-    auto consume = [&](const double *x, double *out, int buf) {
-        const double *sg = a.s2 + buf * N;
-        for (int64_t j = tid; j < N; j += 256) sv[j] = sg[j];
+    auto fetch = [&](int j0, int buf) {
+        x_get<OwnRows<LD>::U>(a, a.x + 2 * (int64_t)buf * N, j0, N, epoch, &bad, [&](int j, double v) { sv[j] = v; });
+    };
+    // with s in LDS: the owned rows of K s, rates -> out
+    auto rates = [&](const double *x, double *out) {
+        K.sweep(sv, Rv, tid, tau);
         __syncthreads();
-        lds_rows(Ks, sv, ld, ldp, Rv, tid, tau);
-        __syncthreads();
-        if (tid < Rv) {  // the dtau-free terms of x came with the preceding barrier
+        if (tid < Rv) {  // the dtau-free terms of x came with the exchange
             const int r = tid;
             out[r] = fault_dv(a.d, tau[r], pdv[r], pdt[r], pth[r]);
             out[R + r] = pth[r];
@@ -876,9 +915,13 @@ __global__ void __launch_bounds__(256) k_persist_ab(PersistArgs a, AbCtrl *actrl
             po[e] = uo[e] + h * acc;
         }
         __syncthreads();
+        ++epoch;
         publish(po, 0);
-        if (!grid_barrier(a, epoch, &bad, pre_of(po))) return;
-        consume(po, fpo, 0);
+        if ((tid >> 6) == 1) pre(po);
+        else fetch(tid < 64 ? tid : tid - 64, 0);
+        __syncthreads();
+        if (bad) return;
+        rates(po, fpo);
         double acc2 = 0.0, vm = 0.0;  // corrector, error and max |v| partials
         for (int e = tid; e < E; e += 256) {
             if (e % R >= Rv) continue;  // padding: yo stays zero
@@ -898,17 +941,23 @@ __global__ void __launch_bounds__(256) k_persist_ab(PersistArgs a, AbCtrl *actrl
             red2[tid >> 6] = vm;
         }
         __syncthreads();
-        if (tid == 0) {
-            a.part[2 * blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
-            a.part[2 * blockIdx.x + 1] = fmax(fmax(red2[0], red2[1]), fmax(red2[2], red2[3]));
-        }
-        // the corrected source vector crosses the same barrier as the error
-        // partials: an accepted step needs no third barrier (a rejected one
-        // leaves buffer 1 unread)
+        ++epoch;
+        if (tid < 2)
+            x_put(xp, 2 * blockIdx.x + tid, epoch,
+                  tid == 0 ? (red[0] + red[1]) + (red[2] + red[3])
+                           : fmax(fmax(red2[0], red2[1]), fmax(red2[2], red2[3])));
+        // the corrected source vector goes out with the error partials: an
+        // accepted step needs no third exchange (a rejected one leaves s unused)
         publish(yo, 1);
-        if (!grid_barrier(a, epoch, &bad, pre_of(yo))) return;
-        for (int w = tid; w < 2 * a.nwg; w += 256) red[w] = a.part[w];
-        __syncthreads();
+        __syncthreads();  // red is written again below
+        if (tid < 64) {
+            for (int w = tid; w < 2 * a.nwg; w += 64)
+                x_get<1>(a, xp, w, w + 1, epoch, &bad, [&](int j, double v) { red[j] = v; });
+            __builtin_amdgcn_wave_barrier();
+        } else {
+            if (tid < 128) pre(yo);
+            fetch(tid - 64, 1);
+        }
         if (tid == 0) {  // k_ab_controller, on the same sums in every workgroup
             Ctrl &c = ac.c;
             double sum = 0.0, vmax = 0.0;
@@ -947,8 +996,9 @@ __global__ void __launch_bounds__(256) k_persist_ab(PersistArgs a, AbCtrl *actrl
             }
         }
         __syncthreads();
+        if (bad) return;
         if (ac.c.accept) {
-            consume(yo, fo, 1);
+            rates(yo, fo);
             for (int e = tid; e < E; e += 256) {  // k_ab_commit
                 double tmp = fo[e];
                 for (int j = 0; j < k; ++j) {
@@ -1010,12 +1060,21 @@ struct oq_stepper {
     // persistent mode (oq_stepper_set_persistent)
     bool persistent = false;
     int p_R = 0, p_nwg = 0;
-    size_t p_lds = 0;
+    size_t p_lds = 0, p_xbytes = 0;
     long long p_wait = 0;
-    oq::DevBuf p_s2, p_part, p_bar, p_abort;
+    oq::DevBuf p_x, p_abort;
 };
 
 namespace oq {
+
+// the persistent kernel of a row length (nullptr: none)
+static const void *persist_kernel(int alg, int64_t ld)
+{
+    if (ld == 512) return alg == 1 ? (const void *)k_persist_ab<512> : (const void *)k_persist<512>;
+    if (ld == 1024) return alg == 1 ? (const void *)k_persist_ab<1024> : (const void *)k_persist<1024>;
+    if (ld == 1536) return alg == 1 ? (const void *)k_persist_ab<1536> : (const void *)k_persist<1536>;
+    return nullptr;
+}
 
 static inline unsigned nb(int64_t n) { return (unsigned)((n + 255) / 256); }
 
@@ -1252,9 +1311,7 @@ int oq_stepper_run(oq_stepper *st, int64_t max_steps, int *retcode)
         a.ctrl = st->ctrl.as<Ctrl>();
         a.u = st->u.as<double>();
         a.k1 = st->k.as<double>();
-        a.s2 = st->p_s2.as<double>();
-        a.part = st->p_part.as<double>();
-        a.bar = st->p_bar.as<unsigned>();
+        a.x = st->p_x.as<unsigned long long>();
         a.abort = st->p_abort.as<int>();
         a.rec = st->rec;
         a.recording = st->recording ? 1 : 0;
@@ -1262,17 +1319,18 @@ int oq_stepper_run(oq_stepper *st, int64_t max_steps, int *retcode)
         a.nwg = st->p_nwg;
         a.max_steps = max_steps;
         a.wait_ticks = st->p_wait;
-        OQ_HIP(hipMemsetAsync(st->p_bar.p, 0, sizeof(unsigned), h->stream));
+        OQ_HIP(hipMemsetAsync(st->p_x.p, 0, st->p_xbytes, h->stream));
+        const void *kfn = persist_kernel(st->alg, h->ld);
         if (st->alg == 1) {
             AbCtrl *actrl = st->ctrl.as<AbCtrl>();
             double *phig = st->k.as<double>();
             void *args[] = {&a, &actrl, &phig};
-            OQ_HIP(hipLaunchCooperativeKernel((const void *)k_persist_ab, dim3(st->p_nwg), dim3(256),
-                                              args, st->p_lds, h->stream));
+            OQ_HIP(hipLaunchCooperativeKernel(kfn, dim3(st->p_nwg), dim3(256), args, st->p_lds,
+                                              h->stream));
         } else {
             void *args[] = {&a};
-            OQ_HIP(hipLaunchCooperativeKernel((const void *)k_persist, dim3(st->p_nwg), dim3(256),
-                                              args, st->p_lds, h->stream));
+            OQ_HIP(hipLaunchCooperativeKernel(kfn, dim3(st->p_nwg), dim3(256), args, st->p_lds,
+                                              h->stream));
         }
         int ab = 0;
         OQ_HIP(hipMemcpyAsync(&ab, st->p_abort.p, sizeof(int), hipMemcpyDeviceToHost, h->stream));
@@ -1281,7 +1339,7 @@ int oq_stepper_run(oq_stepper *st, int64_t max_steps, int *retcode)
         OQ_HIP(hipStreamSynchronize(h->stream));
         if (ab) {
             st->persistent = false;
-            set_error("persistent stepper: a grid barrier timed out; the state is not valid");
+            set_error("persistent stepper: an exchange timed out; the state is not valid");
             return OQ_ERR_STATE;
         }
         if (retcode) *retcode = st->ctrl_host->done ? st->ctrl_host->retcode : OQ_RET_RUNNING;
@@ -1320,27 +1378,28 @@ int oq_stepper_set_persistent(oq_stepper *st, int on)
     OQ_HIP(hipDeviceGetAttribute(&maxlds, hipDeviceAttributeMaxSharedMemoryPerBlock, h->device));
     OQ_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, h->device));
     OQ_REQUIRE(coop != 0, "the device has no cooperative launch");
-    // rows of K per workgroup: as many as fit in 128 KB of LDS
+    // rows of K per workgroup: 128 KB of registers
     const int64_t rows = (int64_t)(131072 / (h->ld * 8));
     OQ_REQUIRE(rows >= 1, "the operator rows are too long for the persistent stepper (N > 16384)");
     const int R = (int)(rows < 64 ? rows : 64);
     const int nwg = (int)((h->N + R - 1) / R);
+    OQ_REQUIRE(nwg <= 128, "the persistent stepper takes at most 128 workgroups (N <= 1280)");
+    const void *kfn = persist_kernel(st->alg, h->ld);  // nwg <= 128: ld is 512, 1024 or 1536
+    OQ_REQUIRE(kfn != nullptr, "the persistent stepper has no kernel for this row length");
     // per owned entry: Tsit5 keeps u, the stage state and seven stages; VCABM5
-    // keeps u, p, f(p), y_{n+1}, f(y_{n+1}) and Phi_0..Phi_5
+    // keeps u, p, f(p), y_{n+1}, f(y_{n+1}) and Phi_0..Phi_5; s, and for Tsit5
+    // two candidate vectors
     const size_t per_entry = st->alg == 1 ? 11 : 9;
-    const size_t lds = ((size_t)R * (h->ld + 2) + h->ld + per_entry * 3 * R) * 8;  // K rows at pitch ld + 2
+    const size_t lds = ((st->alg == 1 ? 1 : 3) * h->ld + per_entry * 3 * R) * 8;
     OQ_REQUIRE((int64_t)lds <= (int64_t)maxlds, "the persistent stepper does not fit in LDS");
-    const void *kfn = st->alg == 1 ? (const void *)k_persist_ab : (const void *)k_persist;
     OQ_HIP(hipFuncSetAttribute(kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     int per_cu = 0;
     OQ_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kfn, 256, lds));
     OQ_REQUIRE(per_cu >= 1 && (int64_t)per_cu * cus >= nwg,
                "the persistent stepper needs more co-resident workgroups than the device holds");
-    OQ_REQUIRE(nwg <= 128, "the persistent stepper takes at most 128 workgroups (N <= 1024)");
-    // two source buffers and, for Tsit5, the four stage-1 candidate vectors
-    int rc = st->p_s2.alloc((size_t)(6 * h->N) * 8);
-    if (!rc) rc = st->p_part.alloc((size_t)(2 * nwg) * 8);
-    if (!rc) rc = st->p_bar.alloc(sizeof(unsigned));
+    // two source vectors, Tsit5's four candidate vectors and the partials
+    st->p_xbytes = (size_t)((st->alg == 1 ? 2 : 6) * h->N + 2 * nwg) * 16;
+    int rc = st->p_x.alloc(st->p_xbytes);
     if (!rc) rc = st->p_abort.alloc(sizeof(int));
     if (rc) return rc;
     OQ_HIP(hipMemsetAsync(st->p_abort.p, 0, sizeof(int), h->stream));
@@ -1348,7 +1407,7 @@ int oq_stepper_set_persistent(oq_stepper *st, int on)
     st->p_R = R;
     st->p_nwg = nwg;
     st->p_lds = lds;
-    // a barrier wait longer than 5 s means a workgroup is gone: abort
+    // an exchange that waits longer than 5 s means a workgroup is gone: abort
     st->p_wait = (long long)(khz > 0 ? khz : 100000) * 5000;
     st->persistent = true;
     return OQ_OK;

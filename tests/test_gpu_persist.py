@@ -1,5 +1,5 @@
 """The persistent stepper (one cooperative launch per chunk of steps, rows
-of K resident in LDS, one grid barrier per RHS) against the graph stepper:
+of K resident in registers, one exchange per RHS) against the graph stepper:
 same controller and method (Tsit5, or VCABM5 with its divided differences
 kept in LDS), so the same accepted steps and the same state up to FP64
 summation order; the recorder gives the same catalogue."""
@@ -49,6 +49,37 @@ def test_persistent_matches_graph_small(oracle, rng, dip, alg):
     k = min(len(stg), len(stp))
     assert np.allclose(stp[:k], stg[:k], rtol=1e-6)
     assert sng.shape[1] == snp.shape[1] and abs(len(sng) - len(snp)) <= 1
+
+
+@pytest.mark.parametrize("alg", ["tsit5", "vcabm5"])
+@pytest.mark.parametrize("nx,nxi", [(1, 1), (33, 1), (32, 16), (27, 19), (64, 16), (41, 25), (64, 20)])
+def test_persistent_sizes(rng, nx, nxi, alg):
+    """One patch, a last workgroup of one patch (33, 513, 1025) and the ends of
+    each row length (512, 1024, 1280), over two launches or more: the state at
+    a fixed time is the graph stepper's, as above."""
+    mf = small_fault(90.0, x=nx * 1e3, xi=nxi * 1e3, d=1e3)
+    assert (mf.nx, mf.nxi) == (nx, nxi)
+    pf = rs_props(mf, rng)
+    v = pf.vpl * np.exp(0.3 * rng.standard_normal((nx, nxi)))
+    u0 = oq.ArrayPartition(v, pf.L / v, np.zeros_like(v))
+    prob = oq.assemble_from_mesh(mf, None, 3e10, 3e10, pf, None, u0, (0.0, 1e8))
+    a = oq.VCABM5() if alg == "vcabm5" else None
+    rg, (tg, _, ug, nag, nrg), _, _ = _run(prob, False, 16, a)
+    rp, (tp, _, up, nap, nrp), _, _ = _run(prob, True, 16, a)
+    assert rg == rp == "Success" and tg == tp and nap + nrp > 16
+    assert abs(nag - nap) <= 1 and abs(nrg - nrp) <= 1
+    assert relerr(up.pack(), ug.pack()) <= 1e-8
+
+
+def test_persistent_refuses_more_than_128_workgroups(rng):
+    mf = small_fault(90.0, x=61e3, xi=21e3, d=1e3)  # 1281 patches
+    pf = rs_props(mf, rng)
+    v = np.full((mf.nx, mf.nxi), pf.vpl)
+    prob = oq.assemble_from_mesh(mf, None, 3e10, 3e10, pf, None, oq.ArrayPartition(v, pf.L / v, 0 * v), (0.0, YEAR))
+    it = oq.Integrator(prob)
+    with pytest.raises(ValueError):
+        it.set_persistent(True)
+    it.close()
 
 
 @pytest.mark.parametrize("alg", ["tsit5", "vcabm5"])
