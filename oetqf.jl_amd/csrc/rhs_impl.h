@@ -219,6 +219,8 @@ struct oq_rhs {
     oq::DevBuf s64;                     // source vector, ld doubles (zero padded)
     oq::DevBuf s32;                     // FP32 copy of s (BF16 operator)
     oq::DevBuf u, du;                   // packed state scratch for the host API
+    double *stage = nullptr;            // its pinned side, of stage_n doubles (from the first call)
+    int64_t stage_n = 0;
     oq::DevBuf tpart;                   // Toeplitz operator: per-chunk partial sums
     oq::DevBuf ftw, fg, fsh, fth;       // DFT operator: twiddles, kernel DFT, S^, T^
     // coupled model with the DFT K_ff (OQ_K_FFT, ne > 0): K holds the mantle
