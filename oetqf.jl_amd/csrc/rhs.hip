@@ -223,12 +223,50 @@ __device__ __forceinline__ void stream_rows(const typename KVec<KT>::V *const (&
     for (int r = 0; r < R; ++r) acc[r] = wave_sum(acc[r]);
 }
 
-// One wavefront streams KTraits::kRows consecutive rows.  Each wavefront
-// starts its sweep over the columns at a different pass (rotation by a
-// multiple of its index): with all wavefronts reading the same column
-// offset of rows whose pitch is a large power of two, the loads would
+// The same sums for the few rows per wavefront of a small operator: D passes
+// of K and s are in flight.
+template <int KT, int R, int D>
+__device__ __forceinline__ void stream_rows_deep(const typename KVec<KT>::V *const (&rp)[R],
+                                                 const double *__restrict__ s, int64_t npass, int64_t p0,
+                                                 int lane, double (&acc)[R])
+{
+    using V = typename KVec<KT>::V;
+    constexpr int E = KTraits<KT>::kPerLane;
+    constexpr int64_t STEP = 64 * E;
+    V kb[D][R];
+    SVec<KT> sb[D];
+    int64_t p = p0;  // next pass to load
+    auto load = [&](V (&k)[R], SVec<KT> &sv) {
+        sv = s_load<KT>(s, p * STEP + lane * E);
+#pragma unroll
+        for (int r = 0; r < R; ++r) k[r] = ld_nt(rp[r] + p * 64);
+        p = (p + 1 == npass) ? 0 : p + 1;
+    };
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] = 0.0;
+#pragma unroll
+    for (int j = 0; j < D; ++j)
+        if (j < npass) load(kb[j], sb[j]);
+    for (int64_t it = 0; it < npass; it += D) {
+#pragma unroll
+        for (int j = 0; j < D; ++j) {
+            if (it + j >= npass) break;
+#pragma unroll
+            for (int r = 0; r < R; ++r) acc[r] += dot16(kb[j][r], sb[j]);
+            if (it + j + D < npass) load(kb[j], sb[j]);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] = wave_sum(acc[r]);
+}
+
+// One wavefront streams R consecutive rows.  The wavefronts of every eight
+// rows start their sweep over the columns at a different pass (rotation by a
+// multiple of the eight rows' index): with all wavefronts reading the same
+// column offset of rows whose pitch is a large power of two, the loads would
 // concentrate on a few HBM channels (measured 4.9 vs 6.1 TB/s, FP64).
-template <int KT>
+// A row's sum has the same bits for every R.
+template <int KT, int R>
 __global__ void __launch_bounds__(KTraits<KT>::kWaves * 64)
     k_rhs_matvec(RhsDev d, const void *__restrict__ Kp, int64_t ld, int64_t nrows, int64_t rowbase,
                  const double *__restrict__ s, const double *__restrict__ tadd, int tcount,
@@ -236,7 +274,6 @@ __global__ void __launch_bounds__(KTraits<KT>::kWaves * 64)
 {
     using T = typename KTraits<KT>::T;
     constexpr int E = KTraits<KT>::kPerLane;  // elements per 16-byte load
-    constexpr int R = KTraits<KT>::kRows;
     constexpr int W = KTraits<KT>::kWaves;
     constexpr int64_t STEP = 64 * E;          // columns per wavefront pass
     const int lane = threadIdx.x & 63;
@@ -256,7 +293,9 @@ __global__ void __launch_bounds__(KTraits<KT>::kWaves * 64)
         rp[r] = reinterpret_cast<const V *>(K + row * ld) + lane;
     }
     double acc[R];
-    stream_rows<KT, R>(rp, s, ld / STEP, (gw * 13) % (ld / STEP), lane, acc);
+    const int64_t npass = ld / STEP, p0 = (row0 / 8 * 13) % npass;
+    if constexpr (R == 8) stream_rows<KT, R>(rp, s, npass, p0, lane, acc);
+    else stream_rows_deep<KT, R, R == 4 ? 4 : 8>(rp, s, npass, p0, lane, acc);
     if (lane < R) {
         double y = acc[0];
 #pragma unroll
@@ -273,14 +312,36 @@ __global__ void __launch_bounds__(KTraits<KT>::kWaves * 64)
 
 static inline unsigned nblk(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
+// Rows per wavefront.  Eight stream fastest where their blocks come in whole
+// rounds of the 256 CUs: FP64, 8192 and 16384 rows 80 and 318 us, with two
+// rows 86 and 319; BF16, 16384 rows 86 us, with two 97.  Elsewhere the last
+// round is partly empty and fewer rows are faster: FP64 10240 rows 156 -> 125
+// us, 5056 rows 43.8 -> 37.7, 2048 rows 16.3 -> 10.9; FP32 (four rows) 5056
+// rows 26.1 -> 24.1, 3104 rows 15.7 -> 13.3.  The smallest operators want a
+// wavefront per row: FP64 512 rows 8.2 -> 6.9 us (two rows: 7.2), 2048 rows
+// the same with one and two; FP32 512 and 2048 rows 7.4 and 11.1 -> 6.5 and 8.4
+// with two (6.8 and 9.3 with one).
+template <int KT>
+static int matvec_rows(int64_t nrows)
+{
+    constexpr bool f32 = KT == OQ_K_FP32;
+    const int64_t blocks = nblk(nrows, KTraits<KT>::kRows * KTraits<KT>::kWaves), rounds = (blocks + 255) / 256;
+    if (nrows > (f32 ? 8192 : 4096) && 10 * blocks >= 9 * 256 * rounds) return 8;
+    return f32 ? (nrows <= 2560 ? 2 : 4) : (nrows <= 1280 ? 1 : 2);
+}
+
 template <int KT>
 static void launch_matvec(oq_rhs *h, const void *K, int64_t ld, int64_t nrows, int64_t rowbase,
                           const double *s, const double *tadd, int tcount, int64_t tstride,
                           const double *u, double *du)
 {
-    constexpr int rows = KTraits<KT>::kRows * KTraits<KT>::kWaves;
-    hipLaunchKernelGGL(k_rhs_matvec<KT>, dim3(nblk(nrows, rows)), dim3(KTraits<KT>::kWaves * 64), 0,
-                       h->stream, h->dev, K, ld, nrows, rowbase, s, tadd, tcount, tstride, u, du);
+    static_assert(KTraits<KT>::kRows == 8, "the rotation goes by eight rows");
+    constexpr int W = KTraits<KT>::kWaves;
+    const int R = matvec_rows<KT>(nrows);
+    const dim3 grid(nblk(nrows, R * W)), block(W * 64);
+    constexpr int R1 = KT == OQ_K_FP32 ? 2 : 1, R2 = 2 * R1;  // matvec_rows' smaller answers
+    const auto k = R == 8 ? k_rhs_matvec<KT, 8> : R == R2 ? k_rhs_matvec<KT, R2> : k_rhs_matvec<KT, R1>;
+    hipLaunchKernelGGL(k, grid, block, 0, h->stream, h->dev, K, ld, nrows, rowbase, s, tadd, tcount, tstride, u, du);
 }
 
 template <int KT>
