@@ -464,7 +464,7 @@ __global__ void __launch_bounds__(256) k_fft_kernel(const double *__restrict__ s
     const int64_t nf = nx * nxi, h = L / 2, tot = (h + 1) * nxi * nxi;
     for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < tot;
          t += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t j = t % nxi, l = (t / nxi) % nxi, f = t / (nxi * nxi);
+        const int64_t f = t % (h + 1), j = t / (h + 1) % nxi, l = t / (h + 1) / nxi;  // a wavefront shares x_m
         const double *col = st + nx * j + nf * l;
         // x_0 + sum_{0<m<nx} x_m (cos(2 pi f m / L) + cos(2 pi f (L - m) / L)) = x_0 + 2 sum x_m cos
         double acc = 0.0;
@@ -475,7 +475,7 @@ __global__ void __launch_bounds__(256) k_fft_kernel(const double *__restrict__ s
             const int64_t kk = k < h ? k : L - k;  // cos(2 pi k / L) = cos(2 pi (L - k) / L)
             acc += col[m] * (k < h ? tw[kk] : (kk == h ? -1.0 : tw[kk]));
         }
-        G[t] = col[0] + 2.0 * acc;
+        G[j + nxi * (l + nxi * f)] = col[0] + 2.0 * acc;
     }
 }
 
