@@ -43,7 +43,7 @@ struct Ctrl {
     double t, t1, dt, dtcur, qold, eest;
     double reltol, abstol, dtmax, dtmin;
     long long iter, maxiters, naccept, nreject;
-    int done, retcode, accept, pad;
+    int done, retcode, accept, take;  // take: the accepted step goes to the snapshot ring
 };
 
 static constexpr int kErrBlocks = 256;
@@ -89,16 +89,121 @@ __global__ void __launch_bounds__(256) k_stage(const Ctrl *__restrict__ c, int s
     y[i] = u[i] + c->dtcur * acc;
 }
 
-// Per-block sums of the squared scaled error (deterministic order).
-__global__ void __launch_bounds__(256) k_err(const Ctrl *__restrict__ c, int64_t n,
-                                             const double *__restrict__ u,
-                                             const double *__restrict__ y,
-                                             const double *__restrict__ k,
-                                             double *__restrict__ part)
+// Recorder (the device side of wsolve, io.jl:51-66): after an accepted
+// step, the step counter advances, (t, max v) goes to a per-step ring, and
+// every `stride`-th accepted step the state goes to a snapshot ring (by the
+// commit kernels).
+struct Recorder {
+    long long *nstep, *nsnap;  // totals since the last drain
+    double *step_t, *step_vmax;
+    double *snap_t, *snap_u;
+    double *snap_du;       // derivative ring (nullptr: not recorded)
+    long long step_cap, snap_cap, stride;
+    int64_t n, nf;
+};
+
+// A double between workgroups without fences: two 64-bit words, number | half,
+// stored and polled as relaxed agent-scope atomics.
+__device__ __forceinline__ void x_put(unsigned long long *x, int64_t i, unsigned ep, double v)
 {
-    __shared__ double red[256];
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v), t = (unsigned long long)ep << 32;
+    __hip_atomic_store(x + 2 * i, t | (b & 0xffffffffull), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(x + 2 * i + 1, t | b >> 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The error kernels end in the workgroup that arrives last, which has the step
+// controller run on the sums of all: a launch of its own for the controller
+// and one for the recorder took 4.6 and 5.9 us of each step.  Every block
+// publishes its two values numbered seq + 1, then counts itself; the last one
+// reads them as they arrive (all are on their way by then) and adds them in
+// the tree order of the block sums.
+struct StepPart {
+    unsigned long long *x;  // kErrBlocks x (sum, maximum)
+    unsigned *seq, *cnt;
+};
+
+// True in the last block, in all of its threads: red[0] is the sum of acc,
+// rmx[0] the maximum of vm over the grid of kErrBlocks blocks of 256.
+__device__ __forceinline__ bool step_last_block(const StepPart &s, double acc, double vm, double *red, double *rmx,
+                                                int *last)
+{
+    const int tid = threadIdx.x;
+    auto tree = [&]() {
+        __syncthreads();
+        for (int o = 128; o > 0; o >>= 1) {
+            if (tid < o) {
+                red[tid] += red[tid + o];
+                rmx[tid] = fmax(rmx[tid], rmx[tid + o]);
+            }
+            __syncthreads();
+        }
+    };
+    red[tid] = acc;
+    rmx[tid] = vm;
+    tree();
+    const unsigned ep = *s.seq + 1;  // the last block moves it on, once all blocks have counted themselves
+    if (tid == 0) {
+        x_put(s.x, 2 * (int64_t)blockIdx.x, ep, red[0]);
+        x_put(s.x, 2 * (int64_t)blockIdx.x + 1, ep, rmx[0]);
+        *last = __hip_atomic_fetch_add(s.cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == kErrBlocks - 1;
+    }
+    __syncthreads();
+    if (!*last) return false;
+    unsigned long long w[4];
+    bool ok;
+    do {
+        ok = true;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) w[q] = __hip_atomic_load(s.x + 4 * tid + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) ok = ok && (unsigned)(w[q] >> 32) == ep;
+    } while (!ok);
+    red[tid] = __longlong_as_double((long long)(w[1] << 32 | (w[0] & 0xffffffffull)));
+    rmx[tid] = __longlong_as_double((long long)(w[3] << 32 | (w[2] & 0xffffffffull)));
+    tree();
+    if (tid == 0) {
+        *s.seq = ep;
+        *s.cnt = 0;
+    }
+    return true;
+}
+
+// An accepted step's entry in the step ring and its slot in the snapshot ring.
+__device__ __forceinline__ void record_step(Ctrl *c, const Recorder &r, double vmax)
+{
+    c->take = 0;
+    if (!r.nstep) return;
+    const long long k = *r.nstep;
+    if (r.step_cap > 0) {
+        r.step_t[k % r.step_cap] = c->t;
+        r.step_vmax[k % r.step_cap] = vmax;
+    }
+    *r.nstep = k + 1;
+    if (r.snap_cap > 0 && c->naccept % r.stride == 0) {
+        c->take = 1;
+        r.snap_t[*r.nsnap % r.snap_cap] = c->t;
+        *r.nsnap += 1;
+    }
+}
+
+// entry i of a taken snapshot: the accepted state and its derivative
+__device__ __forceinline__ void record_entry(const Recorder &r, int64_t i, double u, double du)
+{
+    const int64_t at = (*r.nsnap - 1) % r.snap_cap * r.n + i;
+    r.snap_u[at] = u;
+    if (r.snap_du) r.snap_du[at] = du;
+}
+
+// Per-block sums of the squared scaled error (deterministic order) and max
+// |v|, then PI step-size control (OrdinaryDiffEq's PIController semantics).
+__global__ void __launch_bounds__(256) k_err(Ctrl *c, int64_t n, const double *__restrict__ u,
+                                             const double *__restrict__ y, const double *__restrict__ k,
+                                             StepPart part, Recorder r)
+{
+    __shared__ double red[256], rmx[256];
+    __shared__ int last;
     if (c->done) return;
-    double acc = 0.0;
+    double acc = 0.0, vm = 0.0;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
          i += (int64_t)gridDim.x * blockDim.x) {
         double e = 0.0;
@@ -106,28 +211,9 @@ __global__ void __launch_bounds__(256) k_err(const Ctrl *__restrict__ c, int64_t
         for (int j = 0; j < 7; ++j) e += kTsBt[j] * k[j * n + i];
         const double w = c->dtcur * e / (c->abstol + fmax(fabs(u[i]), fabs(y[i])) * c->reltol);
         acc += w * w;
+        if (i < r.nf) vm = fmax(vm, fabs(y[i]));
     }
-    red[threadIdx.x] = acc;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) part[blockIdx.x] = red[0];
-}
-
-// PI step-size control (OrdinaryDiffEq's PIController semantics).
-__global__ void __launch_bounds__(256) k_controller(Ctrl *c, int64_t n, const double *part)
-{
-    __shared__ double red[256];
-    if (c->done) return;
-    red[threadIdx.x] = part[threadIdx.x];
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-        __syncthreads();
-    }
-    if (threadIdx.x != 0) return;
+    if (!step_last_block(part, acc, vm, red, rmx, &last) || threadIdx.x != 0) return;
     const double beta1 = 7.0 / 50.0, beta2 = 2.0 / 25.0, qmin = 0.2, qmax = 10.0, gamma = 0.9,
                  qoldinit = 1e-4;
     const double eest = sqrt(red[0] / (double)n);
@@ -147,6 +233,7 @@ __global__ void __launch_bounds__(256) k_controller(Ctrl *c, int64_t n, const do
         c->dt = c->dtcur / q;
         c->naccept += 1;
         c->accept = 1;
+        record_step(c, r, rmx[0]);
     } else {
         c->nreject += 1;
         if (!isfinite(eest)) {
@@ -158,66 +245,19 @@ __global__ void __launch_bounds__(256) k_controller(Ctrl *c, int64_t n, const do
     }
 }
 
-// Accepted step: u <- y, k1 <- k7 (FSAL).
+// Accepted step: u <- y, k1 <- k7 (FSAL), and the snapshot if one is taken.
 __global__ void __launch_bounds__(256) k_commit(const Ctrl *__restrict__ c, int64_t n,
                                                 double *__restrict__ u,
                                                 const double *__restrict__ y,
-                                                double *__restrict__ k)
+                                                double *__restrict__ k, Recorder r)
 {
     if (!c->accept) return;
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    u[i] = y[i];
-    k[i] = k[6 * n + i];
-}
-
-// Recorder (the device side of wsolve, io.jl:51-66): after an accepted
-// step, the step counter advances, (t, max v) goes to a per-step ring, and
-// every `stride`-th accepted step the state goes to a snapshot ring.
-struct Recorder {
-    long long *nstep, *nsnap;  // totals since the last drain
-    double *step_t, *step_vmax;
-    double *snap_t, *snap_u;
-    double *snap_du;       // derivative ring (nullptr: not recorded)
-    const double *du;      // f(u) of the accepted state (graph mode)
-    long long step_cap, snap_cap, stride, stride_count;
-    int64_t n, nf;
-};
-
-__global__ void __launch_bounds__(256) k_record(const Ctrl *__restrict__ c, Recorder r,
-                                                const double *__restrict__ u)
-{
-    __shared__ double red[256];
-    __shared__ int take;
-    if (!c->accept) return;
-    double m = 0.0;
-    for (int64_t i = threadIdx.x; i < r.nf; i += blockDim.x) m = fmax(m, fabs(u[i]));
-    red[threadIdx.x] = m;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + o]);
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        const long long k = *r.nstep;
-        if (r.step_cap > 0) {
-            r.step_t[k % r.step_cap] = c->t;
-            r.step_vmax[k % r.step_cap] = red[0];
-        }
-        *r.nstep = k + 1;
-        take = (r.snap_cap > 0) && (c->naccept % r.stride == 0);
-    }
-    __syncthreads();
-    if (!take) return;
-    const long long js = *r.nsnap % r.snap_cap;
-    for (int64_t i = threadIdx.x; i < r.n; i += blockDim.x) r.snap_u[js * r.n + i] = u[i];
-    if (r.snap_du)
-        for (int64_t i = threadIdx.x; i < r.n; i += blockDim.x) r.snap_du[js * r.n + i] = r.du[i];
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        r.snap_t[js] = c->t;
-        *r.nsnap = *r.nsnap + 1;
-    }
+    const double yi = y[i], k7 = k[6 * n + i];
+    u[i] = yi;
+    k[i] = k7;
+    if (c->take) record_entry(r, i, yi, k7);
 }
 
 // ---------------- VCABM5: variable-coefficient Adams-Bashforth-Moulton ----------------
@@ -266,95 +306,85 @@ __device__ void ab_coeffs_wave(int k, double h, const double *hist, double *g, d
     }
 }
 
-__global__ void k_ab_begin(AbCtrl *a)
+// Start of a step (the checks of k_step_begin) and the predictor.  Every block
+// finds the step's length and coefficients for itself and block 0 keeps them
+// for the step's other kernels; what they come from (t, dt, iter, k, hist) is
+// left alone until the controller, and a block that sees done already set
+// would have set it.
+__global__ void __launch_bounds__(256) k_ab_predict(AbCtrl *a, int64_t n, const double *__restrict__ u,
+                                                    const double *__restrict__ phi, double *__restrict__ p)
 {
-    Ctrl *c = &a->c;
-    c->accept = 0;
-    if (c->done) return;
-    if (!(c->t < c->t1)) {
-        c->done = 1;
-        c->retcode = OQ_RET_SUCCESS;
-        return;
+    __shared__ double g[kAbK + 1], beta[kAbK + 1], sdt;
+    __shared__ int stop;
+    const int k = a->k, tid = threadIdx.x;
+    if (tid == 0) {
+        Ctrl *c = &a->c;
+        int done = c->done, ret = -1;
+        double dt = c->dt;
+        if (!done) {
+            if (dt > c->dtmax) dt = c->dtmax;
+            if (c->t + dt > c->t1) dt = c->t1 - c->t;
+            if (!(c->t < c->t1)) ret = OQ_RET_SUCCESS;
+            else if (c->iter >= c->maxiters) ret = OQ_RET_MAXITERS;
+            else if (!(dt >= c->dtmin) || !isfinite(dt)) ret = isfinite(dt) ? OQ_RET_DTMIN : OQ_RET_NONFINITE;
+            done = ret >= 0;
+        }
+        stop = done;
+        sdt = dt;
+        if (blockIdx.x == 0) {
+            c->accept = 0;
+            if (ret >= 0) {
+                c->done = 1;
+                c->retcode = ret;
+            } else if (!done) {
+                c->dtcur = dt;
+                a->kcur = k;
+            }
+        }
     }
-    if (c->iter >= c->maxiters) {
-        c->done = 1;
-        c->retcode = OQ_RET_MAXITERS;
-        return;
+    __syncthreads();
+    if (stop) return;
+    const double dt = sdt;
+    if (tid < 64) ab_coeffs_wave(k, dt, a->hist, g, beta);
+    __syncthreads();
+    if (blockIdx.x == 0 && tid <= k) {
+        a->g[tid] = g[tid];
+        if (tid < k) a->beta[tid] = beta[tid];
     }
-    double dt = c->dt;
-    if (dt > c->dtmax) dt = c->dtmax;
-    if (c->t + dt > c->t1) dt = c->t1 - c->t;
-    if (!(dt >= c->dtmin) || !isfinite(dt)) {
-        c->done = 1;
-        c->retcode = isfinite(dt) ? OQ_RET_DTMIN : OQ_RET_NONFINITE;
-        return;
-    }
-    c->dtcur = dt;
-    c->iter += 1;
-    a->kcur = a->k;
-    ab_coeffs(a->k, dt, a->hist, a->g, a->beta);
-}
-
-__global__ void __launch_bounds__(256) k_ab_predict(const AbCtrl *__restrict__ a, int64_t n,
-                                                    const double *__restrict__ u,
-                                                    const double *__restrict__ phi,
-                                                    double *__restrict__ p)
-{
-    if (a->c.done) return;
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + tid;
     if (i >= n) return;
-    const int k = a->kcur;
     double acc = 0.0;
-    for (int j = 0; j < k; ++j) acc += a->g[j] * a->beta[j] * phi[j * n + i];
-    p[i] = u[i] + a->c.dtcur * acc;
+    for (int j = 0; j < k; ++j) acc += g[j] * beta[j] * phi[j * n + i];
+    p[i] = u[i] + dt * acc;
 }
 
-// corrector and per-block sums of the squared scaled error
-__global__ void __launch_bounds__(256) k_ab_correct(const AbCtrl *__restrict__ a, int64_t n,
-                                                    const double *__restrict__ u,
-                                                    const double *__restrict__ p,
-                                                    const double *__restrict__ fp,
-                                                    const double *__restrict__ phi,
-                                                    double *__restrict__ ynew,
-                                                    double *__restrict__ part)
+// corrector, per-block sums of the squared scaled error and max |v|, then the
+// step-size control
+__global__ void __launch_bounds__(256) k_ab_correct(AbCtrl *a, int64_t n, const double *__restrict__ u,
+                                                    const double *__restrict__ p, const double *__restrict__ fp,
+                                                    const double *__restrict__ phi, double *__restrict__ ynew,
+                                                    StepPart part, Recorder r)
 {
-    __shared__ double red[256];
-    if (a->c.done) return;
+    __shared__ double red[256], rmx[256];
+    __shared__ int last;
+    Ctrl *c = &a->c;
+    if (c->done) return;
     const int k = a->kcur;
-    const double h = a->c.dtcur, gk = a->g[k], dg = a->g[k] - a->g[k - 1];
-    double acc = 0.0;
+    const double h = c->dtcur, gk = a->g[k], dg = a->g[k] - a->g[k - 1];
+    double acc = 0.0, vm = 0.0;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
          i += (int64_t)gridDim.x * blockDim.x) {
         double ph = fp[i];
         for (int j = 0; j < k; ++j) ph -= a->beta[j] * phi[j * n + i];
         const double yn = p[i] + h * gk * ph;
         ynew[i] = yn;
-        const double w = h * dg * ph / (a->c.abstol + fmax(fabs(u[i]), fabs(yn)) * a->c.reltol);
+        const double w = h * dg * ph / (c->abstol + fmax(fabs(u[i]), fabs(yn)) * c->reltol);
         acc += w * w;
+        if (i < r.nf) vm = fmax(vm, fabs(yn));
     }
-    red[threadIdx.x] = acc;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) part[blockIdx.x] = red[0];
-}
-
-__global__ void __launch_bounds__(256) k_ab_controller(AbCtrl *a, int64_t n, const double *part)
-{
-    __shared__ double red[256];
-    Ctrl *c = &a->c;
-    if (c->done) return;
-    red[threadIdx.x] = part[threadIdx.x];
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-        __syncthreads();
-    }
-    if (threadIdx.x != 0) return;
+    if (!step_last_block(part, acc, vm, red, rmx, &last) || threadIdx.x != 0) return;
+    c->iter += 1;
     const double eest = sqrt(red[0] / (double)n);
-    const int k = a->kcur;
     const double q = (eest == 0.0) ? 0.5 : fmax(0.5, fmin(5.0, pow(eest, 1.0 / (k + 1)) / 0.9));
     c->eest = eest;
     if (eest <= 1.0) {
@@ -365,6 +395,7 @@ __global__ void __launch_bounds__(256) k_ab_controller(AbCtrl *a, int64_t n, con
         c->dt = c->dtcur / q;
         c->naccept += 1;
         c->accept = 1;
+        record_step(c, r, rmx[0]);
     } else {
         c->nreject += 1;
         if (!isfinite(eest)) {
@@ -376,25 +407,28 @@ __global__ void __launch_bounds__(256) k_ab_controller(AbCtrl *a, int64_t n, con
     }
 }
 
-// accepted step: u <- y_{n+1}; divided differences of the new derivative
+// accepted step: u <- y_{n+1}; divided differences of the new derivative; the
+// snapshot if one is taken
 __global__ void __launch_bounds__(256) k_ab_commit(const AbCtrl *__restrict__ a, int64_t n,
                                                    double *__restrict__ u,
                                                    const double *__restrict__ ynew,
                                                    const double *__restrict__ fnew,
-                                                   double *__restrict__ phi)
+                                                   double *__restrict__ phi, Recorder r)
 {
     if (!a->c.accept) return;
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const int k = a->kcur;
-    double tmp = fnew[i];
+    const double yi = ynew[i], fi = fnew[i];
+    double tmp = fi;
     for (int j = 0; j < k; ++j) {
         const double old = phi[j * n + i];
         phi[j * n + i] = tmp;
         tmp -= a->beta[j] * old;
     }
     phi[k * n + i] = tmp;
-    u[i] = ynew[i];
+    u[i] = yi;
+    if (a->c.take) record_entry(r, i, yi, fi);
 }
 
 // ---------------- persistent stepper for small fault-only problems ----------------
@@ -438,13 +472,6 @@ struct PersistArgs {
     int recording, R, nwg;
     long long max_steps, wait_ticks;
 };
-
-__device__ __forceinline__ void x_put(unsigned long long *x, int64_t i, unsigned ep, double v)
-{
-    const unsigned long long b = (unsigned long long)__double_as_longlong(v), t = (unsigned long long)ep << 32;
-    __hip_atomic_store(x + 2 * i, t | (b & 0xffffffffull), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(x + 2 * i + 1, t | b >> 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 
 // put(j, value j) for j = j0, j0 + 192, ... < n (at most U of them): waits for
 // each value's words to carry ep.
@@ -1078,6 +1105,13 @@ static const void *persist_kernel(int alg, int64_t ld)
 
 static inline unsigned nb(int64_t n) { return (unsigned)((n + 255) / 256); }
 
+static StepPart step_part(const oq_stepper *st)
+{
+    unsigned long long *x = st->part.as<unsigned long long>();
+    unsigned *q = reinterpret_cast<unsigned *>(x + 4 * kErrBlocks);
+    return {x, q, q + 1};
+}
+
 // One attempted VCABM5 step: two RHS evaluations (the second also runs on a
 // rejected step; its result is not used then).
 static int enqueue_step_ab(oq_stepper *st)
@@ -1088,16 +1122,12 @@ static int enqueue_step_ab(oq_stepper *st)
     double *u = st->u.as<double>(), *p = st->y.as<double>(), *phi = st->k.as<double>();
     double *fp = phi + 6 * n, *ynew = st->ab.as<double>(), *fnew = ynew + n;
     int rc;
-    hipLaunchKernelGGL(k_ab_begin, dim3(1), dim3(1), 0, h->stream, a);
     hipLaunchKernelGGL(k_ab_predict, dim3(nb(n)), dim3(256), 0, h->stream, a, n, u, phi, p);
     if ((rc = rhs_enqueue(h, p, fp))) return rc;
     hipLaunchKernelGGL(k_ab_correct, dim3(kErrBlocks), dim3(256), 0, h->stream, a, n, u, p, fp, phi,
-                       ynew, st->part.as<double>());
-    hipLaunchKernelGGL(k_ab_controller, dim3(1), dim3(256), 0, h->stream, a, n, st->part.as<double>());
+                       ynew, step_part(st), st->rec);
     if ((rc = rhs_enqueue(h, ynew, fnew))) return rc;
-    hipLaunchKernelGGL(k_ab_commit, dim3(nb(n)), dim3(256), 0, h->stream, a, n, u, ynew, fnew, phi);
-    if (st->recording)
-        hipLaunchKernelGGL(k_record, dim3(1), dim3(256), 0, h->stream, &a->c, st->rec, u);
+    hipLaunchKernelGGL(k_ab_commit, dim3(nb(n)), dim3(256), 0, h->stream, a, n, u, ynew, fnew, phi, st->rec);
     OQ_HIP(hipGetLastError());
     return OQ_OK;
 }
@@ -1128,12 +1158,8 @@ static int enqueue_step(oq_stepper *st)
         // more RHS on a finished state is harmless and keeps them graph-safe
         if ((rc = rhs_enqueue(h, y, k + s * n))) return rc;
     }
-    hipLaunchKernelGGL(k_err, dim3(kErrBlocks), dim3(256), 0, h->stream, c, n, u, y, k,
-                       st->part.as<double>());
-    hipLaunchKernelGGL(k_controller, dim3(1), dim3(256), 0, h->stream, c, n, st->part.as<double>());
-    hipLaunchKernelGGL(k_commit, dim3(nb(n)), dim3(256), 0, h->stream, c, n, u, y, k);
-    if (st->recording)
-        hipLaunchKernelGGL(k_record, dim3(1), dim3(256), 0, h->stream, c, st->rec, u);
+    hipLaunchKernelGGL(k_err, dim3(kErrBlocks), dim3(256), 0, h->stream, c, n, u, y, k, step_part(st), st->rec);
+    hipLaunchKernelGGL(k_commit, dim3(nb(n)), dim3(256), 0, h->stream, c, n, u, y, k, st->rec);
     OQ_HIP(hipGetLastError());
     return OQ_OK;
 }
@@ -1202,7 +1228,9 @@ static int stepper_create(oq_rhs *h, const double *u0, double t0, double t1,
     int rc = st->u.alloc((size_t)n * 8);
     if (!rc) rc = st->y.alloc((size_t)n * 8);
     if (!rc) rc = st->k.alloc((size_t)(7 * n) * 8);
-    if (!rc) rc = st->part.alloc(kErrBlocks * 8);
+    const size_t pb = (size_t)kErrBlocks * 32 + 8;  // StepPart
+    if (!rc) rc = st->part.alloc(pb);
+    if (!rc && hipMemsetAsync(st->part.p, 0, pb, h->stream) != hipSuccess) rc = OQ_ERR_HIP;
     if (!rc) rc = st->ctrl.alloc(alg == 1 ? sizeof(AbCtrl) : sizeof(Ctrl));
     if (!rc && alg == 1) rc = st->ab.alloc((size_t)(2 * n) * 8);
     if (!rc && hipHostMalloc((void **)&st->ctrl_host, sizeof(Ctrl), hipHostMallocDefault) != hipSuccess) {
@@ -1460,9 +1488,6 @@ int oq_stepper_record_du(oq_stepper *st, int64_t stride, int64_t snap_capacity,
     r.snap_t = st->rsnap_t.as<double>();
     r.snap_u = st->rsnap_u.as<double>();
     r.snap_du = du ? st->rsnap_du.as<double>() : nullptr;
-    // f(u) of the accepted state: Tsit5 keeps it in k1 (FSAL), VCABM5 in the
-    // second half of its corrector buffer
-    r.du = st->alg == 1 ? st->ab.as<double>() + st->n : st->k.as<double>();
     r.step_cap = step_capacity;
     r.snap_cap = snap_capacity;
     r.stride = stride;
