@@ -116,14 +116,16 @@ __device__ __forceinline__ void x_put(unsigned long long *x, int64_t i, unsigned
 // and one for the recorder took 4.6 and 5.9 us of each step.  Every block
 // publishes its two values numbered seq + 1, then counts itself; the last one
 // reads them as they arrive (all are on their way by then) and adds them in
-// the tree order of the block sums.
+// the tree order of the block sums.  Only blocks that have entries are launched
+// (the others' sums are zeros): their counts meet at one address, and 256 of
+// them cost more than the two launches did.
 struct StepPart {
     unsigned long long *x;  // kErrBlocks x (sum, maximum)
     unsigned *seq, *cnt;
 };
 
 // True in the last block, in all of its threads: red[0] is the sum of acc,
-// rmx[0] the maximum of vm over the grid of kErrBlocks blocks of 256.
+// rmx[0] the maximum of vm over the grid of at most kErrBlocks blocks of 256.
 __device__ __forceinline__ bool step_last_block(const StepPart &s, double acc, double vm, double *red, double *rmx,
                                                 int *last)
 {
@@ -145,21 +147,25 @@ __device__ __forceinline__ bool step_last_block(const StepPart &s, double acc, d
     if (tid == 0) {
         x_put(s.x, 2 * (int64_t)blockIdx.x, ep, red[0]);
         x_put(s.x, 2 * (int64_t)blockIdx.x + 1, ep, rmx[0]);
-        *last = __hip_atomic_fetch_add(s.cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == kErrBlocks - 1;
+        *last = __hip_atomic_fetch_add(s.cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
     }
     __syncthreads();
     if (!*last) return false;
-    unsigned long long w[4];
-    bool ok;
-    do {
-        ok = true;
+    red[tid] = rmx[tid] = 0.0;
+    if (tid < (int)gridDim.x) {
+        unsigned long long w[4];
+        bool ok;
+        do {
+            ok = true;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) w[q] = __hip_atomic_load(s.x + 4 * tid + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            for (int q = 0; q < 4; ++q)
+                w[q] = __hip_atomic_load(s.x + 4 * tid + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) ok = ok && (unsigned)(w[q] >> 32) == ep;
-    } while (!ok);
-    red[tid] = __longlong_as_double((long long)(w[1] << 32 | (w[0] & 0xffffffffull)));
-    rmx[tid] = __longlong_as_double((long long)(w[3] << 32 | (w[2] & 0xffffffffull)));
+            for (int q = 0; q < 4; ++q) ok = ok && (unsigned)(w[q] >> 32) == ep;
+        } while (!ok);
+        red[tid] = __longlong_as_double((long long)(w[1] << 32 | (w[0] & 0xffffffffull)));
+        rmx[tid] = __longlong_as_double((long long)(w[3] << 32 | (w[2] & 0xffffffffull)));
+    }
     tree();
     if (tid == 0) {
         *s.seq = ep;
@@ -205,7 +211,7 @@ __global__ void __launch_bounds__(256) k_err(Ctrl *c, int64_t n, const double *_
     if (c->done) return;
     double acc = 0.0, vm = 0.0;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x) {
+         i += (int64_t)kErrBlocks * blockDim.x) {
         double e = 0.0;
 #pragma unroll
         for (int j = 0; j < 7; ++j) e += kTsBt[j] * k[j * n + i];
@@ -373,7 +379,7 @@ __global__ void __launch_bounds__(256) k_ab_correct(AbCtrl *a, int64_t n, const 
     const double h = c->dtcur, gk = a->g[k], dg = a->g[k] - a->g[k - 1];
     double acc = 0.0, vm = 0.0;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x) {
+         i += (int64_t)kErrBlocks * blockDim.x) {
         double ph = fp[i];
         for (int j = 0; j < k; ++j) ph -= a->beta[j] * phi[j * n + i];
         const double yn = p[i] + h * gk * ph;
@@ -1105,6 +1111,8 @@ static const void *persist_kernel(int alg, int64_t ld)
 
 static inline unsigned nb(int64_t n) { return (unsigned)((n + 255) / 256); }
 
+static unsigned err_blocks(int64_t n) { return nb(n) < (unsigned)kErrBlocks ? nb(n) : (unsigned)kErrBlocks; }
+
 static StepPart step_part(const oq_stepper *st)
 {
     unsigned long long *x = st->part.as<unsigned long long>();
@@ -1124,7 +1132,7 @@ static int enqueue_step_ab(oq_stepper *st)
     int rc;
     hipLaunchKernelGGL(k_ab_predict, dim3(nb(n)), dim3(256), 0, h->stream, a, n, u, phi, p);
     if ((rc = rhs_enqueue(h, p, fp))) return rc;
-    hipLaunchKernelGGL(k_ab_correct, dim3(kErrBlocks), dim3(256), 0, h->stream, a, n, u, p, fp, phi,
+    hipLaunchKernelGGL(k_ab_correct, dim3(err_blocks(n)), dim3(256), 0, h->stream, a, n, u, p, fp, phi,
                        ynew, step_part(st), st->rec);
     if ((rc = rhs_enqueue(h, ynew, fnew))) return rc;
     hipLaunchKernelGGL(k_ab_commit, dim3(nb(n)), dim3(256), 0, h->stream, a, n, u, ynew, fnew, phi, st->rec);
@@ -1158,7 +1166,7 @@ static int enqueue_step(oq_stepper *st)
         // more RHS on a finished state is harmless and keeps them graph-safe
         if ((rc = rhs_enqueue(h, y, k + s * n))) return rc;
     }
-    hipLaunchKernelGGL(k_err, dim3(kErrBlocks), dim3(256), 0, h->stream, c, n, u, y, k, step_part(st), st->rec);
+    hipLaunchKernelGGL(k_err, dim3(err_blocks(n)), dim3(256), 0, h->stream, c, n, u, y, k, step_part(st), st->rec);
     hipLaunchKernelGGL(k_commit, dim3(nb(n)), dim3(256), 0, h->stream, c, n, u, y, k, st->rec);
     OQ_HIP(hipGetLastError());
     return OQ_OK;
