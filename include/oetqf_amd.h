@@ -74,7 +74,9 @@ extern "C" {
  * along x), K_fm and K_mf depend on a patch-cell pair's x offset only
  * through a - m jx and are held as tables of nx_f + m (nx - 1) offsets per
  * fault row and mantle line (49 MB each at the 128x32 fault with 16x16x8
- * cells instead of 403 MB); otherwise they stay dense FP64.  All FP64.
+ * cells instead of 403 MB); otherwise they stay dense FP64.  In the former
+ * case the operator is applied in the frequency domain where its transforms
+ * fit in LDS (three launches).  All FP64.
  * No counterpart in the reference (which multiplies the dense blocks,
  * equation.jl:201-203); entries equal the dense blocks' to rounding. */
 #define OQ_K_FFT_GRID 6
@@ -323,10 +325,11 @@ int oq_stepper_create_vcabm5(oq_rhs *h, const double *u0, double t0, double t1,
                              const oq_solver_opts *opts, oq_stepper **out);
 /* Persistent mode (no counterpart in the reference; the graph stepper's
  * semantics are kept): for fault-only problems with an FP64 operator whose
- * rows fit in LDS of at most 128 workgroups (N <= 1024), oq_stepper_run executes all of
- * its steps in one cooperative launch -- rows of K resident in LDS, grid
- * barriers between the RHS evaluations (Tsit5: 6 per step, the next step's
- * first stage riding on the error-norm barrier; VCABM5: 2 per step) --
+ * rows fit in the registers of at most 128 workgroups (N <= 1280),
+ * oq_stepper_run executes all of its steps in one cooperative launch -- rows
+ * of K resident in registers, exchanges of the source vector between the RHS
+ * evaluations (Tsit5: 6 per step, the next step's first stage riding on the
+ * error norm's; VCABM5: 2 per step) --
  * instead of replaying the per-step graph.  Tsit5 and VCABM5 steppers both
  * qualify.  on = 0 returns to the graph.  OQ_ERR_ARG if the problem does not
  * qualify. */

@@ -210,7 +210,9 @@ def assemble_from_mesh(mf, ma, lam, mu, pf, pa, u0, tspan, ftype=StrikeSlip(), n
     Green's functions built straight into the device operator (no host copy
     of K).  ma = None gives the fault-only problem.  kdtype "fft_grid"
     (coupled, mantle cells on a uniform horizontal grid): K_ff by DFT and
-    K_mm as 2D convolutions of its per-offset kernel; K_fm, K_mf dense."""
+    K_mm as 2D convolutions of its per-offset kernel; K_fm and K_mf along
+    strike where the spacings match (then all of it in the frequency domain),
+    dense otherwise."""
     if kdtype not in _KDTYPES_MESH:
         raise ValueError("kdtype must be one of %s" % sorted(_KDTYPES_MESH))
     keep = _Keep()
@@ -291,7 +293,7 @@ class Integrator:
 
     def set_persistent(self, on=True):
         """Runs whole chunks of steps in one cooperative launch (fault-only
-        problems whose operator rows fit in LDS); ValueError otherwise."""
+        problems of at most 1280 patches); ValueError otherwise."""
         _lib.check(_lib.load().oq_stepper_set_persistent(self.s, 1 if on else 0))
 
     def record(self, stride=1, snap_capacity=0, step_capacity=4096, derivative=False):

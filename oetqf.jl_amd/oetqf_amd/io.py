@@ -132,7 +132,7 @@ def wsolve(prob, alg, file, nstep, getu, ustrs, tstr, stride=1, append=False, fo
     at t0).  Returns the final ODESolution, or None when the file exists and
     neither force nor append is set (io.jl:119-123).  persistent=True runs
     the stepper in one cooperative launch per drain (fault-only problems
-    whose operator rows fit in LDS; Integrator.set_persistent)."""
+    of at most 1280 patches; Integrator.set_persistent)."""
     from .equation import Tsit5, VCABM5
 
     if not isinstance(alg, (Tsit5, VCABM5)):
