@@ -1918,6 +1918,41 @@ static bool off_lattice(double x, double h, double ext)
     return fabs(r - nearbyint(r)) > 1e-6;
 }
 
+// Which tables the meshes carry exactly, that is with shifts no larger than
+// the rounding of the coordinates themselves: every position within 16 ulp of
+// the largest horizontal coordinate of its place on the lattice (generated and
+// gmsh boxes: 5), the m fault spacings' mismatch summed over the columns
+// included, and heights and depths equal bit for bit (in a layer for K_mm, and
+// along a line for K_fm and K_mf too), since faces often pass through patch
+// centres there.  The grid operator, which a caller asks for, takes meshes to
+// mm_grid_detect's and mm_strike_detect's tolerances; from a mantle of 80 km
+// whose spacing misses by the 1e-9 they allow, near entries are off by 2e-8.
+static void exact_tables(const oq_fault_mesh *mf, const oq_hex8_mesh *ma, const MmGrid &g, double hx, double hy,
+                         bool &strike, bool &mm)
+{
+    const int64_t nx = mf->nx, nxy = g.nx * g.ny;
+    const double dxf = nx > 1 ? (mf->x[nx - 1] - mf->x[0]) / (double)(nx - 1) : mf->dx;
+    double big = 0.0;
+    for (int64_t c = 0; c < ma->ne; ++c) big = fmax(big, fmax(fabs(ma->cx[c]), fabs(ma->cy[c])));
+    for (int64_t a = 0; a < 2 * nx; ++a) big = fmax(big, fabs(mf->ax[a]));
+    const double tol = 16.0 * (nextafter(big, INFINITY) - big);
+    const auto near = [tol](double x, double y) { return fabs(x - y) <= tol; };
+    for (int64_t c = 0; c < ma->ne; ++c) {
+        const int64_t ix = c % g.nx, iy = (c / g.nx) % g.ny, b = c / nxy * nxy, l = c - ix;
+        mm = mm && near(ma->cx[c], ma->cx[0] + (double)ix * hx) && near(ma->cy[c], ma->cy[0] + (double)iy * hy) &&
+             near(ma->qx[c] - ma->cx[c], ma->qx[0] - ma->cx[0]) && near(ma->qy[c] - ma->cy[c], ma->qy[0] - ma->cy[0]) &&
+             near(ma->dx[c], ma->dx[0]) && near(ma->dy[c], ma->dy[0]) && ma->cz[c] == ma->cz[b] &&
+             ma->qz[c] == ma->qz[b] && ma->dz[c] == ma->dz[b];
+        strike = strike && ma->cy[c] == ma->cy[l] && ma->qy[c] == ma->qy[l] && ma->dy[c] == ma->dy[l];
+    }
+    for (int64_t a = 0; a < nx; ++a) {
+        const double sh = (double)a * dxf;
+        strike = strike && near(mf->x[a], mf->x[0] + sh) && near(mf->ax[2 * a], mf->ax[0] + sh) &&
+                 near(mf->ax[2 * a + 1], mf->ax[1] + sh);
+    }
+    strike = strike && mm && near((double)(g.nx - 1) * hx, (double)((g.nx - 1) * g.m) * dxf);
+}
+
 // The mantle blocks of the dense operator, K_fm (nf x 6ne, pitch ldf), K_mf
 // (6ne x nf, pitch ldm) and K_mm (6ne x 6ne, pitch ldm), from the meshes.
 // A pair's entries depend on its horizontal offset only (the free surface is
@@ -1928,7 +1963,8 @@ static bool off_lattice(double x, double h, double ext)
 // instead of nx_f nx.  Those are evaluated and written out to the dense rows
 // (4096 patches + 16 x 16 x 8 cells: 48 ms of pairs become 4.3 ms and 0.8 ms
 // of expansion; the entries equal those of the pair kernels over all pairs to
-// rounding, 1e-12).  Taken where it halves the pairs at least, and where no
+// the coordinates' rounding, 1e-12 of the largest).  Taken where it halves the
+// pairs at least, where the meshes carry it (exact_tables), and where no
 // receiver sits on a line or face across which the stress jumps or is
 // singular and that a shift by rounding could move it over: along x and y,
 // receivers off the cells' faces, and cells' receivers off the patches' edges
@@ -1941,9 +1977,10 @@ static int dense_blocks(const oq_fault_mesh *mf, const oq_hex8_mesh *ma, const F
     MmGrid g;
     double hx = 0.0, hy = 0.0;
     const bool grid = mm_grid_detect(ma, g, hx, hy) == nullptr;
-    const bool strike = grid && mm_strike_detect(mf, g, hx) && 2 * g.D <= nx * g.nx;
+    bool strike = grid && mm_strike_detect(mf, g, hx) && 2 * g.D <= nx * g.nx, uniform = grid;
+    if (grid) exact_tables(mf, ma, g, hx, hy, strike, uniform);
     const double X = ma->cx[0], Y = ma->cy[0], T = ma->dx[0], ext = fmax(fabs(T), fabs(ma->dy[0]));
-    bool tfm = strike, tmf = strike, tmm = grid && g.nx * g.ny >= 8;
+    bool tfm = strike, tmf = strike, tmm = uniform && g.nx * g.ny >= 8;
     const double dxf = nx > 1 ? (mf->x[nx - 1] - mf->x[0]) / (double)(nx - 1) : mf->dx;
     for (int e = -1; e <= 1; e += 2)  // patch centres and the cells' x faces
         tfm = tfm && off_lattice(mf->x[0] - (ma->qx[0] + e * T / 2.0), dxf, ext);
