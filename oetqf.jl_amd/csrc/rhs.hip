@@ -312,21 +312,35 @@ __global__ void __launch_bounds__(KTraits<KT>::kWaves * 64)
 
 static inline unsigned nblk(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
-// Rows per wavefront.  Eight stream fastest where their blocks come in whole
-// rounds of the 256 CUs: FP64, 8192 and 16384 rows 80 and 318 us, with two
-// rows 86 and 319; BF16, 16384 rows 86 us, with two 97.  Elsewhere the last
-// round is partly empty and fewer rows are faster: FP64 10240 rows 156 -> 125
-// us, 5056 rows 43.8 -> 37.7, 2048 rows 16.3 -> 10.9; FP32 (four rows) 5056
-// rows 26.1 -> 24.1, 3104 rows 15.7 -> 13.3.  The smallest operators want a
-// wavefront per row: FP64 512 rows 8.2 -> 6.9 us (two rows: 7.2), 2048 rows
-// the same with one and two; FP32 512 and 2048 rows 7.4 and 11.1 -> 6.5 and 8.4
-// with two (6.8 and 9.3 with one).
+// Rows per wavefront.  Eight stream fastest where their blocks nearly fill
+// whole rounds of the 256 CUs; where the last round is mostly empty fewer rows
+// are faster.  Measured with eight and with two (FP32: four), us:
+//   rows (blocks)   FP64         FP32         BF16
+//    6080 (190)     46.5  45.7   26.2  25.5   16.5  15.4
+//    6400 (200)     52.3  59.1   29.2  31.0   17.5  18.8
+//    7680 (240)     71.0  72.6   38.1  39.1   21.1  22.3
+//    8200 (257)     90.0  93.9   48.8  52.0   25.4  27.5
+//    8320 (260)    122    95.4   55.5  54.0   35.7  28.3
+//   10240 (320)    156   123     67.7  65.7   43.2  35.6
+//   10560 (330)    158   143     71.3  76.1   44.9  41.3
+//   12480 (390)    199   200    108   106     55.8  55.6
+//   14400 (450)    248   264    131   137     70.1  72.3
+//   18000 (563)    448   385    211   211    116   107
+//   20000 (625)    506   482    243   245    142   139
+//   22000 (688)    567   565    303   309    156   162
+//   28000 (875)    955   919    487   496    259   265
+// So eight from the part of the rounds that is filled: 77 % of up to two (FP32
+// 64 % of two), 85 % (BF16) or 88 % of more (FP32 any); one block past a round
+// counts as none.  The smallest operators want a wavefront per row: FP64 512
+// rows 8.2 -> 6.9 us (two rows: 7.2), 2048 rows the same with one and two; FP32
+// 512 and 2048 rows 7.4 and 11.1 -> 6.5 and 8.4 with two (6.8 and 9.3 with one).
 template <int KT>
 static int matvec_rows(int64_t nrows)
 {
     constexpr bool f32 = KT == OQ_K_FP32;
-    const int64_t blocks = nblk(nrows, KTraits<KT>::kRows * KTraits<KT>::kWaves), rounds = (blocks + 255) / 256;
-    if (nrows > (f32 ? 8192 : 4096) && 10 * blocks >= 9 * 256 * rounds) return 8;
+    const int64_t blocks = nblk(nrows, KTraits<KT>::kRows * KTraits<KT>::kWaves), rounds = (blocks + 254) / 256;
+    const int64_t part = rounds <= 2 ? (f32 && rounds == 2 ? 64 : 77) : (f32 ? 0 : KT == OQ_K_BF16 ? 85 : 88);
+    if (nrows > 4096 && 100 * blocks >= part * 256 * rounds) return 8;
     return f32 ? (nrows <= 2560 ? 2 : 4) : (nrows <= 1280 ? 1 : 2);
 }
 

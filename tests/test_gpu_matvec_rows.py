@@ -12,7 +12,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("nx,nxi", [(1, 1), (5, 3), (40, 32), (61, 21), (64, 40), (197, 13), (87, 89), (128, 64),
-                                    (257, 32), (211, 58)])
+                                    (257, 32), (211, 58), (197, 32), (199, 32), (205, 40), (260, 32), (330, 32),
+                                    (395, 32)])
 def test_rows_per_wavefront(rng, nx, nxi):
     mf = small_fault(90.0, x=nx * 1e3, xi=nxi * 1e3, d=1e3)
     assert (mf.nx, mf.nxi) == (nx, nxi)
