@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "adams.h"
+#include "exchange.h"
 #include "rhs_impl.h"
 
 namespace oq {
@@ -103,12 +104,17 @@ struct Recorder {
 };
 
 // A double between workgroups without fences: two 64-bit words, number | half,
-// stored and polled as relaxed agent-scope atomics.
+// stored and polled as relaxed agent-scope atomics (exchange.h).
 __device__ __forceinline__ void x_put(unsigned long long *x, int64_t i, unsigned ep, double v)
 {
-    const unsigned long long b = (unsigned long long)__double_as_longlong(v), t = (unsigned long long)ep << 32;
-    __hip_atomic_store(x + 2 * i, t | (b & 0xffffffffull), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(x + 2 * i + 1, t | b >> 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    __hip_atomic_store(x + 2 * i, x_word(ep, (unsigned)b), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(x + 2 * i + 1, x_word(ep, (unsigned)(b >> 32)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ __forceinline__ double x_double(unsigned long long lo, unsigned long long hi)
+{
+    return __longlong_as_double((long long)(hi << 32 | (lo & 0xffffffffull)));
 }
 
 // The error kernels end in the workgroup that arrives last, which has the step
@@ -118,14 +124,20 @@ __device__ __forceinline__ void x_put(unsigned long long *x, int64_t i, unsigned
 // reads them as they arrive (all are on their way by then) and adds them in
 // the tree order of the block sums.  Only blocks that have entries are launched
 // (the others' sums are zeros): their counts meet at one address, and 256 of
-// them cost more than the two launches did.
+// them cost more than the two launches did.  The wait is bounded as the
+// persistent steppers' are: were a value not to arrive, the step would end the
+// run with kRetLost, and oq_stepper_run with an error.
 struct StepPart {
     unsigned long long *x;  // kErrBlocks x (sum, maximum)
     unsigned *seq, *cnt;
+    long long wait;         // clock ticks
 };
 
+static constexpr int kRetLost = -1;  // Ctrl::retcode: an exchange timed out (not one of OQ_RET_*)
+
 // True in the last block, in all of its threads: red[0] is the sum of acc,
-// rmx[0] the maximum of vm over the grid of at most kErrBlocks blocks of 256.
+// rmx[0] the maximum of vm over the grid of at most kErrBlocks blocks of 256,
+// unless *last < 0: a value did not arrive.
 __device__ __forceinline__ bool step_last_block(const StepPart &s, double acc, double vm, double *red, double *rmx,
                                                 int *last)
 {
@@ -154,17 +166,13 @@ __device__ __forceinline__ bool step_last_block(const StepPart &s, double acc, d
     red[tid] = rmx[tid] = 0.0;
     if (tid < (int)gridDim.x) {
         unsigned long long w[4];
-        bool ok;
-        do {
-            ok = true;
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-                w[q] = __hip_atomic_load(s.x + 4 * tid + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) ok = ok && (unsigned)(w[q] >> 32) == ep;
-        } while (!ok);
-        red[tid] = __longlong_as_double((long long)(w[1] << 32 | (w[0] & 0xffffffffull)));
-        rmx[tid] = __longlong_as_double((long long)(w[3] << 32 | (w[2] & 0xffffffffull)));
+        const bool ok = x_poll(
+            w, ep, s.wait,
+            [&](int q) { return __hip_atomic_load(s.x + 4 * tid + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); },
+            [] { return (long long)wall_clock64(); });
+        red[tid] = x_double(w[0], w[1]);
+        rmx[tid] = x_double(w[2], w[3]);
+        if (!ok) *last = -1;
     }
     tree();
     if (tid == 0) {
@@ -220,6 +228,11 @@ __global__ void __launch_bounds__(256) k_err(Ctrl *c, int64_t n, const double *_
         if (i < r.nf) vm = fmax(vm, fabs(y[i]));
     }
     if (!step_last_block(part, acc, vm, red, rmx, &last) || threadIdx.x != 0) return;
+    if (last < 0) {
+        c->done = 1;
+        c->retcode = kRetLost;
+        return;
+    }
     const double beta1 = 7.0 / 50.0, beta2 = 2.0 / 25.0, qmin = 0.2, qmax = 10.0, gamma = 0.9,
                  qoldinit = 1e-4;
     const double eest = sqrt(red[0] / (double)n);
@@ -389,6 +402,11 @@ __global__ void __launch_bounds__(256) k_ab_correct(AbCtrl *a, int64_t n, const 
         if (i < r.nf) vm = fmax(vm, fabs(yn));
     }
     if (!step_last_block(part, acc, vm, red, rmx, &last) || threadIdx.x != 0) return;
+    if (last < 0) {
+        c->done = 1;
+        c->retcode = kRetLost;
+        return;
+    }
     c->iter += 1;
     const double eest = sqrt(red[0] / (double)n);
     const double q = (eest == 0.0) ? 0.5 : fmax(0.5, fmin(5.0, pow(eest, 1.0 / (k + 1)) / 0.9));
@@ -514,7 +532,7 @@ __device__ __forceinline__ void x_get(const PersistArgs &a, const unsigned long 
 #pragma unroll
     for (int u = 0; u < U; ++u)
         if (j0 + 192 * u < n)
-            put(j0 + 192 * u, __longlong_as_double((long long)(w[u][1] << 32 | (w[u][0] & 0xffffffffull))));
+            put(j0 + 192 * u, x_double(w[u][0], w[u][1]));
 }
 
 // The owned rows of K, in registers: sixteen lanes share the rows r = tid / 16
@@ -1080,6 +1098,7 @@ struct oq_stepper {
     oq_rhs *h = nullptr;
     int64_t n = 0;
     oq::DevBuf u, y, k, part, ctrl;
+    long long wait = 0;  // clock ticks an exchange may take
     oq::Ctrl *ctrl_host = nullptr;  // pinned
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -1094,7 +1113,6 @@ struct oq_stepper {
     bool persistent = false;
     int p_R = 0, p_nwg = 0;
     size_t p_lds = 0, p_xbytes = 0;
-    long long p_wait = 0;
     oq::DevBuf p_x, p_abort;
 };
 
@@ -1111,13 +1129,18 @@ static const void *persist_kernel(int alg, int64_t ld)
 
 static inline unsigned nb(int64_t n) { return (unsigned)((n + 255) / 256); }
 
+// an exchange that waits longer than 5 s means that a workgroup is gone
+static long long wait_ticks(int khz) { return (long long)(khz > 0 ? khz : 100000) * 5000; }
+
 static unsigned err_blocks(int64_t n) { return nb(n) < (unsigned)kErrBlocks ? nb(n) : (unsigned)kErrBlocks; }
+
+static constexpr size_t kPartBytes = (size_t)kErrBlocks * 32 + 8;  // StepPart's words, seq and cnt
 
 static StepPart step_part(const oq_stepper *st)
 {
     unsigned long long *x = st->part.as<unsigned long long>();
     unsigned *q = reinterpret_cast<unsigned *>(x + 4 * kErrBlocks);
-    return {x, q, q + 1};
+    return {x, q, q + 1, st->wait};
 }
 
 // One attempted VCABM5 step: two RHS evaluations (the second also runs on a
@@ -1177,6 +1200,7 @@ static int capture_step(oq_stepper *st)
     oq_rhs *h = st->h;
     if (st->exec) { (void)hipGraphExecDestroy(st->exec); st->exec = nullptr; }
     if (st->graph) { (void)hipGraphDestroy(st->graph); st->graph = nullptr; }
+    OQ_HIP(hipMemsetAsync(st->part.p, 0, kPartBytes, h->stream));  // words, seq and cnt in step again
     OQ_HIP(hipStreamSynchronize(h->stream));
     OQ_HIP(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
     int rc = enqueue_step(st);
@@ -1236,9 +1260,10 @@ static int stepper_create(oq_rhs *h, const double *u0, double t0, double t1,
     int rc = st->u.alloc((size_t)n * 8);
     if (!rc) rc = st->y.alloc((size_t)n * 8);
     if (!rc) rc = st->k.alloc((size_t)(7 * n) * 8);
-    const size_t pb = (size_t)kErrBlocks * 32 + 8;  // StepPart
-    if (!rc) rc = st->part.alloc(pb);
-    if (!rc && hipMemsetAsync(st->part.p, 0, pb, h->stream) != hipSuccess) rc = OQ_ERR_HIP;
+    if (!rc) rc = st->part.alloc(kPartBytes);
+    int khz = 0;
+    if (!rc && hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, h->device) != hipSuccess) rc = OQ_ERR_HIP;
+    st->wait = wait_ticks(khz);
     if (!rc) rc = st->ctrl.alloc(alg == 1 ? sizeof(AbCtrl) : sizeof(Ctrl));
     if (!rc && alg == 1) rc = st->ab.alloc((size_t)(2 * n) * 8);
     if (!rc && hipHostMalloc((void **)&st->ctrl_host, sizeof(Ctrl), hipHostMallocDefault) != hipSuccess) {
@@ -1354,7 +1379,7 @@ int oq_stepper_run(oq_stepper *st, int64_t max_steps, int *retcode)
         a.R = st->p_R;
         a.nwg = st->p_nwg;
         a.max_steps = max_steps;
-        a.wait_ticks = st->p_wait;
+        a.wait_ticks = st->wait;
         OQ_HIP(hipMemsetAsync(st->p_x.p, 0, st->p_xbytes, h->stream));
         const void *kfn = persist_kernel(st->alg, h->ld);
         if (st->alg == 1) {
@@ -1392,6 +1417,10 @@ int oq_stepper_run(oq_stepper *st, int64_t max_steps, int *retcode)
         OQ_HIP(hipStreamSynchronize(h->stream));
         if (st->ctrl_host->done) break;
     }
+    if (st->ctrl_host->done && st->ctrl_host->retcode == kRetLost) {
+        set_error("stepper: the exchange of a step's error sums timed out; the state is not valid");
+        return OQ_ERR_STATE;
+    }
     if (retcode) *retcode = st->ctrl_host->done ? st->ctrl_host->retcode : OQ_RET_RUNNING;
     return OQ_OK;
 }
@@ -1408,11 +1437,10 @@ int oq_stepper_set_persistent(oq_stepper *st, int on)
     OQ_REQUIRE(h->ne == 0 && !h->dev.dila,
                "the persistent stepper takes fault-only problems without dilatancy");
     OQ_REQUIRE(h->kdtype == OQ_K_FP64, "the persistent stepper takes an FP64 operator");
-    int coop = 0, cus = 0, maxlds = 0, khz = 0;
+    int coop = 0, cus = 0, maxlds = 0;
     OQ_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, h->device));
     OQ_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device));
     OQ_HIP(hipDeviceGetAttribute(&maxlds, hipDeviceAttributeMaxSharedMemoryPerBlock, h->device));
-    OQ_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, h->device));
     OQ_REQUIRE(coop != 0, "the device has no cooperative launch");
     // rows of K per workgroup: 128 KB of registers
     const int64_t rows = (int64_t)(131072 / (h->ld * 8));
@@ -1443,8 +1471,6 @@ int oq_stepper_set_persistent(oq_stepper *st, int on)
     st->p_R = R;
     st->p_nwg = nwg;
     st->p_lds = lds;
-    // an exchange that waits longer than 5 s means a workgroup is gone: abort
-    st->p_wait = (long long)(khz > 0 ? khz : 100000) * 5000;
     st->persistent = true;
     return OQ_OK;
 }

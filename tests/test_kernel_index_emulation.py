@@ -18,6 +18,7 @@ EMUL = os.path.join(os.path.dirname(os.path.abspath(__file__)), "emul")
 
 @pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
 @pytest.mark.parametrize("name,flags", [("grid_emul", ["-fopenmp"]), ("strike_emul", []),
+                                        ("exchange_emul", []),
                                         ("spectral_emul", ["-g", "-fsanitize=address,undefined", "-fno-sanitize-recover=all"])])
 def test_kernel_index_emulation(tmp_path, name, flags):
     exe = str(tmp_path / name)
