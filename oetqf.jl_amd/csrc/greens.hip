@@ -44,6 +44,12 @@ bool teardown_sync(hipStream_t s)
     return true;
 }
 
+int allow_lds(const void *kernel)
+{
+    OQ_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsMax));
+    return OQ_OK;
+}
+
 static double sin_deg_small(double r) { return sin(r * (M_PI / 180.0)); }
 static double cos_deg_small(double r) { return cos(r * (M_PI / 180.0)); }
 
@@ -748,9 +754,10 @@ int launch_toeplitz_dft(const double *st, int64_t nx, int64_t nxi, double *out, 
 {
     OQ_REQUIRE(nx <= kMaxDftNx, "the device DFT of the Toeplitz kernel takes nx <= 5120");
     const size_t lds = (size_t)(2 * nx) * 8;
-    if (lds > 64 * 1024)
-        OQ_HIP(hipFuncSetAttribute((const void *)k_toeplitz_dft,
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    if (lds > 64 * 1024) {
+        const int rc = allow_lds((const void *)k_toeplitz_dft);
+        if (rc) return rc;
+    }
     hipLaunchKernelGGL(k_toeplitz_dft, dim3((unsigned)(nxi * nxi)), dim3(kDftThreads), lds, s, st, nx, out);
     OQ_HIP(hipGetLastError());
     return OQ_OK;
@@ -760,9 +767,10 @@ int launch_toeplitz_idft(const double *dft, int64_t nx, int64_t nxi, double *st,
 {
     OQ_REQUIRE(nx <= kMaxDftNx, "the device DFT of the Toeplitz kernel takes nx <= 5120");
     const size_t lds = (size_t)(4 * nx) * 8;
-    if (lds > 64 * 1024)
-        OQ_HIP(hipFuncSetAttribute((const void *)k_toeplitz_idft,
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    if (lds > 64 * 1024) {
+        const int rc = allow_lds((const void *)k_toeplitz_idft);
+        if (rc) return rc;
+    }
     hipLaunchKernelGGL(k_toeplitz_idft, dim3((unsigned)(nxi * nxi)), dim3(kDftThreads), lds, s, dft, nx, st);
     OQ_HIP(hipGetLastError());
     return OQ_OK;

@@ -35,6 +35,13 @@ bool teardown_sync(hipStream_t s);
         }                                    \
     } while (0)
 
+// Allows a kernel the largest dynamic LDS of a workgroup.  The limit belongs to
+// the function, for every handle of the process, so all models set this one
+// value: with a model's own size a smaller one would lower it below what a
+// larger one's next launch asks for.
+static constexpr int64_t kLdsMax = 160 * 1024;
+int allow_lds(const void *kernel);
+
 // Degree trigonometry with exact zeros at multiples of 90 degrees
 // (Julia's sind/cosd, used by the reference at mesh.jl:48, GF.jl:79,86).
 double sind(double deg);

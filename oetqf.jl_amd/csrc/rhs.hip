@@ -1291,13 +1291,15 @@ static void grid_launch_r(const oq_rhs *h, const GridMv &a, const GridSt &g2)
 }
 
 template <int R>
-static int grid_lds_attrs(size_t lds)
+static int grid_lds_attrs()
 {
     const void *f[5] = {(const void *)k_grid_fused<R, 1 | 4 | 8>, (const void *)k_grid_fused<R, 1 | 2>,
                         (const void *)k_grid_fused<R, 1>, (const void *)k_grid_fused<R, 4 | 8>,
                         (const void *)k_grid_fused<R, 2>};
-    for (const void *p : f) OQ_HIP(hipFuncSetAttribute(p, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    return OQ_OK;
+    int rc = OQ_OK;
+    for (const void *p : f)
+        if (!rc) rc = allow_lds(p);
+    return rc;
 }
 
 int rhs_enqueue_matvec(oq_rhs *h, const double *u, double *du)
@@ -1578,12 +1580,9 @@ static int fft_setup(oq_rhs *h, const double *st)
     hipLaunchKernelGGL(k_fft_kernel, dim3(grid_capped((hl + 1) * nxi * nxi, 256)), dim3(256), 0, h->stream,
                        st, nx, nxi, L, h->ftw.as<double>(), h->fg.as<double>());
     OQ_HIP(hipGetLastError());
-    OQ_HIP(hipFuncSetAttribute((const void *)k_fft_fwd, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)fft_lds(nx)));
-    OQ_HIP(hipFuncSetAttribute((const void *)k_fft_inv, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)fft_lds(nx)));
-    OQ_HIP(hipFuncSetAttribute((const void *)k_fft_fwd_stage, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)(fft_lds(nx) + (size_t)nx * 8)));
+    const void *k[3] = {(const void *)k_fft_fwd, (const void *)k_fft_inv, (const void *)k_fft_fwd_stage};
+    for (const void *f : k)
+        if ((rc = allow_lds(f))) return rc;
     OQ_HIP(hipStreamSynchronize(h->stream));
     return OQ_OK;
 }
@@ -1643,7 +1642,7 @@ static int mm_grid_shape(MmGrid &g)
     g.nxp = grid_nxp(g.nx, g.r);
     const int64_t Wy = 2 * g.ny - 1, Wp = 2 * g.nxp + 1, nxg = g.nxp / g.r;
     const int64_t U = g.ny * nxg, per = Wy * Wp + 2 * g.ny * g.nxp;
-    OQ_REQUIRE(per * 8 <= 160 * 1024,
+    OQ_REQUIRE(per * 8 <= kLdsMax,
                "OQ_K_FFT_GRID: one source plane of the grid kernel exceeds the LDS of a workgroup "
                "(at most about 60 x 60 cells per layer)");
     int64_t tp = 256 / U;
@@ -1654,8 +1653,7 @@ static int mm_grid_shape(MmGrid &g)
     g.nchunk = (int)((6 * g.nz + tp - 1) / tp);
     g.threads = 256;
     g.lds = (size_t)(tp * per * 8);
-    const size_t lmax = g.lds > kGridOtherLds ? g.lds : kGridOtherLds;
-    return g.r == 8 ? grid_lds_attrs<8>(lmax) : grid_lds_attrs<4>(lmax);
+    return g.r == 8 ? grid_lds_attrs<8>() : grid_lds_attrs<4>();
 }
 
 // Along strike: the fault's centres x[a] and extents ax[a] on one spacing
@@ -2078,9 +2076,7 @@ static int gsp_build(oq_rhs *h)
     hipLaunchKernelGGL(k_gsp_tab_my, dim3(grid_capped(np2 * PH, 256)), dim3(256), 0, h->stream, g, X.as<double2>(),
                        h->spM.as<double2>());
     OQ_HIP(hipGetLastError());
-    const int lds = (int)(gsp_lds(g) * 8);
-    OQ_HIP(hipFuncSetAttribute((const void *)k_gsp_fwd, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-    OQ_HIP(hipFuncSetAttribute((const void *)k_gsp_inv, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    if ((rc = allow_lds((const void *)k_gsp_fwd)) || (rc = allow_lds((const void *)k_gsp_inv))) return rc;
     OQ_HIP(hipStreamSynchronize(h->stream));
     h->spectral = true;
     return OQ_OK;
@@ -2263,7 +2259,7 @@ static int create_from_mesh(int device, const oq_fault_mesh *mf, const oq_hex8_m
             rc = mm_grid_build(ma, h->grid, h->grid.nxp, hx, hy, qu, lambda, mu, h->Tmm, h->stream);
             const MmGrid &gg = h->grid;
             if (!rc && gg.strike && gg.D * 8 <= 64 * 1024 &&
-                gsp_shape(h->spec, mf->nx, mf->nxi, gg.m, gg.nx, gg.ny, gg.nz, kGspM, 160 * 1024)) {
+                gsp_shape(h->spec, mf->nx, mf->nxi, gg.m, gg.nx, gg.ny, gg.nz, kGspM, kLdsMax)) {
                 rc = gsp_build(h);
             } else {
                 if (!rc) rc = mm_grid_parts(h);
