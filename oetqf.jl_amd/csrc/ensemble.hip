@@ -1153,7 +1153,6 @@ struct oq_ensemble {
     oq::EnsH3 h3{};
     oq::DevBuf a, b, L, sigma, eta, vpl, f0, v0, S;
     oq::DevBuf u, y, k, part;
-    oq::DevBuf xfer;  // oq_ensemble_eval: states in the host's layout
     oq::DevBuf ct, cdt, cdtcur, cqold, cna, cnr, citer, cdone, cacc, cret;
     oq::DevBuf vpart, rec_t, rec_v;  // recorder (oq_ensemble_record)
     oq::DevBuf live;                 // EnsDev::live
@@ -1470,16 +1469,15 @@ int oq_ensemble_eval(oq_ensemble *e, const double *u, double *du)
     oq_rhs *h = e->h;
     OQ_HIP(hipSetDevice(h->device));
     const int64_t nM = e->n * e->M;
-    int rc = e->xfer.p ? OQ_OK : e->xfer.alloc((size_t)nM * 8);
-    if (rc) return rc;
-    double *x = e->xfer.as<double>(), *y = e->y.as<double>(), *k = e->k.as<double>();
-    OQ_HIP(hipMemcpyAsync(x, u, (size_t)nM * 8, hipMemcpyHostToDevice, h->stream));
-    rc = launch_transpose(x, e->M, e->n, y, h->stream);
+    // through y and the last stage, both scratch between steps: a run goes on as if there had been no eval
+    double *y = e->y.as<double>(), *k = e->k.as<double>() + 6 * nM;
+    OQ_HIP(hipMemcpyAsync(k, u, (size_t)nM * 8, hipMemcpyHostToDevice, h->stream));
+    int rc = launch_transpose(k, e->M, e->n, y, h->stream);
     if (!rc) rc = set_live(e);
     if (!rc) rc = ens_rhs(e, y, k);
-    if (!rc) rc = launch_transpose(k, e->n, e->M, x, h->stream);
+    if (!rc) rc = launch_transpose(k, e->n, e->M, y, h->stream);
     if (rc) return rc;
-    OQ_HIP(hipMemcpyAsync(du, x, (size_t)nM * 8, hipMemcpyDeviceToHost, h->stream));
+    OQ_HIP(hipMemcpyAsync(du, y, (size_t)nM * 8, hipMemcpyDeviceToHost, h->stream));
     OQ_HIP(hipStreamSynchronize(h->stream));
     return OQ_OK;
 }
@@ -1753,7 +1751,7 @@ int oq_ensemble_time(oq_ensemble *e, int iters, double *ms_eval)
     if ((rc = set_live(e))) return rc;
     OQ_HIP(hipEventRecord(h->ev0, h->stream));
     for (int i = 0; i < iters; ++i)
-        if ((rc = ens_rhs(e, e->y.as<double>(), e->k.as<double>()))) return rc;
+        if ((rc = ens_rhs(e, e->y.as<double>(), e->k.as<double>() + 6 * e->n * e->M))) return rc;
     OQ_HIP(hipEventRecord(h->ev1, h->stream));
     OQ_HIP(hipEventSynchronize(h->ev1));
     float ms = 0.f;

@@ -1225,7 +1225,6 @@ struct oq_group {
     oq::DevBuf P;         // partial row sums of the units (capacity pcap doubles)
     size_t pcap = 0;
     oq::DevBuf u, y, k, part;
-    oq::DevBuf xfer;  // oq_group_eval: states in the host's layout
     oq::DevBuf ct, cdt, cdtcur, cqold, cna, cnr, citer, cdone, cacc, cret;
     oq::DevBuf live;  // GrpDev::live
     oq::GrpDev dev{};
@@ -1869,16 +1868,15 @@ int oq_group_eval(oq_group *e, const double *u, double *du)
     OQ_REQUIRE(e && u && du, "NULL argument");
     OQ_HIP(hipSetDevice(e->device));
     const size_t nb = (size_t)e->ntot * 8;
-    int rc = e->xfer.p ? OQ_OK : e->xfer.alloc(nb);
-    if (rc) return rc;
-    double *x = e->xfer.as<double>();
-    OQ_HIP(hipMemcpyAsync(x, u, nb, hipMemcpyHostToDevice, e->stream));
-    rc = to_entry_major(e, x, e->y.as<double>());
+    // through y and the last stage, both scratch between steps: a run goes on as if there had been no eval
+    double *y = e->y.as<double>(), *k = e->k.as<double>() + 6 * e->ntot;
+    OQ_HIP(hipMemcpyAsync(k, u, nb, hipMemcpyHostToDevice, e->stream));
+    int rc = to_entry_major(e, k, y);
     if (!rc) rc = set_live(e);
-    if (!rc) rc = grp_rhs(e, e->y.as<double>(), e->k.as<double>());
-    if (!rc) rc = from_entry_major(e, e->k.as<double>(), x);
+    if (!rc) rc = grp_rhs(e, y, k);
+    if (!rc) rc = from_entry_major(e, k, y);
     if (rc) return rc;
-    OQ_HIP(hipMemcpyAsync(du, x, nb, hipMemcpyDeviceToHost, e->stream));
+    OQ_HIP(hipMemcpyAsync(du, y, nb, hipMemcpyDeviceToHost, e->stream));
     OQ_HIP(hipStreamSynchronize(e->stream));
     return OQ_OK;
 }
@@ -1891,7 +1889,7 @@ int oq_group_time(oq_group *e, int iters, double *ms_eval)
     if ((rc = set_live(e))) return rc;
     OQ_HIP(hipEventRecord(e->ev0, e->stream));
     for (int i = 0; i < iters; ++i)
-        if ((rc = grp_rhs(e, e->y.as<double>(), e->k.as<double>()))) return rc;
+        if ((rc = grp_rhs(e, e->y.as<double>(), e->k.as<double>() + 6 * e->ntot))) return rc;
     OQ_HIP(hipEventRecord(e->ev1, e->stream));
     OQ_HIP(hipEventSynchronize(e->ev1));
     float ms = 0.f;
