@@ -156,6 +156,13 @@ typedef struct oq_stepper oq_stepper;
 const char *oq_last_error(void);
 int oq_version(void);
 int oq_device_count(int *count);
+/* Device memory between models: destroying a handle frees everything it holds
+ * except operator-sized blocks (32 MiB and more), of which the library keeps at
+ * most 4 GiB in all for the next model it assembles.  They are given back when
+ * one of its own allocations fails, when an ensemble or a group has been
+ * created, and by this call (at any time, from any thread): use it before
+ * another allocator or process needs the memory. */
+int oq_release_memory(void);
 
 /* ---- Green's functions (host output, caller-owned, Julia layout) ---- */
 

@@ -1459,6 +1459,7 @@ int oq_ensemble_create(int device, const oq_fault_mesh *mf, const oq_hex8_mesh *
             return rc;
         }
     }
+    reuse_trim(0);  // the assembly's FP64 operators do not stay beside a batch that may live long
     *out = e;
     return OQ_OK;
 }

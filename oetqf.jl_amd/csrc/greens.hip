@@ -84,9 +84,10 @@ double cosd(double deg)
 // and a program that assembles one model after another soon waits for that
 // on every allocation (57 ms for the 2.1 GB of the composite model, whose
 // assembly takes 7 ms).  At most kReuseBytes are held, the oldest go first,
-// and all of them when an allocation of the library fails.  A block enters
-// only after its device has been waited for (as hipFree does), so it can be
-// handed to any thread and stream.
+// and all of them when an allocation of the library fails, when a batch has
+// been created beside them, or when the caller asks (oq_release_memory).  A
+// block enters only after its device has been waited for (as hipFree does), so
+// it can be handed to any thread and stream.
 static constexpr size_t kReuseMin = (size_t)32 << 20, kReuseBytes = (size_t)4 << 30;
 struct ReuseBlock {
     void *p;
@@ -94,24 +95,30 @@ struct ReuseBlock {
     int device;
 };
 static std::mutex g_reuse_mutex;
-static std::vector<ReuseBlock> &reuse_blocks()
+static ReuseBlock g_reuse[kReuseBytes / kReuseMin];  // oldest first
+static size_t g_reuse_n = 0, g_reuse_held = 0;
+
+// With the lock held: takes block i off the list.
+static ReuseBlock reuse_take(size_t i)
 {
-    static std::vector<ReuseBlock> *v = new std::vector<ReuseBlock>();  // outlives every handle
-    return *v;
+    const ReuseBlock b = g_reuse[i];
+    for (--g_reuse_n; i < g_reuse_n; ++i) g_reuse[i] = g_reuse[i + 1];
+    g_reuse_held -= b.bytes;
+    return b;
 }
 
-// Frees the oldest blocks until at most `keep` bytes are held.
-static void reuse_trim(size_t keep)
+static void reuse_trim_locked(size_t keep)
+{
+    while (g_reuse_n > 0 && g_reuse_held > keep) {
+        const ReuseBlock b = reuse_take(0);
+        if (runtime_usable()) (void)hipFree(b.p);
+    }
+}
+
+void reuse_trim(size_t keep)
 {
     std::lock_guard<std::mutex> lock(g_reuse_mutex);
-    auto &v = reuse_blocks();
-    size_t held = 0;
-    for (const auto &b : v) held += b.bytes;
-    while (!v.empty() && held > keep) {
-        held -= v.front().bytes;
-        if (runtime_usable()) (void)hipFree(v.front().p);
-        v.erase(v.begin());
-    }
+    reuse_trim_locked(keep);
 }
 
 static hipError_t malloc_or_trim(void **p, size_t n)
@@ -143,14 +150,13 @@ int DevBuf::alloc_reuse(size_t n)
     if (n < kReuseMin || hipGetDevice(&dev) != hipSuccess) return alloc(n);
     {
         std::lock_guard<std::mutex> lock(g_reuse_mutex);
-        auto &v = reuse_blocks();
-        for (size_t i = 0; i < v.size(); ++i)
-            if (v[i].device == dev && v[i].bytes >= n && v[i].bytes - n <= n / 8) {
-                p = v[i].p;
+        for (size_t i = 0; i < g_reuse_n; ++i)
+            if (g_reuse[i].device == dev && g_reuse[i].bytes >= n && g_reuse[i].bytes - n <= n / 8) {
+                const ReuseBlock b = reuse_take(i);
+                p = b.p;
                 bytes = n;
-                cap = v[i].bytes;
+                cap = b.bytes;
                 device = dev;
-                v.erase(v.begin() + (long)i);
                 return OQ_OK;
             }
     }
@@ -177,11 +183,10 @@ void DevBuf::release()
     if (p && runtime_usable()) {
         if (device >= 0 && cap <= kReuseBytes && hipGetDevice(&dev) == hipSuccess && dev == device &&
             hipDeviceSynchronize() == hipSuccess) {
-            {
-                std::lock_guard<std::mutex> lock(g_reuse_mutex);
-                reuse_blocks().push_back({p, cap, device});
-            }
-            reuse_trim(kReuseBytes);
+            std::lock_guard<std::mutex> lock(g_reuse_mutex);
+            reuse_trim_locked(kReuseBytes - cap);  // blocks are at least kReuseMin: the list has room
+            g_reuse[g_reuse_n++] = {p, cap, device};
+            g_reuse_held += cap;
         } else {
             (void)hipFree(p);
         }
@@ -788,6 +793,12 @@ static int lrept_of(const oq_fault_mesh *m, double buffer_ratio, double *lrept)
 using namespace oq;
 
 extern "C" {
+
+int oq_release_memory(void)
+{
+    reuse_trim(0);
+    return OQ_OK;
+}
 
 const char *oq_last_error(void) { return g_err.c_str(); }
 

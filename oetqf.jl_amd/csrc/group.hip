@@ -1736,6 +1736,7 @@ int oq_group_create(int device, int64_t ngeo, const oq_fault_mesh *mf,
     c.soffs = e->dsoffs.as<int64_t>(); c.nst = e->dnst.as<int64_t>();
     c.G = (int)ngeo; c.M = (int)M;
     c.live = e->live.as<int>();
+    reuse_trim(0);  // the assembly's FP64 operators do not stay beside a batch that may live long
     *out = e;
     return OQ_OK;
 }

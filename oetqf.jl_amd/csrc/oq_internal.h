@@ -90,6 +90,9 @@ struct DevBuf {
     template <class T> T *as() const { return static_cast<T *>(p); }
 };
 
+// Frees the oldest blocks kept for reuse until at most `keep` bytes are held.
+void reuse_trim(size_t keep);
+
 // Green's builders writing element (r, c) of a block to out[r*rs + c*cs]
 // (device pointer).  Used by the host-output API (Julia column-major) and
 // by oq_rhs_create_from_mesh (dense receiver-major K).

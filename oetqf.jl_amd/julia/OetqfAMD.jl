@@ -45,6 +45,9 @@ function check(rc::Cint)
     rc == 1 ? throw(ArgumentError(lasterror())) : error("oetqf_amd: " * lasterror())
 end
 
+# gives the operator blocks kept for the next model (at most 4 GiB) back to the runtime
+release_memory() = check(ccall((:oq_release_memory, libpath), Cint, ()))
+
 # Vector{NTuple{2,T}} is laid out as 2n contiguous T: pass it as is.
 tupleptr(v::Vector{NTuple{2,Float64}}) = Ptr{Float64}(pointer(v))
 

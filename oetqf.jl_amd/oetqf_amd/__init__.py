@@ -4,7 +4,7 @@ Host-side mirror of the reference's API (src/Oetqf.jl:29-45): mesh
 generation, stress Green's functions, properties, `assemble` and a Tsit5
 `solve`, all backed by the HIP library lib/liboetqf_amd.so through its C ABI.
 """
-from ._lib import OetqfError, device_count, load as load_library  # noqa: F401
+from ._lib import OetqfError, device_count, load as load_library, release_memory  # noqa: F401
 from .ensemble import Ensemble  # noqa: F401
 from .group import Group  # noqa: F401
 from .equation import (ArrayPartition, Integrator, ODEProblem, ODESolution, Tsit5, VCABM5,  # noqa: F401,E501

@@ -96,6 +96,7 @@ PROTOTYPES = {
     "oq_last_error": (ctypes.c_char_p, []),
     "oq_version": (_int, []),
     "oq_device_count": (_int, [ctypes.POINTER(_int)]),
+    "oq_release_memory": (_int, []),
     "oq_gf_okada_ff": (_int, [ctypes.POINTER(FaultMesh), _d, _d, _int, _i64, _d, _pd]),
     "oq_gf_okada_ff_dft": (_int, [ctypes.POINTER(FaultMesh), _d, _d, _int, _i64, _d, _pd]),
     "oq_gf_okada_ff_dft_noalloc": (_int, [ctypes.POINTER(FaultMesh), _d, _d, _int, _i64, _d, _vp, _vp]),
@@ -232,3 +233,10 @@ def device_count():
     n = _int(0)
     check(load().oq_device_count(ctypes.byref(n)))
     return n.value
+
+
+def release_memory():
+    """Gives the device memory that closed models left for the next one (at
+    most 4 GiB of operator blocks) back to the runtime, for another allocator
+    or process to use."""
+    check(load().oq_release_memory())
