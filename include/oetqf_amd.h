@@ -268,7 +268,8 @@ int oq_rhs_eval_device(oq_rhs *h, double t, const double *u, double *du);
 
 /* Sizes: number of state entries, matrix order N = nf + 6ne, bytes of the
  * resident operator (dense K; the Toeplitz kernel; or, coupled DFT, the
- * kernel plus the dense K_fm, K_mf and K_mm blocks). */
+ * kernel plus the dense K_fm, K_mf and K_mm blocks, on a grid their tables or
+ * the spectra that take the tables' place). */
 int oq_rhs_info(oq_rhs *h, int64_t *nstate, int64_t *n, int64_t *kbytes);
 
 /* Copies the dense operator back (N*N doubles, row r = receiver), for tests. */

@@ -135,6 +135,7 @@ int DevBuf::alloc(size_t n)
     release();
     if (n == 0) n = 8;
     if (malloc_or_trim(&p, n) != hipSuccess) {
+        (void)hipGetLastError();  // a caller may go on in less memory
         p = nullptr;
         set_error("hipMalloc of " + std::to_string(n) + " bytes failed");
         return OQ_ERR_NOMEM;

@@ -2082,6 +2082,38 @@ static int gsp_build(oq_rhs *h)
     return OQ_OK;
 }
 
+static std::unique_ptr<GridSource> grid_source(const oq_fault_mesh *mf, const oq_hex8_mesh *ma, const oq_quadrature *q,
+                                               double hx, double hy, double lrept, double lambda, double mu, int ftype,
+                                               int nrept)
+{
+    std::unique_ptr<GridSource> s(new GridSource());
+    const auto keep = [](std::vector<double> &v, const double *p, int64_t n) {
+        v.assign(p, p + n);
+        return v.data();
+    };
+    s->mf = *mf;
+    s->mf.x = keep(s->fault[0], mf->x, mf->nx);
+    s->mf.ax = keep(s->fault[1], mf->ax, 2 * mf->nx);
+    s->mf.y = keep(s->fault[2], mf->y, mf->nxi);
+    s->mf.z = keep(s->fault[3], mf->z, mf->nxi);
+    s->mf.axi = keep(s->fault[4], mf->axi, 2 * mf->nxi);
+    s->ma.ne = ma->ne;
+    const double *src[9] = {ma->cx, ma->cy, ma->cz, ma->qx, ma->qy, ma->qz, ma->dx, ma->dy, ma->dz};
+    const double **dst[9] = {&s->ma.cx, &s->ma.cy, &s->ma.cz, &s->ma.qx, &s->ma.qy, &s->ma.qz, &s->ma.dx, &s->ma.dy, &s->ma.dz};
+    for (int i = 0; i < 9; ++i) *dst[i] = keep(s->mantle[i], src[i], ma->ne);
+    s->quad.nq = q->nq;
+    s->quad.coords = keep(s->qc, q->coords, 3 * q->nq);
+    s->quad.weights = keep(s->qw, q->weights, q->nq);
+    s->hx = hx;
+    s->hy = hy;
+    s->lrept = lrept;
+    s->lambda = lambda;
+    s->mu = mu;
+    s->ftype = ftype;
+    s->nrept = nrept;
+    return s;
+}
+
 // Fused or split launches for the grid model: 20 operator applications of
 // each on zeroed state after 3 of warm-up, keep the faster (ties: fused).
 static int mm_grid_pick(oq_rhs *h)
@@ -2258,9 +2290,20 @@ static int create_from_mesh(int device, const oq_fault_mesh *mf, const oq_hex8_m
         if (!rc && h->mmgrid) {
             rc = mm_grid_build(ma, h->grid, h->grid.nxp, hx, hy, qu, lambda, mu, h->Tmm, h->stream);
             const MmGrid &gg = h->grid;
+            // The spectra (twice the tables' bytes) take the tables' place;
+            // where there is no memory for both at once, the convolution
+            // blocks run on the tables.
             if (!rc && gg.strike && gg.D * 8 <= 64 * 1024 &&
                 gsp_shape(h->spec, mf->nx, mf->nxi, gg.m, gg.nx, gg.ny, gg.nz, kGspM, kLdsMax)) {
                 rc = gsp_build(h);
+                if (rc == OQ_ERR_NOMEM) {
+                    for (DevBuf *b : {&h->spF, &h->spG, &h->spM, &h->spTw, &h->spW}) b->release();
+                    rc = OQ_OK;
+                }
+            }
+            if (!rc && h->spectral) {
+                h->source = grid_source(mf, ma, quad, hx, hy, fu.dev.lrept, lambda, mu, ftype, (int)nrept);
+                for (DevBuf *b : {&h->Ftab, &h->Gtab, &h->Tmm}) b->release();
             } else {
                 if (!rc) rc = mm_grid_parts(h);
                 if (!rc) rc = mm_roles_build(h);
@@ -2578,12 +2621,24 @@ int oq_rhs_get_k(oq_rhs *h, double *k)
     OQ_REQUIRE(h != nullptr && k != nullptr, "NULL argument");
     OQ_HIP(hipSetDevice(h->device));
     const int64_t n = h->N * h->ld;
-    DevBuf tmp;
+    DevBuf tmp, F, G, T;
     const double *src = h->K.as<double>();
     if (h->kdtype == OQ_K_FFT && h->ne > 0) {  // [expanded K_ff  K_fm ; K_mf K_mm]
         const int64_t nf = h->nf, m6 = 6 * h->ne;
         int rc = tmp.alloc((size_t)n * 8);
         if (rc) return rc;
+        if (h->spectral) {  // the tables again
+            const GridSource &g = *h->source;
+            QuadUpload qu;
+            if ((rc = qu.load(&g.quad)) ||
+                (rc = mm_strike_build(&g.mf, &g.ma, h->grid, g.lrept, qu, g.lambda, g.mu, g.ftype, g.nrept, F, G,
+                                      h->stream)) ||
+                (rc = mm_grid_build(&g.ma, h->grid, h->grid.nxp, g.hx, g.hy, qu, g.lambda, g.mu, T, h->stream)))
+                return rc;
+        }
+        const double *Ft = h->spectral ? F.as<double>() : h->Ftab.as<double>(),
+                     *Gt = h->spectral ? G.as<double>() : h->Gtab.as<double>(),
+                     *Tt = h->spectral ? T.as<double>() : h->Tmm.as<double>();
         OQ_HIP(hipMemsetAsync(tmp.p, 0, (size_t)n * 8, h->stream));
         if ((rc = launch_expand_toeplitz(h->stk.as<double>(), h->nx, h->nxi, tmp.as<double>(), h->ld,
                                          h->stream)))
@@ -2593,8 +2648,8 @@ int oq_rhs_get_k(oq_rhs *h, double *k)
                                     (size_t)m6 * 8, (size_t)nf, hipMemcpyDeviceToDevice, h->stream));
         if (h->mmgrid && h->grid.strike) {
             const MmGrid &g = h->grid;
-            launch_expand_strike(h->Ftab.as<double>(), h->Gtab.as<double>(), h->nx, h->nxi, g, tmp.as<double>() + nf,
-                                 h->ld, tmp.as<double>() + nf * h->ld, h->ld, h->stream);
+            launch_expand_strike(Ft, Gt, h->nx, h->nxi, g, tmp.as<double>() + nf, h->ld, tmp.as<double>() + nf * h->ld,
+                                 h->ld, h->stream);
             OQ_HIP(hipGetLastError());
         }
         if (h->mmgrid) {
@@ -2603,7 +2658,7 @@ int oq_rhs_get_k(oq_rhs *h, double *k)
                                         (size_t)h->ldf * 8, (size_t)nf * 8, (size_t)m6, hipMemcpyDeviceToDevice,
                                         h->stream));
             const MmGrid &g = h->grid;
-            launch_expand_mm(h->Tmm.as<double>(), g, g.nxp, tmp.as<double>() + nf * h->ld + nf, h->ld, h->stream);
+            launch_expand_mm(Tt, g, g.nxp, tmp.as<double>() + nf * h->ld + nf, h->ld, h->stream);
             OQ_HIP(hipGetLastError());
         } else {
             OQ_HIP(hipMemcpy2DAsync(tmp.as<double>() + nf * h->ld, (size_t)h->ld * 8, h->K.p, (size_t)h->ld * 8,

@@ -2,6 +2,9 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <memory>
+#include <vector>
+
 #include "grid_spectral.h"
 #include "oq_internal.h"
 
@@ -205,6 +208,17 @@ struct MmGrid {
     bool split = false;             // convolutions and the other roles as two launches (measured faster)
 };
 
+// Copies of what a grid operator was assembled from, for one whose tables are
+// not kept (spectral): oq_rhs_get_k evaluates them again, to the same bits.
+struct GridSource {
+    std::vector<double> fault[5], mantle[9], qc, qw;
+    oq_fault_mesh mf{};
+    oq_hex8_mesh ma{};
+    oq_quadrature quad{};
+    double hx = 0.0, hy = 0.0, lrept = 0.0, lambda = 0.0, mu = 0.0;
+    int ftype = 0, nrept = 0;
+};
+
 }  // namespace oq
 
 struct oq_rhs {
@@ -242,6 +256,7 @@ struct oq_rhs {
     bool spectral = false;
     oq::GridSpec spec{};
     oq::DevBuf spF, spG, spM, spTw, spW;
+    std::unique_ptr<oq::GridSource> source;  // in place of Ftab, Gtab and Tmm
     int64_t ldf = 0;
     oq::MmGrid grid{};
     oq::RhsDev dev{};

@@ -38,3 +38,35 @@ def test_grid_operator_matches_dense(rng, nx, nxi, dip, cells, rfzh):
         p.f.close()
     for k in range(5):
         assert relerr(du[0].x[k], du[1].x[k]) <= 1e-12, k
+
+
+@pytest.mark.parametrize("nx,nxi,cells", [(16, 4, (4, 3, 2)), (17, 2, (17, 1, 2))])
+def test_spectra_take_the_tables_place(rng, nx, nxi, cells):
+    """The resident operator is K_ff's kernel and the spectra alone; expanded,
+    it still has the entries of the pair kernels, and the right-hand side is
+    the same before and after."""
+    mf = oq.gen_mesh("RectOkada", 40e3, 12e3, 40e3 / nx, 12e3 / nxi, 90.0)
+    ma = oq.hex8_box(-20e3, -7e3, -9e3, 40e3, 13e3, -12e3, *cells)
+    pf, pa = rs_props(mf, rng), visc_props(ma, rng, 0.0)
+    v = pf.vpl * np.exp(rng.standard_normal(pf.a.shape))
+    u = oq.ArrayPartition(v, pf.L / v, np.zeros((ma.ne, 6)), 1e6 * rng.standard_normal((ma.ne, 6)), np.zeros(pf.a.shape))
+    p = oq.assemble_from_mesh(mf, ma, 3e10, 2e10, pf, pa, u, (0.0, 1.0), ftype=oq.DipSlip(), kdtype="fft_grid")
+    a, b = oq.similar(u), oq.similar(u)
+    p.f(a, u, None, 0.0)
+    K, nf = p.f.dense_operator(), nx * nxi
+    p.f(b, u, None, 0.0)
+    nbytes = p.f.info()[2]
+    p.f.close()
+    mx, my, mz = cells
+    m, pow2 = nx // mx, lambda n: 1 << (n - 1).bit_length()
+    P, Py = pow2(2 * mx - 1), pow2(max(2, 2 * my - 1))
+    bins, planes = P // 2 + 1, 6 * mz
+    assert nbytes == 8 * nf * nxi + 16 * bins * (2 * planes * my * nxi * m + Py * planes ** 2)
+    want = dict(fm=oq.stress_greens_function(ma, mf, 3e10, 2e10, ftype=oq.DipSlip()),
+                mm=oq.stress_greens_function(ma, 3e10, 2e10, checkeigvals=False))
+    for k, blk in (("fm", K[:nf, nf:]), ("mm", K[nf:, nf:])):
+        assert np.abs(blk - want[k]).max() <= 1e-12 * np.abs(want[k]).max(), k
+    gmf = oq.stress_greens_function(mf, ma, 3e10, 2e10, ftype=oq.DipSlip())
+    assert relerr(K[nf:, :nf], gmf) <= 1e-9  # Okada's closed form from shifted coordinates
+    for x, y in zip(a.x, b.x):
+        assert np.array_equal(x, y)
