@@ -2015,7 +2015,10 @@ static int dense_blocks(const oq_fault_mesh *mf, const oq_hex8_mesh *ma, const F
     }
     int rc = OQ_OK;
     DevBuf F, G, Tm;
+    // the tables are scratch: where there is no memory for them the pairs run, which need none
+    const auto no_room = [&rc]() { return rc == OQ_ERR_NOMEM ? (rc = OQ_OK, true) : false; };
     if (tfm || tmf) rc = mm_strike_build(mf, ma, g, fu.dev.lrept, qu, lambda, mu, ftype, nrept, F, G, s);
+    if (no_room()) tfm = tmf = false;
     if (!rc && (tfm || tmf))
         launch_expand_strike(F.as<double>(), G.as<double>(), nx, nxi, g, tfm ? fm : nullptr, ldf, tmf ? mfp : nullptr,
                              ldm, s);
@@ -2024,6 +2027,7 @@ static int dense_blocks(const oq_fault_mesh *mf, const oq_hex8_mesh *ma, const F
         rc = launch_gf_mf(fu.dev, hu.dev, qu.c.as<double>(), qu.w.as<double>(), qu.nq, lambda, mu, ftype, nrept, mfp,
                           ldm, 1, s);
     if (!rc && tmm) rc = mm_grid_build(ma, g, g.nx, hx, hy, qu, lambda, mu, Tm, s);
+    if (no_room()) tmm = false;
     if (!rc && tmm) launch_expand_mm(Tm.as<double>(), g, g.nx, mm, ldm, s);
     if (!rc && !tmm) rc = launch_gf_mm(hu.dev, qu.c.as<double>(), qu.w.as<double>(), qu.nq, lambda, mu, mm, ldm, 1, s);
     if (rc) return rc;
