@@ -662,6 +662,19 @@ static void ens_split(EnsShape &s, int64_t N, int64_t nchunk, int64_t Mp)
     s.nz = (s.nchunk + s.cps - 1) / s.cps;
 }
 
+// The row sums Y, or where chunks are shared out the chunks' sums instead
+// (esz bytes each); without memory for those the chunks are not shared out.
+static int ens_sums(EnsShape &s, int64_t N, int64_t Mp, size_t esz, DevBuf &part, DevBuf &Y)
+{
+    if (s.nz > 1) {
+        const int rc = part.alloc((size_t)(s.nchunk * N * Mp) * esz);
+        if (rc != OQ_ERR_NOMEM) return rc;
+        s.nz = 1;
+        s.cps = s.nchunk;
+    }
+    return Y.alloc((size_t)(N * Mp) * 8);
+}
+
 template <int WM, int TB, int NW, bool BF>
 static int ens_f32_attr(const EnsShape &s)
 {
@@ -1320,8 +1333,7 @@ static int build_h3(oq_ensemble *e)
     if (!rc) rc = e->hS.alloc((size_t)(e->Mp * s.ldc) * 4);
     if (!rc) rc = e->hssc.alloc((size_t)(s.nchunk * e->Mp) * 8);
     ens_split(e->shape, h->N, s.nchunk, e->Mp);
-    if (!rc && e->shape.nz > 1) rc = e->hpart.alloc((size_t)(s.nchunk * h->N * e->Mp) * 8);
-    if (!rc && e->shape.nz == 1) rc = e->hY.alloc((size_t)(h->N * e->Mp) * 8);
+    if (!rc) rc = ens_sums(e->shape, h->N, e->Mp, 8, e->hpart, e->hY);
     if (rc) return rc;
     s.K = e->hK.as<_Float16>();
     s.rsc = e->hrsc.as<double>();
@@ -1447,8 +1459,7 @@ int oq_ensemble_create(int device, const oq_fault_mesh *mf, const oq_hex8_mesh *
         rc = e->Sm.alloc(sb);
         if (!rc && hipMemsetAsync(e->Sm.p, 0, sb, h->stream) != hipSuccess) rc = OQ_ERR_HIP;
         ens_split(e->shape, h->N, h->ld / kFChunk, e->Mp);
-        if (!rc && e->shape.nz > 1) rc = e->fpart.alloc((size_t)(e->shape.nchunk * h->N * e->Mp) * 4);
-        if (!rc && e->shape.nz == 1) rc = e->fY.alloc((size_t)(h->N * e->Mp) * 8);
+        if (!rc) rc = ens_sums(e->shape, h->N, e->Mp, 4, e->fpart, e->fY);
         if (!rc)
             rc = kdtype == OQ_K_BF16 ? OQ_ENS_TILED(e->shape, ens_f32_attr, OQ_ENS_BF16, e->shape)
                                      : OQ_ENS_TILED(e->shape, ens_f32_attr, OQ_ENS_F32, e->shape);
