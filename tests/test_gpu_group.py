@@ -82,8 +82,11 @@ def test_group_rhs_matches_fp64_oracle(oracle, batch):
 
 
 def test_group_rhs_exact_on_rounded_operator(oracle, batch):
-    """Against the FP64 oracle applied to the FP32 operator itself the error
-    is the FP32 product/partial-sum rounding only."""
+    """Against the FP64 oracle applied to an FP32 operator the error is the
+    rounding of FP32 products and partial sums.  The operator is read from a
+    single model (a group hands out none); the group's own is from pair kernels
+    of its own, and single entries of it round the other way.  They are held to
+    the single model's in test_gpu_batch_operator.py."""
     geoms, members, states, grp, U = batch
     dU = grp.unpack(grp.eval(U))
     mf, ma, pa = geoms[1]
