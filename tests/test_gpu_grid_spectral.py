@@ -70,3 +70,42 @@ def test_spectra_take_the_tables_place(rng, nx, nxi, cells):
     assert relerr(K[nf:, :nf], gmf) <= 1e-9  # Okada's closed form from shifted coordinates
     for x, y in zip(a.x, b.x):
         assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("kind", ["rupture", "one patch"])
+def test_rates_over_many_decades_component_by_component(rng, kind):
+    """Slip rates over 16 decades, and a single patch at 1 m/s on a locked
+    fault: every component of the stress rates against extended-precision sums
+    of the same operator.  The rounding of a transform spreads over its
+    outputs, so each component is held to 64 eps (lg 64 x lg 32 butterflies, two
+    passes and the products) of the largest sum |K||s| within its layer and
+    stress component, not of its own."""
+    nx, nxi, cells = 32, 8, (16, 12, 2)
+    mf = oq.gen_mesh("RectOkada", 80e3, 20e3, 80e3 / nx, 20e3 / nxi, 90.0)
+    ma = oq.hex8_box(-40e3, -20e3, -10e3, 80e3, 40e3, -30e3, *cells)
+    pf, pa = rs_props(mf, rng), visc_props(ma, rng, 0.0)
+    pa = oq.PowerLawViscosityProperty(pa.γ, np.zeros(ma.ne), np.zeros(6))
+    shp = pf.a.shape
+    if kind == "rupture":
+        v = 10.0 ** rng.uniform(-16, 0, shp)
+    else:
+        v = np.full(shp, 1e-16)
+        v[nx // 3, nxi // 2] = 1.0
+    sg = 1e6 * rng.standard_normal((ma.ne, 6))
+    u = oq.ArrayPartition(v, pf.L / v, np.zeros((ma.ne, 6)), sg, np.zeros(shp))
+    p = oq.assemble_from_mesh(mf, ma, 3e10, 3e10, pf, pa, u, (0.0, 1.0), kdtype="fft_grid")
+    K, nf, d = p.f.dense_operator(), nx * nxi, oq.similar(u)
+    p.f(d, u, None, 0.0)
+    p.f.close()
+    dev = sg.copy()
+    for k in (0, 3, 5):
+        dev[:, k] -= (sg[:, 0] + sg[:, 3] + sg[:, 5]) / 3.0
+    s = np.concatenate([(v - pf.vpl).ravel(order="F"), (pa.γ[:, None] * dev).ravel(order="F")])
+    Km = K[nf:].astype(np.longdouble)
+    ref = (Km @ s.astype(np.longdouble)).reshape((ma.ne, 6), order="F")
+    size = (np.abs(Km) @ np.abs(s)).reshape((ma.ne, 6), order="F")
+    layer = np.arange(ma.ne) // (cells[0] * cells[1])
+    for z in range(cells[2]):
+        for k in range(6):
+            err = np.abs(d.x[3][layer == z, k] - ref[layer == z, k]).max()
+            assert err <= 64 * np.finfo(float).eps * size[layer == z, k].max(), (z, k)
