@@ -1305,6 +1305,13 @@ static int set_live(oq_ensemble *e)
     return OQ_OK;
 }
 
+// A buffer for the states in the host's layout: scratch between steps, and not
+// y, the states that oq_ensemble_time evaluates (those of the last eval or stage).
+static double *ens_xfer(oq_ensemble *e)
+{
+    return e->alg == 1 ? e->eab.yn : e->k.as<double>() + 5 * e->n * e->M;
+}
+
 static void ens_destroy(oq_ensemble *e)
 {
     if (!e) return;
@@ -1481,15 +1488,15 @@ int oq_ensemble_eval(oq_ensemble *e, const double *u, double *du)
     oq_rhs *h = e->h;
     OQ_HIP(hipSetDevice(h->device));
     const int64_t nM = e->n * e->M;
-    // through y and the last stage, both scratch between steps: a run goes on as if there had been no eval
-    double *y = e->y.as<double>(), *k = e->k.as<double>() + 6 * nM;
-    OQ_HIP(hipMemcpyAsync(k, u, (size_t)nM * 8, hipMemcpyHostToDevice, h->stream));
-    int rc = launch_transpose(k, e->M, e->n, y, h->stream);
+    // through buffers that are scratch between steps: a run goes on as if there had been no eval
+    double *x = ens_xfer(e), *y = e->y.as<double>(), *k = e->k.as<double>() + 6 * nM;
+    OQ_HIP(hipMemcpyAsync(x, u, (size_t)nM * 8, hipMemcpyHostToDevice, h->stream));
+    int rc = launch_transpose(x, e->M, e->n, y, h->stream);
     if (!rc) rc = set_live(e);
     if (!rc) rc = ens_rhs(e, y, k);
-    if (!rc) rc = launch_transpose(k, e->n, e->M, y, h->stream);
+    if (!rc) rc = launch_transpose(k, e->n, e->M, x, h->stream);
     if (rc) return rc;
-    OQ_HIP(hipMemcpyAsync(du, y, (size_t)nM * 8, hipMemcpyDeviceToHost, h->stream));
+    OQ_HIP(hipMemcpyAsync(du, x, (size_t)nM * 8, hipMemcpyDeviceToHost, h->stream));
     OQ_HIP(hipStreamSynchronize(h->stream));
     return OQ_OK;
 }
@@ -1529,9 +1536,8 @@ static int ens_begin(oq_ensemble *e, const double *u0, const double *tv, const d
     }
     e->alg = alg;
     const std::vector<int> zi(M, 0);
-    // through y, which every step writes before it reads it
-    OQ_HIP(hipMemcpyAsync(e->y.p, u0, (size_t)nM * 8, hipMemcpyHostToDevice, h->stream));
-    int rc = launch_transpose(e->y.as<double>(), M, e->n, e->u.as<double>(), h->stream);
+    OQ_HIP(hipMemcpyAsync(ens_xfer(e), u0, (size_t)nM * 8, hipMemcpyHostToDevice, h->stream));
+    int rc = launch_transpose(ens_xfer(e), M, e->n, e->u.as<double>(), h->stream);
     if (rc) return rc;
     OQ_HIP(hipMemcpyAsync(e->ct.p, tv, M * 8, hipMemcpyHostToDevice, h->stream));
     OQ_HIP(hipMemcpyAsync(e->cdt.p, dtv, M * 8, hipMemcpyHostToDevice, h->stream));
@@ -1745,10 +1751,10 @@ int oq_ensemble_state(oq_ensemble *e, double *t, double *u, int64_t *naccept, in
     if (naccept) OQ_HIP(hipMemcpyAsync(naccept, e->cna.p, M * 8, hipMemcpyDeviceToHost, h->stream));
     if (nreject) OQ_HIP(hipMemcpyAsync(nreject, e->cnr.p, M * 8, hipMemcpyDeviceToHost, h->stream));
     if (retcode) OQ_HIP(hipMemcpyAsync(retcode, e->cret.p, M * 4, hipMemcpyDeviceToHost, h->stream));
-    if (u) {  // through y, scratch between steps
-        const int rc = launch_transpose(e->u.as<double>(), e->n, M, e->y.as<double>(), h->stream);
+    if (u) {
+        const int rc = launch_transpose(e->u.as<double>(), e->n, M, ens_xfer(e), h->stream);
         if (rc) return rc;
-        OQ_HIP(hipMemcpyAsync(u, e->y.p, (size_t)nM * 8, hipMemcpyDeviceToHost, h->stream));
+        OQ_HIP(hipMemcpyAsync(u, ens_xfer(e), (size_t)nM * 8, hipMemcpyDeviceToHost, h->stream));
     }
     OQ_HIP(hipStreamSynchronize(h->stream));
     return OQ_OK;

@@ -1532,6 +1532,13 @@ static void grp_destroy(oq_group *e)
     delete e;
 }
 
+// A buffer for the states in the host's layout: scratch between steps, and not
+// y, the states that oq_group_time evaluates (those of the last eval or stage).
+static double *grp_xfer(oq_group *e)
+{
+    return e->alg == 1 ? e->gab.yn : e->k.as<double>() + 5 * e->ntot;
+}
+
 // Member-major states (geometry g: M members of n_g entries, the host's
 // layout) <-> entry-major segments, both on the device.  soffs holds the
 // offsets of both: a segment has n_g M entries either way.
@@ -1869,15 +1876,15 @@ int oq_group_eval(oq_group *e, const double *u, double *du)
     OQ_REQUIRE(e && u && du, "NULL argument");
     OQ_HIP(hipSetDevice(e->device));
     const size_t nb = (size_t)e->ntot * 8;
-    // through y and the last stage, both scratch between steps: a run goes on as if there had been no eval
-    double *y = e->y.as<double>(), *k = e->k.as<double>() + 6 * e->ntot;
-    OQ_HIP(hipMemcpyAsync(k, u, nb, hipMemcpyHostToDevice, e->stream));
-    int rc = to_entry_major(e, k, y);
+    // through buffers that are scratch between steps: a run goes on as if there had been no eval
+    double *x = grp_xfer(e), *y = e->y.as<double>(), *k = e->k.as<double>() + 6 * e->ntot;
+    OQ_HIP(hipMemcpyAsync(x, u, nb, hipMemcpyHostToDevice, e->stream));
+    int rc = to_entry_major(e, x, y);
     if (!rc) rc = set_live(e);
     if (!rc) rc = grp_rhs(e, y, k);
-    if (!rc) rc = from_entry_major(e, k, y);
+    if (!rc) rc = from_entry_major(e, k, x);
     if (rc) return rc;
-    OQ_HIP(hipMemcpyAsync(du, y, nb, hipMemcpyDeviceToHost, e->stream));
+    OQ_HIP(hipMemcpyAsync(du, x, nb, hipMemcpyDeviceToHost, e->stream));
     OQ_HIP(hipStreamSynchronize(e->stream));
     return OQ_OK;
 }
@@ -1932,9 +1939,8 @@ static int grp_begin(oq_group *e, const double *u0, const double *tv, const doub
     }
     e->alg = alg;
     const std::vector<int> zi(GM, 0);
-    // through y, which every step writes before it reads it
-    OQ_HIP(hipMemcpyAsync(e->y.p, u0, (size_t)e->ntot * 8, hipMemcpyHostToDevice, e->stream));
-    int rc = to_entry_major(e, e->y.as<double>(), e->u.as<double>());
+    OQ_HIP(hipMemcpyAsync(grp_xfer(e), u0, (size_t)e->ntot * 8, hipMemcpyHostToDevice, e->stream));
+    int rc = to_entry_major(e, grp_xfer(e), e->u.as<double>());
     if (rc) return rc;
     OQ_HIP(hipMemcpyAsync(e->ct.p, tv, GM * 8, hipMemcpyHostToDevice, e->stream));
     OQ_HIP(hipMemcpyAsync(e->cdt.p, dtv, GM * 8, hipMemcpyHostToDevice, e->stream));
@@ -2067,10 +2073,10 @@ int oq_group_state(oq_group *e, double *t, double *u, int64_t *naccept, int64_t 
     if (naccept) OQ_HIP(hipMemcpyAsync(naccept, e->cna.p, GM * 8, hipMemcpyDeviceToHost, e->stream));
     if (nreject) OQ_HIP(hipMemcpyAsync(nreject, e->cnr.p, GM * 8, hipMemcpyDeviceToHost, e->stream));
     if (retcode) OQ_HIP(hipMemcpyAsync(retcode, e->cret.p, GM * 4, hipMemcpyDeviceToHost, e->stream));
-    if (u) {  // through y, scratch between steps
-        const int rc = from_entry_major(e, e->u.as<double>(), e->y.as<double>());
+    if (u) {
+        const int rc = from_entry_major(e, e->u.as<double>(), grp_xfer(e));
         if (rc) return rc;
-        OQ_HIP(hipMemcpyAsync(u, e->y.p, (size_t)e->ntot * 8, hipMemcpyDeviceToHost, e->stream));
+        OQ_HIP(hipMemcpyAsync(u, grp_xfer(e), (size_t)e->ntot * 8, hipMemcpyDeviceToHost, e->stream));
     }
     OQ_HIP(hipStreamSynchronize(e->stream));
     return OQ_OK;
