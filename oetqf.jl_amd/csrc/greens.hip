@@ -81,9 +81,10 @@ double cosd(double deg)
 
 // Operator-sized blocks between their release and the next allocation of
 // about that size.  The driver clears freed device memory at about 36 GB/s,
-// and a program that assembles one model after another soon waits for that
-// on every allocation (57 ms for the 2.1 GB of the composite model, whose
-// assembly takes 7 ms).  At most kReuseBytes are held, the oldest go first,
+// and a program that assembles one model after another may wait for that on
+// every allocation: the composite model (2.1 GB) took 53 ms a pass with the list
+// switched off and takes 6.5 with it (7.5 without it in processes that do not
+// come to wait).  At most kReuseBytes are held, the oldest go first,
 // and all of them when an allocation of the library fails, when a batch has
 // been created beside them, or when the caller asks (oq_release_memory).  A
 // block enters only after its device has been waited for (as hipFree does), so

@@ -1,6 +1,6 @@
 """The ensemble GEMMs' shapes: member tiles of 32, 64, 128 and 256 with the
 chunks of a row sum shared out over workgroups, one chunk each (the small
-models) or several (16512 rows, tiles of up to 64), and not shared out (16512
+models with FP32 and BF16) or several (16512 rows, tiles of up to 64), and not shared out (16512
 rows, tiles of 128 and 256; 33280 rows, all tiles).  Every shape adds the same
 products in the same order, so a member's derivative has the same bits whatever
 the ensemble around it; and it equals the member's own FP64 right-hand side to
