@@ -76,7 +76,9 @@ extern "C" {
  * fault row and mantle line (49 MB each at the 128x32 fault with 16x16x8
  * cells instead of 403 MB); otherwise they stay dense FP64.  In the former
  * case the operator is applied in the frequency domain where its transforms
- * fit in LDS (three launches).  All FP64.
+ * fit in LDS (three launches), and its spectra (127 MB there) take the tables'
+ * place; without memory for both at once the tables are applied as
+ * convolutions.  All FP64.
  * No counterpart in the reference (which multiplies the dense blocks,
  * equation.jl:201-203); entries equal the dense blocks' to rounding. */
 #define OQ_K_FFT_GRID 6
