@@ -2424,8 +2424,9 @@ static int host_eval(oq_rhs *h, const HostPart *parts, int np)
         return rc;
     }
     hipLaunchKernelGGL(k_copy_state, dim3(nblk(n, 256)), dim3(256), 0, h->stream, du, h->stage, n);
-    OQ_HIP(hipGetLastError());
-    OQ_HIP(hipStreamSynchronize(h->stream));
+    const hipError_t launched = hipGetLastError();
+    OQ_HIP(hipStreamSynchronize(h->stream));  // whatever the launches said: the pinned state is refilled next
+    OQ_HIP(launched);
     for (int i = 0; i < np; ++i) memcpy(parts[i].out, h->stage + parts[i].at, (size_t)parts[i].n * 8);
     return OQ_OK;
 }

@@ -1262,7 +1262,10 @@ static int stepper_create(oq_rhs *h, const double *u0, double t0, double t1,
     if (!rc) rc = st->k.alloc((size_t)(7 * n) * 8);
     if (!rc) rc = st->part.alloc(kPartBytes);
     int khz = 0;
-    if (!rc && hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, h->device) != hipSuccess) rc = OQ_ERR_HIP;
+    if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, h->device) != hipSuccess) {
+        (void)hipGetLastError();
+        khz = 0;  // wait_ticks' own rate
+    }
     st->wait = wait_ticks(khz);
     if (!rc) rc = st->ctrl.alloc(alg == 1 ? sizeof(AbCtrl) : sizeof(Ctrl));
     if (!rc && alg == 1) rc = st->ab.alloc((size_t)(2 * n) * 8);
