@@ -1504,16 +1504,19 @@ int oq_stepper_record_du(oq_stepper *st, int64_t stride, int64_t snap_capacity,
                "stride >= 1 and non-negative capacities required");
     oq_rhs *h = st->h;
     OQ_HIP(hipSetDevice(h->device));
-    int rc;
-    if ((rc = st->rcnt.alloc(2 * sizeof(long long)))) return rc;
-    if ((rc = st->rstep_t.alloc((size_t)step_capacity * 8))) return rc;
-    if ((rc = st->rstep_v.alloc((size_t)step_capacity * 8))) return rc;
-    if ((rc = st->rsnap_t.alloc((size_t)snap_capacity * 8))) return rc;
-    if ((rc = st->rsnap_u.alloc((size_t)(snap_capacity * st->n) * 8))) return rc;
-    if (du) {
-        if ((rc = st->rsnap_du.alloc((size_t)(snap_capacity * st->n) * 8))) return rc;
-    } else {
-        st->rsnap_du.release();
+    int rc = st->rcnt.alloc(2 * sizeof(long long));
+    if (!rc) rc = st->rstep_t.alloc((size_t)step_capacity * 8);
+    if (!rc) rc = st->rstep_v.alloc((size_t)step_capacity * 8);
+    if (!rc) rc = st->rsnap_t.alloc((size_t)snap_capacity * 8);
+    if (!rc) rc = st->rsnap_u.alloc((size_t)(snap_capacity * st->n) * 8);
+    if (!rc && du) rc = st->rsnap_du.alloc((size_t)(snap_capacity * st->n) * 8);
+    if (rc || !du) st->rsnap_du.release();
+    if (rc) {  // no recorder: the captured step and the persistent one must not keep the old buffers
+        for (DevBuf *b : {&st->rcnt, &st->rstep_t, &st->rstep_v, &st->rsnap_t, &st->rsnap_u}) b->release();
+        st->rec = Recorder{};
+        st->recording = false;
+        const int cc = capture_step(st);
+        return cc ? cc : rc;
     }
     const long long zero[2] = {0, 0};
     OQ_HIP(hipMemcpyAsync(st->rcnt.p, zero, sizeof(zero), hipMemcpyHostToDevice, h->stream));
